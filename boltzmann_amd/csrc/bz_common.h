@@ -143,10 +143,43 @@ __device__ __forceinline__ void two_sum_acc(double a, double b, double& s, doubl
   c += se + pe;
 }
 
-// 64-lane sum (result broadcast to every lane of the wave).
+// A 64-bit value moved across lanes by a DPP control (no LDS access).
+template <int CTRL>
+__device__ __forceinline__ double dpp_move(double v) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(v), CTRL, 0xf, 0xf, true);
+  const int hi = __builtin_amdgcn_mov_dpp(__double2hiint(v), CTRL, 0xf, 0xf, true);
+  return __hiloint2double(hi, lo);
+}
+// lane ^ 1, lane ^ 2, 7 - lane of each 8, 15 - lane of each 16, and rotations by 4 and 8 in 16 lanes
+constexpr int kDppXor1 = 0xB1, kDppXor2 = 0x4E, kDppHalfMirror = 0x141, kDppMirror = 0x140, kDppRor4 = 0x124,
+              kDppRor8 = 0x128;
+
+// v + the value of the other half wave (lane ^ 32), of the other row of 16 (lane ^ 16): the swap
+// instructions hand every lane both operands, in the same order.
+__device__ __forceinline__ double add_half_waves(double v) {
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  const auto a = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+  const auto b = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+  return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+}
+__device__ __forceinline__ double add_rows(double v) {
+  const unsigned lo = (unsigned)__double2loint(v), hi = (unsigned)__double2hiint(v);
+  const auto a = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+  const auto b = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+  return __hiloint2double((int)b[0], (int)a[0]) + __hiloint2double((int)b[1], (int)a[1]);
+}
+
+// 64-lane sum (result broadcast to every lane of the wave): the butterfly over lane ^ 32, 16, 8,
+// 4, 2, 1 with swap instructions and DPP moves, which take no LDS round trip (a rotation by 8 or 4
+// in a row of 16 brings the partner's value once the larger distances are summed).  The same
+// additions as six shuffles through the LDS crossbar.
 __device__ __forceinline__ double wave_sum(double v) {
-#pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) v += __shfl_xor(v, off, 64);
+  v = add_half_waves(v);
+  v = add_rows(v);
+  v += dpp_move<kDppRor8>(v);
+  v += dpp_move<kDppRor4>(v);
+  v += dpp_move<kDppXor2>(v);
+  v += dpp_move<kDppXor1>(v);
   return v;
 }
 

@@ -1,9 +1,8 @@
 // Planning of the per-grid tables of the fused 0D solver (bz_grid0d_t) from the dense
 // operators of one grid, for callers without the Python layer.  The same steps as the
 // Python planner: the union sparsity pattern in the permuted order i' = (npr-1-p) ns + l,
-// its row profiles, the lane-slot schedule of the factorisation by interval colouring
-// (rows enter their slot 2W steps before their first column), the register levels per
-// W-step chunk, and the floating-point tables (operator profiles, mass Cholesky rows, u,
+// its row profiles, the slot schedule of the blocked factorisation by interval colouring,
+// and the floating-point tables (operator profiles, mass Cholesky rows, u,
 // uhat, M uhat, growth vectors) formed by this library's kernels.  The planner owns every
 // device array it allocates; bz_free_grid0d releases them.
 #include <algorithm>
@@ -20,7 +19,6 @@
 
 namespace {
 
-constexpr int kPrefetchWindows = 2;
 
 struct Plan0D {
   std::vector<void*> allocs;
@@ -111,18 +109,24 @@ int bz_plan_grid0d(int npr, int ns, int nop, const double* const* ops, const dou
   int max_row = 0;
   for (int i = 0; i < n; ++i) max_row = std::max(max_row, prof_off[i + 1] - prof_off[i]);
 
-  // interval colouring: row i holds a slot from step first_i - 2W to its pivot step i;
-  // rows in order of their start take the lowest free slot id
-  std::vector<int> start(n), order(n);
-  for (int i = 0; i < n; ++i) start[i] = first[i] - kPrefetchWindows * W;
-  for (int i = 0; i < n; ++i) order[i] = i;
+  // interval colouring (plan0d.tile_schedule): row i reads the column groups of four first_i >> 2
+  // .. (i >> 2) + NG and its slot goes to a row whose first group lies beyond them; with the e-e
+  // pattern a slot is held from step first_i - 2W to the pivot step i, which the one-pivot-a-step
+  // factorisation needs.  Rows in order of their start take the lowest free slot id.
+  const int NG = (W + 2) / 4;
+  std::vector<int> start(n), end(n), order(n);
+  for (int i = 0; i < n; ++i) {
+    start[i] = ee_pattern ? first[i] - 2 * W : first[i] >> 2;
+    end[i] = ee_pattern ? i - 1 : (i >> 2) + NG;
+    order[i] = i;
+  }
   std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return start[a] < start[b]; });
   using PI = std::pair<int, int>;
-  std::priority_queue<PI, std::vector<PI>, std::greater<PI>> alive;   // (pivot step, slot)
+  std::priority_queue<PI, std::vector<PI>, std::greater<PI>> alive;   // (end, slot)
   std::priority_queue<int, std::vector<int>, std::greater<int>> free_ids;
   std::vector<std::vector<int>> slot_rows;
   for (int i : order) {
-    while (!alive.empty() && alive.top().first <= start[i]) {
+    while (!alive.empty() && alive.top().first < start[i]) {
       free_ids.push(alive.top().second);
       alive.pop();
     }
@@ -135,26 +139,18 @@ int bz_plan_grid0d(int npr, int ns, int nop, const double* const* ops, const dou
       slot_rows.emplace_back();
     }
     slot_rows[s].push_back(i);
-    alive.push(PI(i, s));
+    alive.push(PI(end[i], s));
   }
   const int used = int(slot_rows.size());
-  const int R = std::max(1, (used + 63) / 64);
-  const int nslots = 64 * R;
-  std::vector<int> slot_first(nslots, -1), sched_next(n, -1);
+  // tables of the one-pivot-a-step form (e-e) have a multiple of 64 slots, the others never
+  const int nslots = ee_pattern ? 64 * std::max(1, (used + 63) / 64) : used + (used % 64 == 0);
+  std::vector<int> slot_first((nslots + 63) / 64 * 64, -1), sched_next(n, -1);
   for (int s = 0; s < used; ++s) {
     slot_first[s] = slot_rows[s][0];
     for (size_t a = 0; a + 1 < slot_rows[s].size(); ++a) sched_next[slot_rows[s][a]] = slot_rows[s][a + 1];
   }
-  const int nchunk = (n + W - 1) / W;
-  std::vector<int> levels(nchunk, 1);
-  for (int s = 0; s < used; ++s) {
-    const int lev = s / 64 + 1;
-    if (lev == 1) continue;
-    for (int i : slot_rows[s]) {
-      const int a = std::max(0, start[i]);
-      for (int c = a / W; c <= i / W; ++c) levels[c] = std::max(levels[c], lev);
-    }
-  }
+  // one level per W-step chunk: the kernels of this library do not read it
+  const std::vector<int> levels((n + W - 1) / W, 1);
   std::vector<uint32_t> ent_rc;
   ent_rc.reserve(P);
   for (int i = 0; i < n; ++i)

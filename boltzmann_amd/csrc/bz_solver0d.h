@@ -18,12 +18,10 @@
 //   * shared per grid: operator values in row profile storage (columns
 //     first_col[i]..min(i+bw, n-1)), nop arrays: C_0..C_{S-1}, C_Tg, A_E, M
 //   * per instance: K profile (sum of the scaled operators, built for the whole
-//     batch by k_prepare0d), U rows (WP doubles each, 1/U_jj first).
-// Lane/slot mapping: slot s lives in lane s % 64, register level s / 64.  A host
-// schedule assigns rows to slots so that no two rows alive at the same step share
-// a slot (a row is alive from step first_col - 2W, when its prefetch starts, to its
-// pivot step) and uses level 1+ only where more than 64 rows are alive; every
-// W-step chunk runs only the levels its rows occupy.
+//     batch by k_prepare0d), U rows (WP doubles each).
+// Slot mapping: slot s is row s % 16 of tile s / 16 (factor_tiles).  A host schedule
+// assigns rows to slots so that no two rows share a slot whose columns are read at the
+// same time.
 //
 // This header holds the device code and the launch templates; it is included by the
 // translation units that instantiate them per window width (bz_solver0d_w<W>.hip) and by
@@ -50,6 +48,7 @@ struct GridDev {
   const double* mchol;      // [n][4]  banded Cholesky of M (permuted), L[i, i-d*ns]
   const int* chunk_levels;  // [ceil(n/W)] register levels alive in each W-step chunk
   const unsigned* ent_rc;   // [P] (row << 16) | column of every profile entry
+  int keep_mass;            // the staged mass factor has LDS of its own (set by the launch)
 };
 
 struct BatchDev {
@@ -83,10 +82,10 @@ struct EEDev {
   const double* g_lo;
 };
 
-// Per-window dispatch (one translation unit per window width W, every register level R
+// Per-window dispatch (one translation unit per window width W, the instantiated tile counts
 // of that window): steady Newton (ee: NULL or the frozen e-e potentials), transient step,
-// e-e factorisation and preconditioner application.  Each returns BZ_EINVAL when no
-// instance of its window matches g.nslots / 64.
+// e-e factorisation and preconditioner application.  Each returns BZ_EINVAL when g.nslots
+// needs more tiles than the largest instance has.
 #define BZ0D_DECLARE_WINDOW(W)                                                                         \
   int steady_w##W(const GridDev& g, const BatchDev& b, hipStream_t s, const EEDev* ee);               \
   int transient_w##W(const GridDev& g, const BatchDev& b, double cdt, const double* ustart, double* avg, \
@@ -134,61 +133,22 @@ __device__ __forceinline__ double fast_rcp(double a) {
   return r;
 }
 
-// y = K x over the flat profile: entries are lane-strided (coalesced loads, no
-// dependence between iterations) and accumulated into y[row] with LDS atomics.  Groups of
-// U entries per lane issue all their loads before the first atomic, so a group waits on
-// memory once.  y must be zeroed and synchronised by the caller.
-__device__ void flat_matvec(int P, const double* __restrict__ kp, const unsigned* __restrict__ rc,
-                            const double* __restrict__ x, double* y, int lane) {
-  constexpr int U = 8;
-  int e0 = lane;
-  for (; e0 + 64 * (U - 1) < P; e0 += 64 * U) {
-    unsigned v[U];
-    double a[U];
-#pragma unroll
-    for (int u = 0; u < U; ++u) {
-      v[u] = rc[e0 + 64 * u];
-      a[u] = kp[e0 + 64 * u];
-    }
-#pragma unroll
-    for (int u = 0; u < U; ++u) atomicAdd(&y[v[u] >> 16], a[u] * x[v[u] & 0xffffu]);
-  }
-  for (int e = e0; e < P; e += 64) {
-    const unsigned v = rc[e];
-    atomicAdd(&y[v >> 16], kp[e] * x[v & 0xffffu]);
-  }
+// Compensated (s, e) += the pair of another lane.
+template <int CTRL>
+__device__ __forceinline__ void dd_reduce(double& s, double& e) {
+#pragma clang fp contract(off)
+  const double s2 = dpp_move<CTRL>(s), e2 = dpp_move<CTRL>(e);
+  const double t = s + s2, z = t - s;
+  const double er = (s - (t - z)) + (s2 - z);
+  s = t;
+  e = e + e2 + er;
 }
 
-// In-place solve M z = b in the permuted order: every l-block (stride ns) is the
-// reversed radial mass block with banded Cholesky rows lc[q*4 + d] = L[q, q-d]
-// (d = 0 entry stored inverted, out-of-band entries zero) held in LDS; lanes
-// 0..ns-1 each own one block and carry the last three values in registers.
-__device__ void mass_solve(int ns, int npr, const double* __restrict__ lc, double* __restrict__ b, int lane) {
-  if (lane < ns) {
-    const int l = lane;
-    double y1 = 0.0, y2 = 0.0, y3 = 0.0;
-    for (int q = 0; q < npr; ++q) {
-      const double* L = lc + q * 4;
-      double s = b[q * ns + l];
-      s = fma(-L[1], y1, s);
-      s = fma(-L[2], y2, s);
-      s = fma(-L[3], y3, s);
-      const double y = s * L[0];
-      b[q * ns + l] = y;
-      y3 = y2; y2 = y1; y1 = y;
-    }
-    double z1 = 0.0, z2 = 0.0, z3 = 0.0;
-    for (int q = npr - 1; q >= 0; --q) {
-      double s = b[q * ns + l];
-      if (q + 1 < npr) s = fma(-lc[(q + 1) * 4 + 1], z1, s);
-      if (q + 2 < npr) s = fma(-lc[(q + 2) * 4 + 2], z2, s);
-      if (q + 3 < npr) s = fma(-lc[(q + 3) * 4 + 3], z3, s);
-      const double z = s * lc[q * 4];
-      b[q * ns + l] = z;
-      z3 = z2; z2 = z1; z1 = z;
-    }
-  }
-}
+// Pointers into LDS, marked as such: a function the compiler keeps out of line would
+// otherwise access LDS with generic (flat) instructions, which also wait on global loads.
+typedef __attribute__((address_space(3))) double lds_double;
+typedef __attribute__((address_space(3))) int lds_int;
+typedef __attribute__((address_space(1))) double glb_double;
 
 __device__ __forceinline__ double dot(const double* __restrict__ a, const double* __restrict__ b, int n, int lane) {
   double s = 0.0;
@@ -202,7 +162,7 @@ __device__ double dot_dd(const double* __restrict__ a, const double* __restrict_
   double s = 0.0, c = 0.0;
   for (int i = lane; i < n; i += 64) two_sum_acc(a[i], b[i], s, c);
 #pragma unroll
-  for (int off = 32; off >= 1; off >>= 1) {
+  for (int off = 32; off >= 16; off >>= 1) {
 #pragma clang fp contract(off)
     const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
     const double t = s + s2, z = t - s;
@@ -210,15 +170,18 @@ __device__ double dot_dd(const double* __restrict__ a, const double* __restrict_
     s = t;
     c = c + c2 + e;
   }
+  dd_reduce<kDppRor8>(s, c);
+  dd_reduce<kDppRor4>(s, c);
+  dd_reduce<kDppXor2>(s, c);
+  dd_reduce<kDppXor1>(s, c);
   return s + c;
 }
 
 // y = M x from the M profile (M is l-block diagonal, radial 7-band: columns i + d*ns, |d| <= 3).
-__device__ void mass_matvec(int n, int ns, const double* __restrict__ mprof, const int* __restrict__ first_col,
-                            const int* __restrict__ poff, const double* __restrict__ x, double* __restrict__ y,
-                            int lane) {
+__device__ void mass_matvec(int n, int ns, const double* __restrict__ mprof, const int2* __restrict__ rt,
+                            const double* __restrict__ x, double* __restrict__ y, int lane) {
   for (int i = lane; i < n; i += 64) {
-    const int base = poff[i] - first_col[i];
+    const int base = rt[i].y;
     double s = 0.0;
 #pragma unroll
     for (int d = -3; d <= 3; ++d) {
@@ -229,24 +192,158 @@ __device__ void mass_matvec(int n, int ns, const double* __restrict__ mprof, con
   }
 }
 
-// Pointers into LDS, marked as such: a function the compiler keeps out of line would
-// otherwise access LDS with generic (flat) instructions, which also wait on global loads.
-typedef __attribute__((address_space(3))) double lds_double;
-typedef __attribute__((address_space(3))) int lds_int;
-typedef __attribute__((address_space(3))) short lds_short;
-typedef __attribute__((address_space(1))) double glb_double;
+// ---------------------------------------------------------------- matrix-core profile LU
+//
+// The elimination runs in blocks of four pivots on the FP64 matrix cores.  Alive rows sit in
+// slots, 16 to a tile; a tile holds, per lane 16 q + row (q = 0..3), column 4 h + q of its row
+// for the column groups h = g (the panel) and g + 1 .. g + NG (what the upper bandwidth of four
+// pivots reaches), one register each, and the three right-hand sides (q = which one).  That is
+// the operand layout of v_mfma_f64_4x4x4f64 (A: lane i + 4 b + 16 k, B: lane j + 4 b + 16 k,
+// D: lane j + 4 b + 16 i, b the block) and of v_mfma_f64_16x16x4f64 (A: lane i + 16 k, B: lane
+// j + 16 k, accumulator element m of lane l: D[4 m + l / 16][l % 16]), so a panel register is
+// an operand as it stands and nothing is transposed between steps:
+//   multipliers  L^T = U11^-T panel^T         one 4x4x4 per tile
+//   update       window^T -= U12^T L^T        one 16x16x4 per tile (ring and right-hand sides)
+// The pivot rows of a block are published through LDS (they may sit in any slot); every lane
+// factorises the 4 x 4 pivot block in registers and eliminates the column of U it supplies.
+// Bound: the chain publish -> 4 x 4 LU (four reciprocals) -> two matrix instructions per block
+// with one wavefront per SIMD, issue slots with two.  One row per lane and one pivot per step on
+// the vector pipe took about 200 instructions per pivot for 28 multiply-adds; here it is about
+// 75.
+typedef double v4d __attribute__((ext_vector_type(4)));
+typedef unsigned int v2u __attribute__((ext_vector_type(2)));
+typedef __attribute__((address_space(3))) v4d lds_v4d;
 
-// Register state of the factorisation: R levels of row slots per lane.  Each slot also
-// holds the row that takes it next (nrow), so that one LDS read of that row's entry gives
-// all a slot change needs.  b1/b2/b3 hold the row's right-hand-side values, eliminated up
-// to the current step (read from Y1/Y2/Y3 when the row enters; b3 only with three
-// right-hand sides).
-template <int W, int R>
-struct FactorState {
-  int row[R], fc[R], off[R], nrow[R];
-  unsigned vmask[R];
-  double w[R][W], nk[R][W], b1[R], b2[R], b3[R];
+__device__ __forceinline__ double mfma4(double a, double b, double c) {
+  return __builtin_amdgcn_mfma_f64_4x4x4f64(a, b, c, 0, 0, 0);
+}
+__device__ __forceinline__ v4d mfma16(double a, double b, v4d c) {
+  return __builtin_amdgcn_mfma_f64_16x16x4f64(a, b, c, 0, 0, 0);
+}
+
+// Column groups of four right of a pivot block that its U rows reach (bw <= W - 1).
+template <int W>
+constexpr int trail_groups() { return (W + 2) / 4; }
+
+// Rows of one instance's profile (or of its U rows) read through a buffer descriptor: an offset
+// past the end reads as zero, which is how columns outside a row's profile are masked.
+struct ProfileBuf {
+  __amdgpu_buffer_rsrc_t r;
 };
+constexpr int kOutside = 0x40000000;       // beyond every profile (n < 32768, P * 8 < 2^30 checked on the host)
+
+__device__ __forceinline__ ProfileBuf profile_buf(const double* p, int count) {
+  return {__builtin_amdgcn_make_buffer_rsrc((void*)p, 0, count * 8, 0x00020000)};
+}
+__device__ __forceinline__ double buf_load(const ProfileBuf& b, int byte) {
+  const v2u v = __builtin_amdgcn_raw_buffer_load_b64(b.r, byte, 0, 0);
+  return __hiloint2double((int)v.y, (int)v.x);
+}
+
+// A store past the end is dropped.
+__device__ __forceinline__ void buf_store(const ProfileBuf& b, int byte, double v) {
+  v2u w;
+  w.x = (unsigned)__double2loint(v);
+  w.y = (unsigned)__double2hiint(v);
+  __builtin_amdgcn_raw_buffer_store_b64(w, b.r, byte, 0, 0);
+}
+
+// The lane index hidden from the optimiser: what a phase derives from it is formed where the
+// phase starts and not kept in registers (spilled, in the end) through all other phases.
+__device__ __forceinline__ int fresh_lane(int lane) {
+  asm volatile("" : "+v"(lane));
+  return lane;
+}
+
+__device__ __forceinline__ void wave_lds_fence() {
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Row sums of the instance profile, sum_c k[row][c] x[c], eight lanes to a row and eight rows at
+// a time (64-byte segments of a row per load; rows taken harmonic by harmonic, so the eight rows
+// of a pass have about the same length).  A step is 32 columns of the eight rows; the entries of
+// the next two steps are in flight while one is summed (a step waited on memory for several
+// times what its sums take).  DD: -k x in compensated arithmetic (s, e), else the plain sum in
+// s.  fin(row, s, e) runs on one lane per row.
+template <bool DD, class Fin>
+__device__ __forceinline__ void row_sums(int n, int ns, int npr, int bw, int P, const int2* __restrict__ rt,
+                                         const double* __restrict__ kp, const double* __restrict__ x_, int lane,
+                                         Fin fin) {
+  lane = fresh_lane(lane);
+  const ProfileBuf kb = profile_buf(kp, P);
+  const lds_double* x = (const lds_double*)x_;
+  const int sub = lane & 7;
+  int p = lane >> 3, l = 0, row = 0, c = 0, lc = -1, off = 0;      // the row whose entries are fetched next
+  struct Step {
+    double k[4];
+    int c, row;
+    bool last;
+  };
+  auto set_row = [&]() {
+    while (p >= npr && l < ns) {
+      p -= npr;
+      ++l;
+    }
+    const bool ok = l < ns;
+    row = ok ? p * ns + l : -1;
+    const int2 v = rt[ok ? row : 0];
+    lc = ok ? min(row + bw, n - 1) : -1;
+    c = (v.x & 0xffff) + sub;
+    off = 8 * v.y;
+  };
+  auto fetch = [&](Step& s) {
+    s.c = c;
+    s.row = row;
+#pragma unroll
+    for (int u = 0; u < 4; ++u) s.k[u] = buf_load(kb, c + 8 * u <= lc ? off + 8 * (c + 8 * u) : kOutside);
+    s.last = !__any(c + 32 <= lc);
+    if (s.last) {
+      p += 8;
+      set_row();
+    } else {
+      c += 32;
+    }
+  };
+  double s = 0.0, e = 0.0;
+  auto sum = [&](const Step& b) {
+    double xv[4];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) xv[u] = x[min(b.c + 8 * u, n - 1)];
+#pragma unroll
+    for (int u = 0; u < 4; ++u) {
+      if constexpr (DD) two_sum_acc(-b.k[u], xv[u], s, e);
+      else s = fma(b.k[u], xv[u], s);
+    }
+    if (b.last) {
+      if constexpr (DD) {
+        dd_reduce<kDppXor1>(s, e);
+        dd_reduce<kDppXor2>(s, e);
+        dd_reduce<kDppHalfMirror>(s, e);
+      } else {
+        s += dpp_move<kDppXor1>(s);
+        s += dpp_move<kDppXor2>(s);
+        s += dpp_move<kDppHalfMirror>(s);
+      }
+      if (b.row >= 0 && sub == 0) fin(b.row, s, e);
+      s = 0.0;
+      e = 0.0;
+    }
+  };
+  Step b0, b1, b2;
+  set_row();
+  fetch(b0);
+  fetch(b1);
+  do {
+    fetch(b2);
+    sum(b0);
+    fetch(b0);
+    sum(b1);
+    fetch(b1);
+    sum(b2);
+  } while (__any(b0.row >= 0));
+}
 
 // Row table, one int2 per row i: x = first profile column of i (low 16 bits) | (next row
 // in i's slot << 16, -1 for none), y = profile offset of i minus that column (entries of
@@ -261,356 +358,494 @@ __device__ __forceinline__ void fill_rowtab(const GridDev& g, int2* __restrict__
   }
 }
 
-// Slot state for row `row` (row < 0: an empty slot, first column INT_MAX, never valid).
-__device__ __forceinline__ void row_enter(int2 v, int row, int& fc, int& off, int& nrow) {
-  fc = (row >= 0) ? (v.x & 0xffff) : 0x7fffffff;
-  off = (row >= 0) ? v.y : 0;
-  nrow = (row >= 0) ? (v.x >> 16) : -1;
-}
-
-// One W-step chunk of the factorisation running levels 0..RA-1 only.  SL: also store the
-// multipliers l_rj of L at the profile positions of (r, j) in lout.  TAIL: the chunk may
-// end past row n-1 (only the last one); full chunks carry no exit test, so the compiler
-// places no spill reloads for an exit path inside the steps (a reload waits on the
-// in-order memory counter, i.e. on every column prefetch issued before it).
-template <int W, int R, int RA, bool SL, bool TAIL, int NRHS>
-__device__ __forceinline__ void factor_chunk(int j0, int n, int bw, FactorState<W, R>& s,
-                                             const glb_double* __restrict__ kprof, const lds_int* __restrict__ s_succ,
-                                             lds_double* __restrict__ Y1, lds_double* __restrict__ Y2,
-                                             lds_double* __restrict__ Y3,
-                                             lds_double* __restrict__ s_piv, lds_double* __restrict__ s_junk,
-                                             glb_double* __restrict__ urows, int WP, int lane,
-                                             glb_double* __restrict__ lout) {
-#pragma unroll
-  for (int t = 0; t < W; ++t) {
-    const int j = j0 + t;
-    if (TAIL && j >= n) break;
-    // --- locate the pivot row j: lane lp, level rr (both wave-uniform)
-    int lp = 0, rr = 0;
-#pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const unsigned long long bl = __ballot(s.row[r] == j);
-      if (bl) { lp = __ffsll((long long)bl) - 1; rr = r; }
-    }
-    lp = __builtin_amdgcn_readfirstlane(lp);
-    rr = __builtin_amdgcn_readfirstlane(rr);
-    const int hit = (lane == lp) ? rr : -1;
-    // --- publish U_jj..U_j,j+W-1 and the two rhs values.  Every lane stores (no divergent
-    // branch): level rr of the pivot lane into s_piv, the others into their own row of
-    // s_junk.
-    {
-      lds_double* dst = (lane == lp) ? s_piv : s_junk + lane;
-#pragma unroll
-      for (int r = 0; r < RA; ++r) {
-        if (rr == r) {
-#pragma unroll
-          for (int k = 0; k < W; ++k) dst[k] = s.w[r][(t + k) % W];
-          dst[W] = s.b1[r];
-          dst[W + 1] = s.b2[r];
-          if constexpr (NRHS == 3) dst[W + 2] = s.b3[r];
-        }
-      }
-    }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    double pv[W];
-#pragma unroll
-    for (int k = 0; k < W; ++k) pv[k] = s_piv[k];
-    const double pb1 = s_piv[W], pb2 = s_piv[W + 1];
-    const double pb3 = (NRHS == 3) ? (double)s_piv[W + 2] : 0.0;
-    const double rinv = fast_rcp(pv[0]);
-    // --- U row j (1/U_jj first) and the eliminated rhs; every lane stores entry lane % WP
-    {
-      const int kk = lane % WP;
-      urows[(size_t)j * WP + kk] = (kk == 0) ? rinv : s_piv[kk];
-      Y1[j] = pb1;
-      Y2[j] = pb2;
-      if constexpr (NRHS == 3) Y3[j] = pb3;
-    }
-    // --- eliminate column j (rows whose first column lies beyond j have a zero there: their
-    // window may still hold the previous row of the slot), shift in column j+W (prefetched
-    // W steps ago)
-#pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const double m = (j >= s.fc[r]) ? s.w[r][t] * rinv : 0.0;
-      if (SL && s.row[r] > j && j >= s.fc[r]) lout[s.off[r] + j] = m;
-#pragma unroll
-      for (int k = 1; k < W; ++k) s.w[r][(t + k) % W] = fma(-m, pv[k], s.w[r][(t + k) % W]);
-      s.b1[r] = fma(-m, pb1, s.b1[r]);
-      s.b2[r] = fma(-m, pb2, s.b2[r]);
-      if constexpr (NRHS == 3) s.b3[r] = fma(-m, pb3, s.b3[r]);
-      s.w[r][t] = ((s.vmask[r] >> t) & 1u) ? s.nk[r][t] : 0.0;
-    }
-    // --- retire the pivot row; its slot takes the next scheduled row (one LDS read).  Its
-    // window is not cleared: the shift-ins of the next W steps overwrite every position
-    // (with zero, vmask being clear), and the row's first column is at least 2W steps away.
-    if (lane == lp) {
-#pragma unroll
-      for (int r = 0; r < RA; ++r) {
-        if (hit == r) {
-          const int nr = s.nrow[r];
-          s.row[r] = nr;
-          s.vmask[r] = 0u;
-          const int q = nr >= 0 ? nr : 0;
-          s.b1[r] = (nr >= 0) ? Y1[q] : 0.0;     // entry values of the right-hand sides of the new row
-          s.b2[r] = (nr >= 0) ? Y2[q] : 0.0;
-          if constexpr (NRHS == 3) s.b3[r] = (nr >= 0) ? Y3[q] : 0.0;
-          row_enter(make_int2(s_succ[2 * q], s_succ[2 * q + 1]), nr, s.fc[r], s.off[r], s.nrow[r]);
-        }
-      }
-    }
-    // --- branch-free prefetch of column j+2W (invalid columns read entry 0 and are masked);
-    // a 32-bit index from the instance's profile base
-#pragma unroll
-    for (int r = 0; r < RA; ++r) {
-      const int c = j + 2 * W;
-      const bool valid = (c >= s.fc[r]) && (c <= min(s.row[r] + bw, n - 1));
-      const unsigned idx = valid ? (unsigned)(s.off[r] + c) : 0u;
-      s.nk[r][t] = kprof[idx];
-      s.vmask[r] = (s.vmask[r] & ~(1u << t)) | ((valid ? 1u : 0u) << t);
+// The row whose columns a slot is reading.  Row i reads the groups first_col >> 2 .. (i >> 2) +
+// NG; the schedule gives its successor no column before group (i >> 2) + NG + 1.  LEFT: only the
+// columns left of the row's pivot block (the stored L factor).
+template <int NG, bool LEFT>
+struct SlotRow {
+  int fc, cnt, off8, lim, row, next;
+  __device__ __forceinline__ void enter(const lds_int* rt, int r, int n, int bw) {
+    row = r;
+    const int q = row >= 0 ? row : 0;
+    const int tx = rt[2 * q], ty = rt[2 * q + 1];
+    fc = tx & 0xffff;
+    cnt = LEFT ? max(0, (row & ~3) - fc) : min(row + bw, n - 1) - fc + 1;
+    off8 = ty * 8;
+    lim = (row >> 2) + NG;
+    next = tx >> 16;
+    if (row < 0) {
+      cnt = 0;
+      lim = 0x7fffffff;
+      next = -1;
     }
   }
+  __device__ __forceinline__ void advance(const lds_int* rt, int h, int n, int bw) {
+    if (h > lim) enter(rt, next, n, bw);
+  }
+  // byte offset of the row's entry in column c (past the end outside its profile)
+  __device__ __forceinline__ int at(int c) const { return (unsigned)(c - fc) < (unsigned)cnt ? off8 + 8 * c : kOutside; }
+  __device__ __forceinline__ double load(const ProfileBuf& kb, int c) const { return buf_load(kb, at(c)); }
+};
+
+// 4 x 4 LU without pivoting of the pivot block a[k][c], and what the block step needs of it.
+struct PivotBlock {
+  double l10, l20, l21, l30, l31, l32;      // unit lower factor
+  double u01, u02, u03, u12, u13, u23;      // strict upper factor
+  double r0, r1, r2, r3;                    // reciprocals of the diagonal
+  __device__ __forceinline__ void factor(v4d c0, v4d c1, v4d c2, v4d c3) {   // columns
+    r0 = fast_rcp(c0[0]);
+    l10 = c0[1] * r0; l20 = c0[2] * r0; l30 = c0[3] * r0;
+    u01 = c1[0]; u02 = c2[0]; u03 = c3[0];
+    const double a11 = fma(-l10, u01, c1[1]);
+    r1 = fast_rcp(a11);
+    u12 = fma(-l10, u02, c2[1]);
+    u13 = fma(-l10, u03, c3[1]);
+    l21 = fma(-l20, u01, c1[2]) * r1;
+    l31 = fma(-l30, u01, c1[3]) * r1;
+    const double a22 = fma(-l21, u12, fma(-l20, u02, c2[2]));
+    r2 = fast_rcp(a22);
+    u23 = fma(-l21, u13, fma(-l20, u03, c3[2]));
+    l32 = fma(-l31, u12, fma(-l30, u02, c2[3])) * r2;
+    r3 = fast_rcp(fma(-l32, u23, fma(-l31, u13, fma(-l30, u03, c3[3]))));
+  }
+};
+
+// L^-1 of a block column v (four pivot rows): the substitution of the elimination itself
+__device__ __forceinline__ v4d lower_apply(double l10, double l20, double l21, double l30, double l31, double l32,
+                                           v4d v) {
+  v4d u;
+  u[0] = v[0];
+  u[1] = fma(-l10, u[0], v[1]);
+  u[2] = fma(-l21, u[1], fma(-l20, u[0], v[2]));
+  u[3] = fma(-l32, u[2], fma(-l31, u[1], fma(-l30, u[0], v[3])));
+  return u;
 }
 
-// Factorise A = K - mu M (the instance profile already holds K - mu M; permuted order,
-// no pivoting) and forward-eliminate NRHS (2 or 3) right-hand sides whose entry values are
-// read from Y1, Y2 (and Y3) when a row enters its slot.  Y*[j] are overwritten by the
-// eliminated values at pivot step j, which is never before the entry of row j.  U rows
-// (1/U_jj first) go to urows.  The column prefetch is branch-free so that every step issues
-// a fixed number of loads and the memory-counter waits can be counted statically.
-template <int W, int R, bool SL = false, int NRHS = 2>
-__device__ void factor_forward(const GridDev& g, const double* __restrict__ kprof_,
-                               const int2* __restrict__ succ_,
-                               double* __restrict__ y1_, double* __restrict__ y2_, double* __restrict__ y3_,
-                               double* __restrict__ piv_,
-                               double* __restrict__ junk_, double* __restrict__ urows_, int WP, int lane,
-                               double* __restrict__ lout_ = nullptr) {
+__device__ __forceinline__ double pick4(v4d v, int k) {
+  const double a = (k & 1) ? v[1] : v[0], b = (k & 1) ? v[3] : v[2];
+  return (k & 2) ? b : a;
+}
+
+// Factorise A = K - mu M (the instance profile already holds it; permuted order, no pivoting)
+// and forward-eliminate NRHS (1 to 3) right-hand sides whose entry values are read from Y1, Y2,
+// Y3 when a row enters its slot (never after its own pivot step); Y*[j] receive the eliminated
+// values.  U goes to urows, row j at urows[j * WP]: offset d >= 1 holds -U[j][j + d] for columns
+// right of the pivot block, and the block's own part holds U11^-1 (upper triangular, at the same
+// offsets as U11).  SL: the multipliers of L at the profile positions of lout.
+// s_piv: 16 (NG + 2) doubles of LDS, 32-byte aligned.
+template <int W, int T, bool SL, int NRHS>
+__device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof, const int2* __restrict__ rt_,
+                             double* __restrict__ y1_, double* __restrict__ y2_, double* __restrict__ y3_,
+                             double* __restrict__ piv_, double* __restrict__ urows, int lane,
+                             double* __restrict__ lout_ = nullptr) {
+  lane = fresh_lane(lane);
+  constexpr int NG = trail_groups<W>(), WP = (W + 1) & ~1, NX = NG > 4 ? NG - 4 : 0;
+  constexpr bool Y16 = NG <= 3;                      // the right-hand sides ride in the 16x16x4 tile
+  constexpr int YR = Y16 ? NG : 0;                   // as its element YR
   const int n = g.n, bw = g.bw;
-  const glb_double* kprof = (const glb_double*)kprof_;
-  glb_double* urows = (glb_double*)urows_;
+  const int q = lane >> 4, a16 = lane & 15, i4 = lane & 3;
+  const ProfileBuf kb = profile_buf(kprof, g.P), ub = profile_buf(urows, n * WP);
   glb_double* lout = (glb_double*)lout_;
-  const lds_int* s_succ = (const lds_int*)succ_;          // the row table as int pairs
-  lds_double* Y1 = (lds_double*)y1_;
-  lds_double* Y2 = (lds_double*)y2_;
-  lds_double* Y3 = (lds_double*)y3_;
-  lds_double* s_piv = (lds_double*)piv_;
-  lds_double* s_junk = (lds_double*)junk_;
-  FactorState<W, R> s;
+  const lds_int* rt = (const lds_int*)rt_;
+  lds_double* piv = (lds_double*)piv_;
+  lds_double* yq = (lds_double*)(q == 0 ? y1_ : (q == 1 || NRHS < 3) ? y2_ : y3_);        // entry values of this lane
+  const int qq = a16 & 3, m = a16 >> 2;
+  lds_double* yw = (lds_double*)(qq == 0 ? y1_ : (qq == 1 || NRHS < 3) ? y2_ : y3_);      // where eliminated ones go
+  const bool ywl = Y16 ? (m == NG && qq < NRHS) : (a16 < NRHS);
+  // where this lane's entry of U12 (per position u of the block in the ring) and of U11^-1 goes
+  // inside the four U rows of a block
+  int uo[NG], ux[NX ? NX * NG : 1];
 #pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int rw = g.slot_first[r * 64 + lane];
-    s.row[r] = rw;
-    const int lc = (rw >= 0) ? min(rw + bw, n - 1) : -1;
-    const int q = rw >= 0 ? rw : 0;
-    row_enter(make_int2(s_succ[2 * q], s_succ[2 * q + 1]), rw, s.fc[r], s.off[r], s.nrow[r]);
-    s.b1[r] = (rw >= 0) ? Y1[q] : 0.0;
-    s.b2[r] = (rw >= 0) ? Y2[q] : 0.0;
-    s.b3[r] = 0.0;
-    if constexpr (NRHS == 3) s.b3[r] = (rw >= 0) ? (double)Y3[q] : 0.0;
-    s.vmask[r] = 0u;
+  for (int u = 0; u < NG; ++u) {
+    const int o = 4 * (m > u ? m - u : m - u + NG) + qq - q;
+    uo[u] = (m < NG && o <= bw) ? (q * WP + o) * 8 : kOutside;
 #pragma unroll
-    for (int k = 0; k < W; ++k) {
-      const int c0 = k, c1 = W + k;
-      double v0 = 0.0, a1 = 0.0;
-      if (c0 >= s.fc[r] && c0 <= lc) v0 = kprof[s.off[r] + c0];
-      if (c1 >= s.fc[r] && c1 <= lc) {
-        a1 = kprof[s.off[r] + c1];
-        s.vmask[r] |= 1u << k;
-      }
-      s.w[r][k] = v0; s.nk[r][k] = a1;
+    for (int x = 0; x < NX; ++x) {
+      const int ox = 4 * (4 + x > u ? 4 + x - u : 4 + x - u + NG) + i4 - q;
+      ux[u * NX + x] = (a16 < 4 && ox <= bw) ? (q * WP + ox) * 8 : kOutside;
     }
   }
-  // Wait for the initial window loads here, once: with them still in flight at the loop
-  // entry, the compiler's wait analysis would put a full vector-memory wait in every chunk.
-  // (gfx9 s_waitcnt fields: vmcnt 0, expcnt 7, lgkmcnt 15.)
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  // Y1/Y2/Y3 double as the entry values of the right-hand sides: a row entering its
-  // slot during step j has index > j, and Y*[i] is only overwritten at pivot step i.
-  const int nfull = n / W;
-  for (int ch = 0; ch < nfull; ++ch)
-    factor_chunk<W, R, R, SL, false, NRHS>(ch * W, n, bw, s, kprof, s_succ, Y1, Y2, Y3, s_piv, s_junk, urows, WP,
-                                             lane, lout);
-  // last partial chunk: all levels (running a level with no rows is harmless)
-  if (nfull * W < n)
-    factor_chunk<W, R, R, SL, true, NRHS>(nfull * W, n, bw, s, kprof, s_succ, Y1, Y2, Y3, s_piv, s_junk, urows, WP,
-                                            lane, lout);
-}
+  const int ui_o = (a16 < 4 && i4 >= q) ? (q * WP + i4 - q) * 8 : kOutside;
 
-// Forward solve L y = b with the unit lower factor stored by factor_forward<SL = true> in the
-// profile positions of its multipliers (lprof), for one right-hand side held in Y (entry
-// values in, eliminated values out; in place).  The same lane slots, row table and 2W column
-// prefetch as the factorisation, with the stored multipliers streamed instead of the rows of
-// K - mu M and no window update: per step and level one load and one FMA.  The elimination
-// order per row is the factorisation's, so the result equals the fused elimination bitwise.
-template <int W, int R, bool TAIL>
-__device__ __forceinline__ void forward_chunk(int j0, int n, FactorState<W, R>& s, const glb_double* __restrict__ lp,
-                                              const lds_int* __restrict__ s_succ, lds_double* __restrict__ Y,
-                                              lds_double* __restrict__ s_piv, lds_double* __restrict__ s_junk,
-                                              int lane) {
+  // Per tile: P the panel, R4 ring registers 0..3 (and the right-hand sides), RX ring register 4
+  // and Y when they do not fit the 16x16x4 tile, F the groups read ahead.
+  SlotRow<NG, false> st[T];
+  int crow[T];                                       // row being eliminated in the slot
+  int cfc[SL ? T : 1], coff[SL ? T : 1];             // its first column and profile offset (SL)
+  double P[T], F[T][NG], RX[NX ? T : 1], Y[Y16 ? 1 : T];
+  v4d R4[T];
 #pragma unroll
-  for (int t = 0; t < W; ++t) {
-    const int j = j0 + t;
-    if (TAIL && j >= n) break;
-    int lpv = 0, rr = 0;
-#pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const unsigned long long bl = __ballot(s.row[r] == j);
-      if (bl) { lpv = __ffsll((long long)bl) - 1; rr = r; }
+  for (int t = 0; t < T; ++t) {
+    const int slot = 16 * t + a16;
+    const int row = slot < g.nslots ? g.slot_first[slot] : -1;
+    st[t].enter(rt, row, n, bw);
+    crow[t] = row;
+    if constexpr (SL) {
+      cfc[t] = st[t].fc;
+      coff[t] = st[t].off8 >> 3;
     }
-    lpv = __builtin_amdgcn_readfirstlane(lpv);
-    rr = __builtin_amdgcn_readfirstlane(rr);
-    const int hit = (lane == lpv) ? rr : -1;
-    {
-      lds_double* dst = (lane == lpv) ? s_piv : s_junk + lane;
+    const double y0 = (q < NRHS && row >= 0) ? (double)yq[row] : 0.0;
+    P[t] = st[t].load(kb, q);
+    R4[t] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
-      for (int r = 0; r < R; ++r)
-        if (rr == r) dst[0] = s.b1[r];
+    for (int s = 1; s <= NG; ++s) {
+      const double v = st[t].load(kb, 4 * s + q);
+      if (s % NG < 4) R4[t][s % NG < 4 ? s % NG : 0] = v;
+      else RX[NX ? t : 0] = v;
     }
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    const double pb = s_piv[0];
-    Y[j] = pb;
+    if constexpr (Y16) R4[t][YR] = y0;
+    else Y[t] = y0;
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const double m = (j >= s.fc[r] && s.row[r] > j) ? s.w[r][t] : 0.0;
-      s.b1[r] = fma(-m, pb, s.b1[r]);
-      s.w[r][t] = ((s.vmask[r] >> t) & 1u) ? s.nk[r][t] : 0.0;
+    for (int s = 0; s < NG; ++s) {
+      st[t].advance(rt, NG + 1 + s, n, bw);
+      F[t][s] = st[t].load(kb, 4 * (NG + 1 + s) + q);
     }
-    if (lane == lpv) {
+  }
+  // Whole rounds of NG blocks (the ring positions are constants); a block past the last row
+  // factorises the identity on empty tiles and its stores fall past the end.  An exit inside a
+  // round would put register copies, and so a wait for every load ahead, on the loop edge.
+  const int nb = (n + 3) >> 2;
+  for (int g0 = 0; g0 < nb; g0 += NG) {
 #pragma unroll
-      for (int r = 0; r < R; ++r) {
-        if (hit == r) {
-          const int nr = s.nrow[r];
-          s.row[r] = nr;
-          s.vmask[r] = 0u;
-          const int q = nr >= 0 ? nr : 0;
-          s.b1[r] = (nr >= 0) ? Y[q] : 0.0;
-          row_enter(make_int2(s_succ[2 * q], s_succ[2 * q + 1]), nr, s.fc[r], s.off[r], s.nrow[r]);
+    for (int u = 0; u < NG; ++u) {
+      const int gb = g0 + u;
+      // --- publish the pivot rows: column col, row k of the block at piv[4 col + k]; the columns
+      // are the panel, the ring groups in order and the right-hand sides.  Rows past n - 1 are
+      // rows of the identity.
+      if (4 * gb + 4 > n) {
+        for (int e = lane; e < 16 * (NG + 2); e += 64)
+          if (4 * gb + (e & 3) >= n) piv[e] = (e >> 2) == (e & 3) ? 1.0 : 0.0;
+      }
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if ((crow[t] >> 2) == gb) {
+          lds_double* pk = piv + 4 * q + (crow[t] & 3);
+          pk[0] = P[t];
+#pragma unroll
+          for (int r = 0; r < NG; ++r) pk[16 * (r > u ? r - u : r - u + NG)] = r < 4 ? R4[t][r < 4 ? r : 0] : RX[NX ? t : 0];
+          pk[16 * (NG + 1)] = Y16 ? R4[t][YR] : Y[Y16 ? 0 : t];
+          // the slot's next row (already the one being read): no column of it has arrived yet
+          const int nr = st[t].row;
+          crow[t] = nr;
+          P[t] = 0.0;
+          R4[t] = v4d{0.0, 0.0, 0.0, 0.0};
+          if constexpr (NX > 0) RX[t] = 0.0;
+          const double y0 = (q < NRHS && nr >= 0) ? (double)yq[nr] : 0.0;
+          if constexpr (Y16) R4[t][YR] = y0;
+          else Y[t] = y0;
+          if constexpr (SL) {
+            cfc[t] = st[t].fc;
+            coff[t] = st[t].off8 >> 3;
+          }
         }
       }
-    }
+      // --- where the next group of every slot is read from
+      int nx_o[T];
 #pragma unroll
-    for (int r = 0; r < R; ++r) {
-      const int c = j + 2 * W;
-      const bool valid = (c >= s.fc[r]) && (c < s.row[r]);
-      const unsigned idx = valid ? (unsigned)(s.off[r] + c) : 0u;
-      s.nk[r][t] = lp[idx];
-      s.vmask[r] = (s.vmask[r] & ~(1u << t)) | ((valid ? 1u : 0u) << t);
-    }
-  }
-}
-
-template <int W, int R>
-__device__ void forward_solve_stored(const GridDev& g, const double* __restrict__ lprof_,
-                                     const int2* __restrict__ succ_, double* __restrict__ y_,
-                                     double* __restrict__ piv_, double* __restrict__ junk_, int lane) {
-  const int n = g.n;
-  const glb_double* lp = (const glb_double*)lprof_;
-  const lds_int* s_succ = (const lds_int*)succ_;
-  lds_double* Y = (lds_double*)y_;
-  lds_double* s_piv = (lds_double*)piv_;
-  lds_double* s_junk = (lds_double*)junk_;
-  FactorState<W, R> s;
-#pragma unroll
-  for (int r = 0; r < R; ++r) {
-    const int rw = g.slot_first[r * 64 + lane];
-    s.row[r] = rw;
-    const int q = rw >= 0 ? rw : 0;
-    row_enter(make_int2(s_succ[2 * q], s_succ[2 * q + 1]), rw, s.fc[r], s.off[r], s.nrow[r]);
-    s.b1[r] = (rw >= 0) ? Y[q] : 0.0;
-    s.vmask[r] = 0u;
-#pragma unroll
-    for (int k = 0; k < W; ++k) {
-      const int c0 = k, c1 = W + k;
-      double v0 = 0.0, a1 = 0.0;
-      if (c0 >= s.fc[r] && c0 < rw) v0 = lp[s.off[r] + c0];
-      if (c1 >= s.fc[r] && c1 < rw) {
-        a1 = lp[s.off[r] + c1];
-        s.vmask[r] |= 1u << k;
+      for (int t = 0; t < T; ++t) {
+        st[t].advance(rt, gb + 2 * NG + 1, n, bw);
+        nx_o[t] = st[t].at(4 * (gb + 2 * NG + 1) + q);
       }
-      s.w[r][k] = v0; s.nk[r][k] = a1;
-    }
-  }
-  __builtin_amdgcn_s_waitcnt(0x0F70);
-  const int nfull = n / W;
-  for (int ch = 0; ch < nfull; ++ch) forward_chunk<W, R, false>(ch * W, n, s, lp, s_succ, Y, s_piv, s_junk, lane);
-  if (nfull * W < n) forward_chunk<W, R, true>(nfull * W, n, s, lp, s_succ, Y, s_piv, s_junk, lane);
-}
-
-// Back substitution U z = y for the NRHS right-hand sides held in Y1/Y2(/Y3) (in place).
-// U rows are staged through LDS in chunks of 2W rows: all 64 lanes load the next chunk
-// (contiguous, coalesced) into registers while lanes 0..NRHS-1 (one right-hand side each)
-// sweep the current chunk from LDS; the window z[] holds z_{j+1..j+W-1} at static
-// positions j mod W (chunk bases are multiples of W).
-template <int W, int NRHS = 2>
-__device__ void back_substitute(int n, const double* __restrict__ urows, int WP, double* __restrict__ Y1,
-                                double* __restrict__ Y2, double* __restrict__ Y3, double* __restrict__ stg_,
-                                int lane) {
-  constexpr int CH = 2 * W;
-  constexpr int PER = (CH * ((W + 1) & ~1) + 63) / 64;   // doubles per lane per chunk
-  const int csize = CH * WP;
-  // Y1, Y2 and stg are in LDS: say so, so that the accesses are LDS instructions (counted
-  // apart from the global loads of the next chunk) rather than generic ones
-  typedef __attribute__((address_space(3))) double lds_double;
-  lds_double* Y = (lds_double*)(lane == 0 ? Y1 : (lane == 1 || NRHS < 3) ? Y2 : Y3);
-  lds_double* stg = (lds_double*)stg_;
-  double z[W];
+      wave_lds_fence();
+      const lds_v4d* pc = (const lds_v4d*)piv;
+      // the column of U this lane supplies: ring register m (or the right-hand sides)
+      const v4d vc = pc[4 * (m < NG ? (m > u ? m - u : m - u + NG) : NG + 1) + qq];
+      v4d vx[NX + 1];
 #pragma unroll
-  for (int k = 0; k < W; ++k) z[k] = 0.0;
-  const int nch = (n + CH - 1) / CH;
-  double buf[PER];
-  {
-    const int base = (nch - 1) * CH * WP;
-    const int lim = n * WP;
+      for (int x = 0; x < NX; ++x) vx[x] = pc[4 * (4 + x > u ? 4 + x - u : 4 + x - u + NG) + i4];
+      if constexpr (!Y16) vx[NX] = pc[4 * (NG + 1) + i4];
+      PivotBlock pb;
+      pb.factor(pc[0], pc[1], pc[2], pc[3]);
+      // column i4 of U11^-1; this lane's entry is row q of it
+      v4d xi;
+      xi[3] = i4 == 3 ? pb.r3 : 0.0;
+      xi[2] = fma(-pb.u23, xi[3], i4 == 2 ? 1.0 : 0.0) * pb.r2;
+      xi[1] = fma(-pb.u12, xi[2], fma(-pb.u13, xi[3], i4 == 1 ? 1.0 : 0.0)) * pb.r1;
+      xi[0] = fma(-pb.u01, xi[1], fma(-pb.u02, xi[2], fma(-pb.u03, xi[3], i4 == 0 ? 1.0 : 0.0))) * pb.r0;
+      const double ui = pick4(xi, q);
+      const double nu = -pick4(lower_apply(pb.l10, pb.l20, pb.l21, pb.l30, pb.l31, pb.l32, vc), q);
+      double nx[NX + 1];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const int o = lane + 64 * e;
-      const int gi = base + o;
-      buf[e] = urows[(o < csize && gi < lim) ? gi : 0];
-    }
+      for (int x = 0; x < NX + (Y16 ? 0 : 1); ++x)
+        nx[x] = -pick4(lower_apply(pb.l10, pb.l20, pb.l21, pb.l30, pb.l31, pb.l32, vx[x]), q);
+      // --- multipliers of every tile, then the updates (independent products back to back)
+      double l[T];
 #pragma unroll
-    for (int e = 0; e < PER; ++e) {
-      const int o = lane + 64 * e;
-      if (o < csize) stg[o] = buf[e];
-    }
-  }
-  __syncthreads();
-  for (int c = nch - 1; c >= 0; --c) {
-    if (c > 0) {
-      const int base = (c - 1) * CH * WP;
+      for (int t = 0; t < T; ++t) l[t] = mfma4(ui, P[t], 0.0);
 #pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int o = lane + 64 * e;
-        buf[e] = urows[base + (o < csize ? o : 0)];
+      for (int t = 0; t < T; ++t) {
+        R4[t] = mfma16(nu, l[t], R4[t]);
+        if constexpr (NX > 0) RX[t] = mfma4(nx[0], l[t], RX[t]);
+        if constexpr (!Y16) Y[t] = mfma4(nx[NX], l[t], Y[t]);
       }
-    }
-    if (lane < NRHS) {
-      const int j0 = c * CH;
+      // --- U rows, U11^-1, eliminated right-hand sides
+      buf_store(ub, uo[u] + gb * (4 * WP * 8), nu);
+      buf_store(ub, ui_o + gb * (4 * WP * 8), ui);
 #pragma unroll
-      for (int tt = CH - 1; tt >= 0; --tt) {
-        const int j = j0 + tt;
-        if (j < n) {
-          const lds_double* ur = stg + tt * WP;
-          double sum = Y[j];
+      for (int x = 0; x < NX; ++x) buf_store(ub, ux[u * NX + x] + gb * (4 * WP * 8), nx[x]);
+      const int j = 4 * gb + q;
+      if (ywl && j < n) yw[j] = Y16 ? -nu : -nx[NX];
+      if constexpr (SL) {
 #pragma unroll
-          for (int k = W - 1; k >= 1; --k) sum = fma(-ur[k], z[(tt + k) % W], sum);
-          const double zj = sum * ur[0];
-          z[tt % W] = zj;
-          Y[j] = zj;
+        for (int t = 0; t < T; ++t)
+          if (crow[t] >= 0 && 4 * gb + q >= cfc[t]) lout[coff[t] + 4 * gb + q] = l[t];
+        // the strict lower part of the pivot block's own factor
+        if (a16 < q && j < n) {
+          const int c = 4 * gb + a16;
+          if (c >= (rt[2 * j] & 0xffff)) {
+            const double lv = q == 1 ? pb.l10 : q == 2 ? (a16 == 0 ? pb.l20 : pb.l21)
+                                                       : (a16 == 0 ? pb.l30 : a16 == 1 ? pb.l31 : pb.l32);
+            lout[rt[2 * j + 1] + c] = lv;
+          }
         }
       }
-    }
-    __syncthreads();
-    if (c > 0) {
+      // --- the next panel, the group read NG blocks ago into the ring, and the next read
+      constexpr int RN = NG;
 #pragma unroll
-      for (int e = 0; e < PER; ++e) {
-        const int o = lane + 64 * e;
-        if (o < csize) stg[o] = buf[e];
+      for (int t = 0; t < T; ++t) {
+        const int r = (u + 1) % RN;
+        if (r < 4) {
+          P[t] = R4[t][r < 4 ? r : 0];
+          R4[t][r < 4 ? r : 0] = F[t][u];
+        } else {
+          P[t] = RX[NX ? t : 0];
+          RX[NX ? t : 0] = F[t][u];
+        }
+        F[t][u] = buf_load(kb, nx_o[t]);
       }
     }
-    __syncthreads();
+  }
+}
+
+// Forward solve L y = b with the unit lower factor stored by factor_tiles<SL = true>, one
+// right-hand side in Y (entry values in, eliminated values out; in place).  The same slots and
+// blocks with the stored multipliers streamed as panels: per tile and block one load and one
+// 4x4x4 product.  The order of the operations on a row is the factorisation's.
+template <int W, int T>
+__device__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof, const int2* __restrict__ rt_,
+                              double* __restrict__ y_, double* __restrict__ piv_, int lane) {
+  lane = fresh_lane(lane);
+  constexpr int NG = trail_groups<W>(), PF = 4;
+  const int n = g.n, bw = g.bw;
+  const int q = lane >> 4, a16 = lane & 15;
+  const ProfileBuf lb = profile_buf(lprof, g.P);
+  const lds_int* rt = (const lds_int*)rt_;
+  lds_double* yl = (lds_double*)y_;
+  lds_double* piv = (lds_double*)piv_;
+  SlotRow<NG, true> st[T];
+  int crow[T];
+  double Y[T], F[T][PF], D[PF];
+  // entry (q, a16) of the block's own unit lower factor, a16 < q
+  auto diag = [&](int gb) -> double {
+    const int j = 4 * gb + q, c = 4 * gb + a16;
+    const int jr = min(j, n - 1);
+    const bool ok = a16 < q && j < n && c >= (rt[2 * jr] & 0xffff);
+    return buf_load(lb, ok ? 8 * (rt[2 * jr + 1] + c) : kOutside);
+  };
+#pragma unroll
+  for (int t = 0; t < T; ++t) {
+    const int slot = 16 * t + a16;
+    const int row = slot < g.nslots ? g.slot_first[slot] : -1;
+    st[t].enter(rt, row, n, bw);
+    crow[t] = row;
+    Y[t] = row >= 0 ? (double)yl[row] : 0.0;
+  }
+#pragma unroll
+  for (int s = 0; s < PF; ++s) {
+#pragma unroll
+    for (int t = 0; t < T; ++t) {
+      st[t].advance(rt, s, n, bw);
+      F[t][s] = st[t].load(lb, 4 * s + q);
+    }
+    D[s] = diag(s);
+  }
+  const int nb = (n + 3) >> 2;
+  for (int g0 = 0; g0 < nb; g0 += PF) {
+#pragma unroll
+    for (int u = 0; u < PF; ++u) {
+      const int gb = g0 + u;
+      if (lane < 4 && 4 * gb + lane >= n) piv[lane] = 0.0;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        if ((crow[t] >> 2) == gb) {
+          if (q == 0) piv[crow[t] & 3] = Y[t];
+          const int nr = rt[2 * crow[t]] >> 16;
+          crow[t] = nr;
+          Y[t] = nr >= 0 ? (double)yl[nr] : 0.0;
+        }
+      }
+      int nx_o[T];
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        st[t].advance(rt, gb + PF, n, bw);
+        nx_o[t] = st[t].at(4 * (gb + PF) + q);
+      }
+      wave_lds_fence();
+      const v4d v = *(const lds_v4d*)piv;
+      auto rl = [&](int k, int c) -> double {
+        const int l = 16 * k + c;
+        return __hiloint2double(__builtin_amdgcn_readlane(__double2hiint(D[u]), l),
+                                __builtin_amdgcn_readlane(__double2loint(D[u]), l));
+      };
+      const v4d y = lower_apply(rl(1, 0), rl(2, 0), rl(2, 1), rl(3, 0), rl(3, 1), rl(3, 2), v);
+      const double yk = pick4(y, q);
+      if (a16 == 0 && 4 * gb + q < n) yl[4 * gb + q] = yk;
+#pragma unroll
+      for (int t = 0; t < T; ++t) {
+        Y[t] = mfma4(-yk, F[t][u], Y[t]);
+        F[t][u] = buf_load(lb, nx_o[t]);
+      }
+      D[u] = diag(gb + PF);
+    }
+  }
+}
+
+// Back substitution U z = y for the NRHS right-hand sides held in Y1/Y2(/Y3) (in place), blocks
+// of four rows: z_g = U11^-1 (y_g - sum_s U_(g,g+s) z_(g+s)), every product one 4x4x4 whose
+// result is the next one's operand as it stands; only two of them wait on the block before.
+template <int W, int NRHS>
+__device__ void back_tiles(const GridDev& g, const double* __restrict__ urows, double* __restrict__ Y1,
+                           double* __restrict__ Y2, double* __restrict__ Y3, int lane) {
+  lane = fresh_lane(lane);
+  constexpr int NG = trail_groups<W>(), WP = (W + 1) & ~1, PD = NG <= 3 ? 2 * NG : NG;
+  const int n = g.n, bw = g.bw;
+  const int q = lane >> 4, j4 = lane & 3, b4 = (lane >> 2) & 3;
+  const ProfileBuf ub = profile_buf(urows, n * WP);
+  lds_double* yj = (lds_double*)(j4 == 0 || NRHS < 2 ? Y1 : (j4 == 1 || NRHS < 3) ? Y2 : Y3);
+  const bool live = j4 < NRHS;
+  // operand A[i][k]: lane i + 4 b + 16 k; byte offsets inside a block's four rows
+  int uo[NG + 1];
+  uo[0] = q >= j4 ? (j4 * WP + q - j4) * 8 : kOutside;
+#pragma unroll
+  for (int s = 1; s <= NG; ++s) uo[s] = 4 * s + q - j4 <= bw ? (j4 * WP + 4 * s + q - j4) * 8 : kOutside;
+  const int nb = (n + 3) >> 2;
+  const int nu = (nb + PD - 1) / PD * PD;             // blocks past the last read as zero rows
+  double A[PD][NG + 1], Z[NG];
+#pragma unroll
+  for (int s = 0; s < NG; ++s) Z[s] = 0.0;
+#pragma unroll
+  for (int u = 0; u < PD; ++u)
+#pragma unroll
+    for (int s = 0; s <= NG; ++s) A[u][s] = buf_load(ub, uo[s] + (nu - PD + u) * (4 * WP * 8));
+  auto rhs = [&](int gb) -> double {
+    const int j = 4 * gb + q;
+    const double v = yj[min(max(j, 0), n - 1)];
+    return (live && j < n) ? v : 0.0;
+  };
+  double yn = rhs(nu - 1);
+  for (int g0 = nu - PD; g0 >= 0; g0 -= PD) {
+#pragma unroll
+    for (int u = PD - 1; u >= 0; --u) {
+      const int gb = g0 + u;
+      double acc = yn;
+      yn = rhs(gb - 1);
+#pragma unroll
+      for (int s = NG; s >= 1; --s) acc = mfma4(A[u][s], Z[(u + s) % NG], acc);
+      const double z = mfma4(A[u][0], acc, 0.0);
+      Z[u % NG] = z;
+      if (b4 == 0 && live && 4 * gb + q < n) yj[4 * gb + q] = z;
+      // rows of block gb - PD; a negative block is past the end as an unsigned offset
+#pragma unroll
+      for (int s = 0; s <= NG; ++s) A[u][s] = buf_load(ub, gb >= PD ? uo[s] + (gb - PD) * (4 * WP * 8) : kOutside);
+    }
+  }
+}
+
+// The radial mass Cholesky factor staged for mass_solve, rows of four: lc[4 q + d] for d <= q % 4
+// is entry (q, q - d) of the inverse of the 4 x 4 diagonal block that row q lies in, for d > q % 4
+// the factor's own entry L[q, q - d] (zero before the first column).  One lane per block.
+__device__ void stage_mass(const GridDev& g, double* __restrict__ lc, int lane) {
+  lane = fresh_lane(lane);
+  const int nb = (g.npr + 3) >> 2;
+  for (int b = lane; b < nb; b += 64) {
+    double L[4][4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const int q = 4 * b + i;
+#pragma unroll
+      for (int d = 0; d < 4; ++d) {
+        const double v = g.mchol[(size_t)(min(q, g.npr - 1) * g.ns) * 4 + d];
+        L[i][d] = q >= g.npr ? (d == 0 ? 1.0 : 0.0) : (q - d >= 0 ? v : 0.0);
+      }
+    }
+    const double i0 = 1.0 / L[0][0], i1 = 1.0 / L[1][0], i2 = 1.0 / L[2][0], i3 = 1.0 / L[3][0];
+    const double x10 = -(L[1][1] * i0) * i1;
+    const double x21 = -(L[2][1] * i1) * i2;
+    const double x20 = -fma(L[2][2], i0, L[2][1] * x10) * i2;
+    const double x32 = -(L[3][1] * i2) * i3;
+    const double x31 = -fma(L[3][2], i1, L[3][1] * x21) * i3;
+    const double x30 = -fma(L[3][3], i0, fma(L[3][2], x10, L[3][1] * x20)) * i3;
+    const double o[4][4] = {{i0, L[0][1], L[0][2], L[0][3]},
+                            {i1, x10, L[1][2], L[1][3]},
+                            {i2, x21, x20, L[2][3]},
+                            {i3, x32, x31, x30}};
+#pragma unroll
+    for (int i = 0; i < 4; ++i)
+      if (4 * b + i < g.npr)
+#pragma unroll
+        for (int d = 0; d < 4; ++d) lc[16 * b + 4 * i + d] = o[i][d];
+  }
+}
+
+// In-place solve M z = b in the permuted order: every l-block (stride ns) is the reversed radial
+// mass block with half bandwidth 3, lc from stage_mass.  Blocks of four rows as 4x4x4 matrix
+// products, the harmonics in the columns (ns <= 16): y_g = D_g (b_g - S_g y_(g-1)), then
+// z_g = D_g^T (y_g - S_(g+1)^T z_(g+1)); the result of a product is the next one's operand as it
+// stands, so a block waits on two products (about 260 dependent steps of four multiply-adds and
+// their LDS reads before).
+__device__ void mass_solve(int ns, int npr, const double* __restrict__ lc_, double* __restrict__ b_, int lane) {
+  lane = fresh_lane(lane);
+  const lds_double* lc = (const lds_double*)lc_;
+  lds_double* b = (lds_double*)b_;
+  const int i = lane & 3, k = lane >> 4, col = lane & 15;
+  const int nb = (npr + 3) >> 2;
+  // operands A[i][k]: -S_g (row 4 g + i, offset 4 + i - k, when i < k) and D_g (offset i - k)
+  auto opS = [&](int g) -> double {
+    const int r = 4 * g + i;
+    const double v = lc[4 * min(r, npr - 1) + ((4 + i - k) & 3)];
+    return (i < k && r < npr && g > 0) ? -v : 0.0;
+  };
+  auto opD = [&](int g) -> double {
+    const int r = 4 * g + i;
+    const double v = lc[4 * min(r, npr - 1) + ((i - k) & 3)];
+    return (i >= k && r < npr) ? v : 0.0;
+  };
+  // transposed: -S_(g+1)^T (row 4 g + 4 + k, offset 4 + k - i, when k < i) and D_g^T
+  auto opSt = [&](int g) -> double {
+    const int r = 4 * g + 4 + k;
+    const double v = lc[4 * min(r, npr - 1) + ((4 + k - i) & 3)];
+    return (k < i && r < npr) ? -v : 0.0;
+  };
+  auto opDt = [&](int g) -> double {
+    const int r = 4 * g + k;
+    const double v = lc[4 * min(r, npr - 1) + ((k - i) & 3)];
+    return (k >= i && r < npr) ? v : 0.0;
+  };
+  auto rhs = [&](int g) -> double {
+    const int r = 4 * g + k;
+    const double v = b[max(0, min(r, npr - 1)) * ns + min(col, ns - 1)];
+    return (r < npr && col < ns) ? v : 0.0;
+  };
+  auto put = [&](int g, double v) {
+    const int r = 4 * g + k;
+    if (r < npr && col < ns) b[r * ns + col] = v;
+  };
+  double y = 0.0, S = opS(0), D = opD(0), v = rhs(0);
+  for (int g = 0; g < nb; ++g) {
+    const int gn = min(g + 1, nb - 1);
+    const double Sn = opS(gn), Dn = opD(gn), vn = rhs(gn);
+    y = mfma4(D, mfma4(S, y, v), 0.0);
+    put(g, y);
+    S = Sn; D = Dn; v = vn;
+  }
+  double z = 0.0;
+  S = opSt(nb - 1); D = opDt(nb - 1); v = rhs(nb - 1);
+  for (int g = nb - 1; g >= 0; --g) {
+    const int gn = max(g - 1, 0);
+    const double Sn = opSt(gn), Dn = opDt(gn), vn = rhs(gn);
+    z = mfma4(D, mfma4(S, z, v), 0.0);
+    put(g, z);
+    S = Sn; D = Dn; v = vn;
   }
 }
 
@@ -653,19 +888,32 @@ __global__ void k_prepare0d(GridDev g, BatchDev b) {
   }
 }
 
-// LDS: four n-vectors R0..R3 (a pad after R2 so that R1..R2 can hold the 4*npr mass
-// Cholesky coefficients), the back-substitution stage STG[2W*WP], the pivot row
-// PIV[PIVN], then the row table (int2 per row).
+// LDS: the published pivot block PIV first (32-byte aligned), four n-vectors R0..R3, the staged
+// mass factor LC (4*npr doubles), then the row table (int2 per row).  Where LC would cost a
+// wavefront per CU or pass 64 KB it shares R1..R2 (with a pad after R2) and is staged again for
+// every residual.
 __host__ __device__ __forceinline__ int zpad(int n, int npr) { return (4 * npr > 2 * n) ? (4 * npr - 2 * n) : 0; }
 
 template <int W>
-__host__ __device__ constexpr int piv_len() { return (W + 4) & ~1; }   // U row + three right-hand sides
+__host__ __device__ constexpr int piv_len() { return 16 * (trail_groups<W>() + 2); }
 
+// Waves per SIMD the register state of T tiles leaves room for (a tile holds 2 NG + 2 doubles and
+// its read position per lane); one wave may also use the accumulation registers.
+template <int W, int T>
+constexpr int tile_waves() { return T * (trail_groups<W>() + 2) <= 30 ? 2 : 1; }
+
+// `vecs` n-vectors beside R1 and R2; sets g.keep_mass
 template <int W>
-size_t newton_lds_bytes(int n, int npr) {
-  constexpr int WP = (W + 1) & ~1;
-  return (size_t)(4 * n + zpad(n, npr) + 2 * W * WP + piv_len<W>()) * sizeof(double) + (size_t)n * sizeof(int2);
+size_t newton_lds_bytes(GridDev& g, int vecs) {
+  const size_t rest = (size_t)((vecs + 2) * g.n + piv_len<W>()) * sizeof(double) + (size_t)g.n * sizeof(int2);
+  const size_t keep = rest + (size_t)4 * g.npr * sizeof(double), share = rest + (size_t)zpad(g.n, g.npr) * sizeof(double);
+  constexpr size_t cu = 160 * 1024;
+  g.keep_mass = keep <= 64 * 1024 && (cu / keep >= 8 || cu / keep == cu / share);
+  return g.keep_mass ? keep : share;
 }
+
+// Profiles and U rows are read through 32-bit byte offsets below kOutside.
+inline bool fits_offsets(const GridDev& g) { return g.P > 0 && g.P < kOutside / 8 && g.n < 32768; }
 
 // |(I - uhat uhat^T) v| for v = ca A + cx X + cp P (two passes: explicit projection, no
 // |v|^2 - (u.v)^2 cancellation); P may be null (cp ignored).
@@ -715,20 +963,18 @@ __device__ double proj_norm3(const double* A, double ca, const double* X, double
 //    combination, and a residual predicted from them is not; the true residual is.)
 // Global scratch rows of the instance (b.vec, kVecRows x n): 0 growth vector w, 1 x (the
 // base point of the line search), 2 M x, 3 y3, 4..10 unshifted K on the band of M, 11 p.
-template <int W, int R>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 : 2))) void k_newton0d(GridDev g, BatchDev b) {
-  extern __shared__ double lds[];
+template <int W, int T>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W, T>()))) void k_newton0d(GridDev g, BatchDev b) {
+  extern __shared__ __align__(32) double lds[];
   const int n = g.n, lane = threadIdx.x, inst = blockIdx.x;
   constexpr int WP = (W + 1) & ~1;
-  constexpr int PIVN = piv_len<W>();
-  double* R0 = lds;                                        // x; y3 -> delta -> p during a step
+  double* PIV = lds;                                       // published pivot block
+  double* R0 = PIV + piv_len<W>();                         // x; y3 -> delta -> p during a step
   double* R1 = R0 + n;                                     // M uhat -> z1
   double* R2 = R1 + n;                                     // M x -> z2
-  double* R3 = R2 + n + zpad(n, g.npr);                    // y3 -> T = M^-1 y3
-  double* STG = R3 + n;                                    // back-substitution stage
-  double* PIV = STG + 2 * W * WP;                          // published pivot row
-  int2* SC = reinterpret_cast<int2*>(PIV + PIVN);
-  double* LCH = R1;                                        // mass Cholesky stage (R1..R2 free)
+  double* LC = g.keep_mass ? R2 + n : R1;                  // staged mass factor (R1..R2 free in a residual)
+  double* R3 = R2 + n + (g.keep_mass ? 4 * g.npr : zpad(n, g.npr));   // y3 -> T = M^-1 y3
+  int2* SC = reinterpret_cast<int2*>(R3 + n);
 
   double* kprof = b.kprof + (size_t)inst * g.P;           // K, then K - mu M on the band of M
   const double* __restrict__ mprof = g.opprof + (size_t)(g.nop - 1) * g.P;
@@ -737,13 +983,15 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
   double* XG = WV + n;
   double* MXG = XG + n;
   double* Y3G = MXG + n;
-  double* KB0 = Y3G + n;                                   // [7][n] unshifted K on the band of M
+  double* KB0 = Y3G + n;                                   // [n][7] unshifted K on the band of M
   double* PG = KB0 + 7 * n;                                // the step p
   double* urows = b.urows + (size_t)inst * n * WP;
 
   // ---------------- row table into LDS, initial iterate (original (n,B) layout -> permuted)
   fill_rowtab(g, SC, lane);
+  if (g.keep_mass) stage_mass(g, LC, lane);
   for (int i = lane; i < n; i += 64) R0[i] = b.x[(size_t)orig_index(i, g.ns, g.npr) * b.B + inst];
+  const ProfileBuf mb = profile_buf(mprof, g.P), kpb = profile_buf(kprof, g.P), kbb = profile_buf(KB0, 7 * n);
   __syncthreads();
 
   // residual at the point in R0 for the coefficient cq: x normalised in place, K' in the
@@ -754,56 +1002,59 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
     for (int i = lane; i < n; i += 64) R0[i] = R0[i] / ux;
     __syncthreads();
     const double mu = dot_dd(WV, R0, n, lane);
-    for (int i = lane; i < n; i += 64) {
-      const int2 rtb = SC[i];
-      const int base = rtb.y;
-      const int fc = rtb.x & 0xffff;
-      const int lc = min(i + g.bw, n - 1);
-      double kv[7], mv[7];
+    // the band of M, lane d of eight on offset d - 3 of a row, eight rows to a pass and four
+    // passes' loads in flight
+    for (int i0 = lane >> 3; i0 - (lane >> 3) < n; i0 += 32) {
+      const int d = lane & 7;
+      double mv[4], kv[4];
+      int eo[4], bo[4];
 #pragma unroll
-      for (int d = 0; d < 7; ++d) {
-        const int c = i + (d - 3) * g.ns;
-        const bool ok = (c >= 0) && (c < n);
-        const int cc = ok ? c : i;                 // the diagonal: always in the row
-        mv[d] = ok ? mprof[base + cc] : 0.0;
-        kv[d] = first ? kprof[base + cc] : KB0[(size_t)d * n + i];
+      for (int u = 0; u < 4; ++u) {
+        const int i = i0 + 8 * u, c = i + (d - 3) * g.ns;
+        const bool ok = i < n && d < 7 && c >= 0 && c < n;
+        eo[u] = ok ? 8 * (SC[min(i, n - 1)].y + c) : kOutside;
+        bo[u] = ok ? 8 * (7 * i + d) : kOutside;
+        mv[u] = buf_load(mb, eo[u]);
+        kv[u] = first ? buf_load(kpb, eo[u]) : buf_load(kbb, bo[u]);
       }
-      double mx = 0.0, corr = 0.0;
 #pragma unroll
-      for (int d = 0; d < 7; ++d) {
-        const int c = i + (d - 3) * g.ns;
-        if ((c >= 0) && (c < n)) {
+      for (int u = 0; u < 4; ++u) {
 #pragma clang fp contract(off)
-          if (first) KB0[(size_t)d * n + i] = kv[d];
-          mx = fma(mv[d], R0[c], mx);
-          const double pm = mu * mv[d];
-          const double pe = fma(mu, mv[d], -pm);
-          const double hi = kv[d] - pm;                      // TwoSum(kv, -pm)
-          const double z = hi - kv[d];
-          const double lo = ((kv[d] - (hi - z)) + (-pm - z)) - pe;
-          const double kr = hi + lo;                         // K' rounded once
-          kprof[base + c] = kr;
-          corr = fma(lo - (kr - hi), R0[c], corr);           // K' - kr, to the residual
+        const int i = i0 + 8 * u, c = i + (d - 3) * g.ns;
+        const double xc = R0[max(0, min(c, n - 1))];         // weight zero outside the row
+        if (first) buf_store(kbb, bo[u], kv[u]);
+        const double pm = mu * mv[u];
+        const double pe = fma(mu, mv[u], -pm);
+        const double hi = kv[u] - pm;                        // TwoSum(kv, -pm)
+        const double z = hi - kv[u];
+        const double lo = ((kv[u] - (hi - z)) + (-pm - z)) - pe;
+        const double kr = hi + lo;                           // K' rounded once
+        buf_store(kpb, eo[u], kr);
+        double mx = mv[u] * xc, corr = (lo - (kr - hi)) * xc;  // K' - kr, to the residual
+        mx += dpp_move<kDppXor1>(mx);
+        corr += dpp_move<kDppXor1>(corr);
+        mx += dpp_move<kDppXor2>(mx);
+        corr += dpp_move<kDppXor2>(corr);
+        mx += dpp_move<kDppHalfMirror>(mx);
+        corr += dpp_move<kDppHalfMirror>(corr);
+        if (d == 0 && i < n) {
+          R3[i] = corr;
+          MXG[i] = mx;
         }
       }
-      double s = 0.0, e = 0.0;
-#pragma unroll 4
-      for (int c = fc; c <= lc; ++c) two_sum_acc(-kprof[base + c], R0[c], s, e);
-      e -= corr;
+    }
+    first = false;
+    __syncthreads();                                       // K' of every row before any row is summed
+    row_sums<true>(n, g.ns, g.npr, g.bw, g.P, SC, kprof, R0, lane, [&](int i, double s, double e) {
+      e -= R3[i];
       two_sum_acc(cq, g.muhat[i], s, e);
       const double y3 = s + e;
       R3[i] = y3;
       Y3G[i] = y3;
-      MXG[i] = mx;
-    }
-    first = false;
-    for (int e = lane; e < 4 * g.npr; e += 64) {
-      const int q = e >> 2, dd = e & 3;
-      const double v = g.mchol[(size_t)(q * g.ns) * 4 + dd];
-      LCH[e] = (dd == 0) ? 1.0 / v : ((q - dd >= 0) ? v : 0.0);
-    }
+    });
+    if (!g.keep_mass) stage_mass(g, LC, lane);
     __syncthreads();
-    mass_solve(g.ns, g.npr, LCH, R3, lane);
+    mass_solve(g.ns, g.npr, LC, R3, lane);
     __syncthreads();
     return proj_norm3(R3, 1.0, R0, 0.0, nullptr, 0.0, UH, n, lane);
   };
@@ -832,9 +1083,9 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
       R2[i] = MXG[i];
     }
     __syncthreads();
-    factor_forward<W, R, false, 3>(g, kprof, SC, R1, R2, R0, PIV, STG, urows, WP, lane);
+    factor_tiles<W, T, false, 3>(g, kprof, SC, R1, R2, R0, PIV, urows, lane);
     __syncthreads();
-    back_substitute<W, 3>(n, urows, WP, R1, R2, R0, STG, lane);
+    back_tiles<W, 3>(g, urows, R1, R2, R0, lane);
     __syncthreads();
     // ---- step p = delta + a z1 + b z2
     double s11 = 0.0, s12 = 0.0, s13 = 0.0, wz1 = 0.0, wz2 = 0.0, wz3 = 0.0;
@@ -958,189 +1209,7 @@ __global__ void k_ee_profile_add(GridDev g, BatchDev b, EEDev e) {
   }
 }
 
-// The preconditioner with the factorisation kept: once per Newton step, L (multipliers, in
-// the profile positions of the instance, lprof) and U (urows) of K_x - mu M, and
-// z1 = (K_x - mu M)^-1 M uhat with s1 = uhat.z1 (permuted order); then every application
-// is a mass product, one profile forward solve and one back substitution.
-template <int W, int R>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 : 2))) void k_ee_factor(
-    GridDev g, BatchDev b, const int* __restrict__ active, double* __restrict__ lprof, double* __restrict__ z1,
-    double* __restrict__ s1) {
-  extern __shared__ double lds[];
-  const int n = g.n, lane = threadIdx.x, inst = blockIdx.x;
-  if (active && !active[inst]) return;
-  constexpr int WP = (W + 1) & ~1;
-  constexpr int PIVN = piv_len<W>();
-  double* Z1 = lds + n;
-  double* Z2 = Z1 + n;
-  double* AV = Z2 + n + zpad(n, g.npr);
-  double* STG = AV + n;
-  double* PIV = STG + 2 * W * WP;
-  int2* SC = reinterpret_cast<int2*>(PIV + PIVN);
-  const double* kprof = b.kprof + (size_t)inst * g.P;
-  double* urows = b.urows + (size_t)inst * n * WP;
-  fill_rowtab(g, SC, lane);
-  for (int i = lane; i < n; i += 64) {
-    Z1[i] = g.muhat[i];
-    Z2[i] = 0.0;
-  }
-  __syncthreads();
-  factor_forward<W, R, true>(g, kprof, SC, Z1, Z2, nullptr, PIV, STG, urows, WP, lane, lprof + (size_t)inst * g.P);
-  __syncthreads();
-  back_substitute<W>(n, urows, WP, Z1, Z2, nullptr, STG, lane);
-  __syncthreads();
-  const double su = dot(g.uhat, Z1, n, lane);
-  for (int i = lane; i < n; i += 64) z1[(size_t)inst * n + i] = Z1[i];
-  if (lane == 0) s1[inst] = su;
-}
-
-// Forward solve with the stored unit lower factor, row by row; the profile rows are staged
-// through LDS in chunks of whole rows (at most LBUF entries) with the next chunk's loads in
-// flight (registers) while the current chunk is swept, so the sweep waits on LDS only.
-constexpr int LBUF = 1024;
-
-template <int W>
-__global__ __launch_bounds__(64) void k_ee_precond_apply(GridDev g, BatchDev b, const int* __restrict__ active,
-                                                         const double* __restrict__ lprof,
-                                                         const double* __restrict__ z1, const double* __restrict__ s1,
-                                                         const double* __restrict__ v, double* __restrict__ out,
-                                                         double* __restrict__ outT) {
-  extern __shared__ double lds[];
-  const int n = g.n, lane = threadIdx.x, inst = blockIdx.x;
-  if (active && !active[inst]) return;
-  constexpr int WP = (W + 1) & ~1;
-  constexpr int PER = LBUF / 64;
-  double* VV = lds;
-  double* Y1 = VV + n;
-  double* Y2 = Y1 + n;
-  double* STG = Y2 + n;
-  double* SB = STG + 2 * W * WP;                 // two stages of LBUF
-  int* PO = reinterpret_cast<int*>(SB + 2 * LBUF);
-  short* FC = reinterpret_cast<short*>(PO + (n + 1));
-  const double* __restrict__ mprof = g.opprof + (size_t)(g.nop - 1) * g.P;
-  const double* __restrict__ L = lprof + (size_t)inst * g.P;
-  const double* urows = b.urows + (size_t)inst * n * WP;
-  for (int i = lane; i < n; i += 64) {
-    VV[i] = v[(size_t)inst * n + orig_index(i, g.ns, g.npr)];
-    Y1[i] = 0.0;
-    FC[i] = (short)g.first_col[i];
-  }
-  for (int i = lane; i <= n; i += 64) PO[i] = g.prof_off[i];
-  __syncthreads();
-  mass_matvec(n, g.ns, mprof, g.first_col, g.prof_off, VV, Y2, lane);
-  // rows [r0, r_end(r0)) fit one stage (every row has at most LBUF entries: checked at launch)
-  auto r_end = [&](int r0) {
-    int r1 = r0 + 1;
-    while (r1 < n && PO[r1 + 1] - PO[r0] <= LBUF) ++r1;
-    return r1;
-  };
-  double reg[PER];
-  int r0 = 0, r1 = r_end(0), st = 0;
-  {
-    const int e0 = PO[0], cnt = PO[r1] - e0;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int o = lane + 64 * k;
-      if (o < cnt) SB[o] = L[e0 + o];
-    }
-  }
-  __syncthreads();
-  while (r0 < n) {
-    const int r2 = (r1 < n) ? r_end(r1) : n;
-    const int e1 = PO[r1], cnt1 = PO[r2] - e1;    // cnt1 = 0 after the last stage
-    if (cnt1 > 0) {
-#pragma unroll
-      for (int k = 0; k < PER; ++k) {
-        const int o = lane + 64 * k;
-        reg[k] = L[e1 + (o < cnt1 ? o : 0)];
-      }
-    }
-    const double* S = SB + st * LBUF;
-    const int base = PO[r0];
-    if (PO[r1] - base > 128 * (r1 - r0)) {
-      // long rows (more than 128 entries on average, few rows per stage): each row's sum over
-      // its columns left of the diagonal is split across the 64 lanes and reduced
-      for (int i = r0; i < r1; ++i) {
-        const int fc = FC[i], off = PO[i] - base - fc;
-        double acc = 0.0;
-        for (int j = fc + lane; j < i; j += 64) acc = fma(-S[off + j], Y2[j], acc);
-        acc = wave_sum(acc);
-        if (lane == 0) Y2[i] += acc;
-        __syncthreads();
-      }
-    } else
-    // blocks of 64 rows, lane t owning row blk0 + t: first the columns left of the block
-    // (values final), then the unit lower triangle of the block, one column per step with
-    // the finished value broadcast from its lane
-    for (int blk0 = r0; blk0 < r1; blk0 += 64) {
-      const int nb = min(64, r1 - blk0);
-      const int i = blk0 + lane;
-      const bool act = lane < nb;
-      const int fc = act ? (int)FC[i] : 0;
-      const int off = act ? PO[i] - base - fc : 0;
-      double acc = act ? Y2[i] : 0.0;
-      if (act)
-        for (int j = fc; j < blk0; ++j) acc = fma(-S[off + j], Y2[j], acc);
-      for (int t = 0; t < nb; ++t) {
-        const int j = blk0 + t;
-        const int lo = __builtin_amdgcn_readlane(__double2loint(acc), t);
-        const int hi = __builtin_amdgcn_readlane(__double2hiint(acc), t);
-        const double yj = __hiloint2double(hi, lo);
-        if (act && i > j && j >= fc) acc = fma(-S[off + j], yj, acc);
-      }
-      if (act) Y2[i] = acc;
-      __syncthreads();
-    }
-    double* D = SB + (st ^ 1) * LBUF;
-#pragma unroll
-    for (int k = 0; k < PER; ++k) {
-      const int o = lane + 64 * k;
-      if (o < cnt1) D[o] = reg[k];
-    }
-    __syncthreads();
-    st ^= 1;
-    r0 = r1;
-    r1 = r2;
-  }
-  back_substitute<W>(n, urows, WP, Y1, Y2, nullptr, STG, lane);
-  __syncthreads();
-  const double c = -dot(g.uhat, Y2, n, lane) / s1[inst];
-  const double* Z1 = z1 + (size_t)inst * n;
-  for (int i = lane; i < n; i += 64) {
-    const int o = orig_index(i, g.ns, g.npr);
-    const double z = fma(c, Z1[i], Y2[i]);
-    out[(size_t)inst * n + o] = z;
-    if (outT) outT[(size_t)o * b.B + inst] = z;
-  }
-}
-
-template <int W, int R>
-int launch_ee_factor(const GridDev& g, const BatchDev& b, const int* active, double* lprof, double* z1, double* s1,
-                     hipStream_t stream) {
-  const size_t lds = newton_lds_bytes<W>(g.n, g.npr);
-  if (lds > 64 * 1024) return BZ_EINVAL;
-  hipLaunchKernelGGL((k_ee_factor<W, R>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1);
-  BZ_LAUNCH_CHECK();
-  return BZ_OK;
-}
-
-template <int W>
-int launch_ee_apply(const GridDev& g, const BatchDev& b, const int* active, const double* lprof, const double* z1,
-                    const double* s1, const double* v, double* out, double* outT, hipStream_t stream) {
-  constexpr int WP = (W + 1) & ~1;
-  const size_t lds = (size_t)(3 * g.n + 2 * W * WP + 2 * LBUF) * sizeof(double) + (size_t)(g.n + 1) * sizeof(int) +
-                     (size_t)g.n * sizeof(short);
-  if (lds > 64 * 1024 || g.max_row > LBUF) return BZ_EINVAL;
-  hipLaunchKernelGGL((k_ee_precond_apply<W>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1, v, out,
-                     outT);
-  BZ_LAUNCH_CHECK();
-  return BZ_OK;
-}
-
-template <int W, int R>
-int launch_newton(const GridDev& g, const BatchDev& b, hipStream_t stream, const EEDev* ee = nullptr) {
-  const size_t lds = newton_lds_bytes<W>(g.n, g.npr);
-  if (lds > 64 * 1024) return BZ_EINVAL;
+inline int launch_prepare(const GridDev& g, const BatchDev& b, hipStream_t stream, const EEDev* ee = nullptr) {
   const long work = (long)b.B * g.P;
   const int blocks = (int)std::min<long>((work + 255) / 256, 8192);
   hipLaunchKernelGGL(k_prepare0d, dim3(blocks), dim3(256), 0, stream, g, b);
@@ -1149,7 +1218,16 @@ int launch_newton(const GridDev& g, const BatchDev& b, hipStream_t stream, const
     hipLaunchKernelGGL(k_ee_profile_add, dim3(blocks), dim3(256), 0, stream, g, b, *ee);
     BZ_LAUNCH_CHECK();
   }
-  hipLaunchKernelGGL((k_newton0d<W, R>), dim3(b.B), dim3(64), lds, stream, g, b);
+  return BZ_OK;
+}
+
+template <int W, int T>
+int launch_newton(GridDev g, const BatchDev& b, hipStream_t stream, const EEDev* ee = nullptr) {
+  const size_t lds = newton_lds_bytes<W>(g, 2);
+  if (lds > 64 * 1024 || !fits_offsets(g)) return BZ_EINVAL;
+  const int rc = launch_prepare(g, b, stream, ee);
+  if (rc != BZ_OK) return rc;
+  hipLaunchKernelGGL((k_newton0d<W, T>), dim3(b.B), dim3(64), lds, stream, g, b);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }
@@ -1166,24 +1244,22 @@ int launch_newton(const GridDev& g, const BatchDev& b, hipStream_t stream, const
 // sides, and the iterates are the reference's.  The iteration count and the stopping
 // test follow the reference loop (the convergence test of an iterate is made before
 // its update, and the update is still applied), per instance.
-template <int W, int R>
-__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 : 2))) void k_transient0d(GridDev g, BatchDev b,
+template <int W, int T>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W, T>()))) void k_transient0d(GridDev g, BatchDev b,
                                                                                            double cdt,
                                                                                            const double* ustart,
                                                                                            double* avg) {
-  extern __shared__ double lds[];
+  extern __shared__ __align__(32) double lds[];
   const int n = g.n, lane = threadIdx.x, inst = blockIdx.x;
   constexpr int WP = (W + 1) & ~1;
-  constexpr int PIVN = piv_len<W>();
-  double* X = lds;
+  double* PIV = lds;
+  double* X = PIV + piv_len<W>();
   double* Z1 = X + n;
   double* Z2 = Z1 + n;
-  double* AV = Z2 + n + zpad(n, g.npr);
-  double* STG = AV + n;
-  double* PIV = STG + 2 * W * WP;
-  double* U0 = PIV + PIVN;
+  double* LC = g.keep_mass ? Z2 + n : Z1;
+  double* AV = Z2 + n + (g.keep_mass ? 4 * g.npr : zpad(n, g.npr));
+  double* U0 = AV + n;
   int2* SC = reinterpret_cast<int2*>(U0 + n);
-  double* LCH = Z1;
 
   double* kprof = b.kprof + (size_t)inst * g.P;
   const double* __restrict__ mprof = g.opprof + (size_t)(g.nop - 1) * g.P;
@@ -1192,6 +1268,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
   double* urows = b.urows + (size_t)inst * n * WP;
 
   fill_rowtab(g, SC, lane);
+  if (g.keep_mass) stage_mass(g, LC, lane);
   for (int i = lane; i < n; i += 64) {
     const size_t o = (size_t)orig_index(i, g.ns, g.npr) * b.B + inst;
     X[i] = b.x[o];                              // initial iterate
@@ -1214,16 +1291,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
 
   // G(X) into AV; returns |G|
   auto residual = [&]() -> double {
-    for (int e = lane; e < 4 * g.npr; e += 64) {
-      const int q = e >> 2, dd = e & 3;
-      const double v = g.mchol[(size_t)(q * g.ns) * 4 + dd];
-      LCH[e] = (dd == 0) ? 1.0 / v : ((q - dd >= 0) ? v : 0.0);
-    }
-    for (int i = lane; i < n; i += 64) AV[i] = 0.0;
+    if (!g.keep_mass) stage_mass(g, LC, lane);
+    row_sums<false>(n, g.ns, g.npr, g.bw, g.P, SC, kprof, X, lane, [&](int i, double s, double) { AV[i] = s; });
     __syncthreads();
-    flat_matvec(g.P, kprof, g.ent_rc, X, AV, lane);
-    __syncthreads();
-    mass_solve(g.ns, g.npr, LCH, AV, lane);
+    mass_solve(g.ns, g.npr, LC, AV, lane);
     __syncthreads();
     const double mu = dot(WV, X, n, lane);
     double su = 0.0;
@@ -1256,23 +1327,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
   while (!conv && it < b.max_iter) {
     if (it > 0) rr = residual();
     conv = (rr / r0 < b.rtol) || (rr < b.atol);
-    mass_matvec(n, g.ns, mprof, g.first_col, g.prof_off, AV, Z2, lane);
+    mass_matvec(n, g.ns, mprof, SC, AV, Z2, lane);
     if (it == 0 || lp == nullptr) {
       for (int i = lane; i < n; i += 64) Z1[i] = g.muhat[i];
       __syncthreads();
-      if (lp) factor_forward<W, R, true>(g, kprof, SC, Z1, Z2, nullptr, PIV, STG, urows, WP, lane, lp);
-      else factor_forward<W, R>(g, kprof, SC, Z1, Z2, nullptr, PIV, STG, urows, WP, lane);
+      if (lp) factor_tiles<W, T, true, 2>(g, kprof, SC, Z1, Z2, nullptr, PIV, urows, lane, lp);
+      else factor_tiles<W, T, false, 2>(g, kprof, SC, Z1, Z2, nullptr, PIV, urows, lane);
       __syncthreads();
-      back_substitute<W>(n, urows, WP, Z1, Z2, nullptr, STG, lane);
+      back_tiles<W, 2>(g, urows, Z1, Z2, nullptr, lane);
       __syncthreads();
       su = dot(UH, Z1, n, lane);
       if (lp)
         for (int i = lane; i < n; i += 64) ZU[i] = Z1[i];
     } else {
       __syncthreads();
-      forward_solve_stored<W, R>(g, lp, SC, Z2, PIV, STG, lane);
+      forward_tiles<W, T>(g, lp, SC, Z2, PIV, lane);
       __syncthreads();
-      back_substitute<W, 1>(n, urows, WP, Z2, nullptr, nullptr, STG, lane);
+      back_tiles<W, 1>(g, urows, Z2, nullptr, nullptr, lane);
       for (int i = lane; i < n; i += 64) Z1[i] = ZU[i];
       __syncthreads();
     }
@@ -1296,18 +1367,26 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
   }
 }
 
-template <int W, int R>
-int launch_transient(const GridDev& g, const BatchDev& b, double cdt, const double* ustart, double* avg,
+template <int W, int T>
+int launch_transient(GridDev g, const BatchDev& b, double cdt, const double* ustart, double* avg,
                      hipStream_t stream) {
-  const size_t lds = newton_lds_bytes<W>(g.n, g.npr) + (size_t)g.n * sizeof(double);   // + U0
-  if (lds > 64 * 1024) return BZ_EINVAL;
-  const long work = (long)b.B * g.P;
-  const int blocks = (int)std::min<long>((work + 255) / 256, 8192);
-  hipLaunchKernelGGL(k_prepare0d, dim3(blocks), dim3(256), 0, stream, g, b);
-  BZ_LAUNCH_CHECK();
-  hipLaunchKernelGGL((k_transient0d<W, R>), dim3(b.B), dim3(64), lds, stream, g, b, cdt, ustart, avg);
+  const size_t lds = newton_lds_bytes<W>(g, 3);
+  if (lds > 64 * 1024 || !fits_offsets(g)) return BZ_EINVAL;
+  const int rc = launch_prepare(g, b, stream);
+  if (rc != BZ_OK) return rc;
+  hipLaunchKernelGGL((k_transient0d<W, T>), dim3(b.B), dim3(64), lds, stream, g, b, cdt, ustart, avg);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }
 
 }  // namespace
+
+// Runs `launch<W, T>` with the smallest instantiated tile count T that holds g.nslots slots.
+#define BZ0D_FOR_TILES(W_, launch, g, ...)                      \
+  const int tiles = ((g).nslots + 15) / 16;                     \
+  if (tiles <= 3) return launch<W_, 3>(g, __VA_ARGS__);         \
+  if (tiles <= 5) return launch<W_, 5>(g, __VA_ARGS__);         \
+  if (tiles <= 8) return launch<W_, 8>(g, __VA_ARGS__);         \
+  if (tiles <= 12) return launch<W_, 12>(g, __VA_ARGS__);       \
+  if (W_ >= 17 && tiles <= 16) return launch<W_, (W_ >= 17 ? 16 : 12)>(g, __VA_ARGS__); \
+  return BZ_EINVAL;

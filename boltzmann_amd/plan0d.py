@@ -115,6 +115,41 @@ def plan_structure(mask_orig, npr, ns, window_fn):
     }
 
 
+def tile_schedule(first_col, bw, W):
+    """Slot schedule of the blocked factorisation: (slot_first, sched_next, nslots).
+
+    The kernel walks the columns in groups of four.  Row i reads the groups first_col >> 2 to
+    (i >> 2) + NG, NG the groups its pivot block reaches to the right, so its slot can go to a row
+    whose first group is not before (i >> 2) + NG + 1.  Rows in order of their first group take
+    the lowest free slot (72 slots at n = 387; the lead of two windows that one pivot at a time
+    needs took 78).  nslots is the slot count, one more where that is a multiple of 64: such
+    counts are those of the one-pivot-a-step tables."""
+    first = np.asarray(first_col, dtype=np.int64)
+    n = len(first)
+    NG = (W + 2) // 4
+    grp = first >> 2
+    alive, free_ids, slot_rows = [], [], []
+    for i in np.argsort(grp, kind="stable"):
+        while alive and alive[0][0] < grp[i]:
+            heapq.heappush(free_ids, heapq.heappop(alive)[1])
+        if free_ids:
+            s = heapq.heappop(free_ids)
+        else:
+            s = len(slot_rows)
+            slot_rows.append([])
+        slot_rows[s].append(int(i))
+        heapq.heappush(alive, ((int(i) >> 2) + NG, s))
+    nslots = len(slot_rows) + (len(slot_rows) % 64 == 0)
+    slot_first = np.full(64 * ((nslots + 63) // 64), -1, dtype=np.int64)
+    sched_next = np.full(n, -1, dtype=np.int64)
+    for s, rs in enumerate(slot_rows):
+        slot_first[s] = rs[0]
+        for a, b in zip(rs[:-1], rs[1:]):
+            assert grp[b] >= (a >> 2) + NG + 1, "slot overlap"
+            sched_next[a] = b
+    return slot_first, sched_next, nslots
+
+
 class SolverTables:
     """Device tables of one grid for bz_steady_solve_0d."""
 
@@ -143,8 +178,14 @@ class SolverTables:
         i32 = lambda a: torch.from_numpy(np.ascontiguousarray(a, dtype=np.int32)).to(dev)
         self.first_col = i32(st["first_col"])
         self.prof_off = i32(st["prof_off"])
-        self.slot_first = i32(st["slot_first"])
-        self.sched_next = i32(st["sched_next"])
+        # the e-e path eliminates one pivot at a time and needs the lead of two windows; its tables
+        # have nslots a multiple of 64
+        if extra_mask is None:
+            slot_first, sched_next, nslots = tile_schedule(st["first_col"], st["bw"], st["W"])
+        else:
+            slot_first, sched_next, nslots = st["slot_first"], st["sched_next"], st["nslots"]
+        self.slot_first = i32(slot_first)
+        self.sched_next = i32(sched_next)
         self.chunk_levels = i32(st["chunk_levels"])
         self.ent_rc = torch.from_numpy(st["ent_rc"].view(np.int32).copy()).to(dev)
         P = st["P"]
@@ -191,7 +232,7 @@ class SolverTables:
         self.W = st["W"]
         self.WP = (self.W + 1) & ~1
         self.struct = _lib.Grid0D(
-            n=n, ns=ns, npr=npr, bw=st["bw"], S=self.S, nop=self.nop, P=P, nslots=st["nslots"],
+            n=n, ns=ns, npr=npr, bw=st["bw"], S=self.S, nop=self.nop, P=P, nslots=nslots,
             first_col=self.first_col.data_ptr(), prof_off=self.prof_off.data_ptr(),
             opprof=self.opprof.data_ptr(), slot_first=self.slot_first.data_ptr(),
             sched_next=self.sched_next.data_ptr(), muhat=self.muhat.data_ptr(), uhat=self.uhat.data_ptr(),

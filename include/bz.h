@@ -98,14 +98,18 @@ typedef struct {
   const int* first_col;   /* [n]   first column of each row profile            */
   const int* prof_off;    /* [n+1] offsets of the row profiles                  */
   const double* opprof;   /* [nop][P]  C_0..C_{S-1}, C_Tg, A_E, M in profiles   */
-  const int* slot_first;  /* [nslots] first row of every lane slot (-1: none)  */
+  const int* slot_first;  /* [nslots rounded up to 64] first row of every row slot (-1: none).
+                             nslots a multiple of 64: slots held from step first_col - 2W to the
+                             pivot step, for the one-pivot-a-step solver (tables with the e-e
+                             pattern); any other count: the blocked solver's schedule, a slot held
+                             while the row's column groups of four are read                  */
   const int* sched_next;  /* [n]   next row of the same slot (-1: none)         */
   const double* muhat;    /* [n]   M uhat                                       */
   const double* uhat;     /* [n]   u / |u|                                      */
   const double* u;        /* [n]   mass vector u                                */
   const double* wsp;      /* [nop-1][n] W_m = Op_m^T M^-1 u (zero row: operator not in the growth term) */
   const double* mchol;    /* [n][4] banded Cholesky rows of M                   */
-  const int* chunk_levels;    /* [ceil(n/W)] register levels alive per W-step chunk */
+  const int* chunk_levels;    /* [ceil(n/W)] register levels alive per W-step chunk (not read) */
   const unsigned* ent_rc;     /* [P] (row << 16) | column of every profile entry    */
   int max_row;                /* longest row profile (entries)                      */
 } bz_grid0d_t;
