@@ -369,6 +369,27 @@ size_t lane_newton_lds_bytes(int n, int npr) {
   return (size_t)(4 * n + zpad(n, npr) + 2 * W * WP + lane_piv_len<W>()) * sizeof(double) + (size_t)n * sizeof(int2);
 }
 
+// |(I - uhat uhat^T) v| for v = ca A + cx X + cp P (two passes: explicit projection, no
+// |v|^2 - (u.v)^2 cancellation); P may be null (cp ignored).
+__device__ double proj_norm3(const double* A, double ca, const double* X, double cx, const double* P, double cp,
+                             const double* __restrict__ uh, int n, int lane) {
+  double su = 0.0;
+  for (int i = lane; i < n; i += 64) {
+    double v = fma(ca, A[i], cx * X[i]);
+    if (P) v = fma(cp, P[i], v);
+    su = fma(uh[i], v, su);
+  }
+  su = wave_sum(su);
+  double s2 = 0.0;
+  for (int i = lane; i < n; i += 64) {
+    double v = fma(ca, A[i], cx * X[i]);
+    if (P) v = fma(cp, P[i], v);
+    const double rp = v - su * uh[i];
+    s2 = fma(rp, rp, s2);
+  }
+  return sqrt(wave_sum(s2));
+}
+
 template <int W, int R>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 : 2))) void k_newton0d_lane(GridDev g, BatchDev b) {
   extern __shared__ double lds[];

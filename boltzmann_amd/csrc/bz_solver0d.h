@@ -156,27 +156,6 @@ __device__ __forceinline__ double dot(const double* __restrict__ a, const double
   return wave_sum(s);
 }
 
-// Dot product in compensated arithmetic (per-lane TwoProduct/TwoSum accumulation, then a
-// compensated butterfly across the wavefront): about as accurate as a sum in twice FP64.
-__device__ double dot_dd(const double* __restrict__ a, const double* __restrict__ b, int n, int lane) {
-  double s = 0.0, c = 0.0;
-  for (int i = lane; i < n; i += 64) two_sum_acc(a[i], b[i], s, c);
-#pragma unroll
-  for (int off = 32; off >= 16; off >>= 1) {
-#pragma clang fp contract(off)
-    const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
-    const double t = s + s2, z = t - s;
-    const double e = (s - (t - z)) + (s2 - z);
-    s = t;
-    c = c + c2 + e;
-  }
-  dd_reduce<kDppRor8>(s, c);
-  dd_reduce<kDppRor4>(s, c);
-  dd_reduce<kDppXor2>(s, c);
-  dd_reduce<kDppXor1>(s, c);
-  return s + c;
-}
-
 // y = M x from the M profile (M is l-block diagonal, radial 7-band: columns i + d*ns, |d| <= 3).
 __device__ void mass_matvec(int n, int ns, const double* __restrict__ mprof, const int2* __restrict__ rt,
                             const double* __restrict__ x, double* __restrict__ y, int lane) {
@@ -259,6 +238,41 @@ __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
   __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+}
+
+// Entries lane, lane + 64, ... of a global vector of n, eight loads in flight: f(i, value), i < n.
+template <class F>
+__device__ __forceinline__ void for_entries(const ProfileBuf& a, int n, int lane, F f) {
+  for (int i0 = lane; i0 - lane < n; i0 += 512) {
+    double v[8];
+#pragma unroll
+    for (int u = 0; u < 8; ++u) v[u] = buf_load(a, 8 * (i0 + 64 * u));
+#pragma unroll
+    for (int u = 0; u < 8; ++u)
+      if (i0 + 64 * u < n) f(i0 + 64 * u, v[u]);
+  }
+}
+
+// Dot product with a vector in LDS in compensated arithmetic (per-lane TwoProduct/TwoSum
+// accumulation, then a compensated butterfly across the wavefront): about as accurate as a sum in
+// twice FP64.
+__device__ double dot_dd(const double* __restrict__ a, const double* __restrict__ b, int n, int lane) {
+  double s = 0.0, c = 0.0;
+  for_entries(profile_buf(a, n), n, lane, [&](int i, double v) { two_sum_acc(v, b[i], s, c); });
+#pragma unroll
+  for (int off = 32; off >= 16; off >>= 1) {
+#pragma clang fp contract(off)
+    const double s2 = __shfl_xor(s, off, 64), c2 = __shfl_xor(c, off, 64);
+    const double t = s + s2, z = t - s;
+    const double e = (s - (t - z)) + (s2 - z);
+    s = t;
+    c = c + c2 + e;
+  }
+  dd_reduce<kDppRor8>(s, c);
+  dd_reduce<kDppRor4>(s, c);
+  dd_reduce<kDppXor2>(s, c);
+  dd_reduce<kDppXor1>(s, c);
+  return s + c;
 }
 
 // Row sums of the instance profile, sum_c k[row][c] x[c], eight lanes to a row and eight rows at
@@ -374,6 +388,7 @@ struct SlotRow {
     lim = (row >> 2) + NG;
     next = tx >> 16;
     if (row < 0) {
+      fc = 0x7fffffff;
       cnt = 0;
       lim = 0x7fffffff;
       next = -1;
@@ -434,7 +449,7 @@ __device__ __forceinline__ double pick4(v4d v, int k) {
 // offsets as U11).  SL: the multipliers of L at the profile positions of lout.
 // s_piv: 16 (NG + 2) doubles of LDS, 32-byte aligned.
 template <int W, int T, bool SL, int NRHS>
-__device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof, const int2* __restrict__ rt_,
+__device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof, const int2* __restrict__ rt_,
                              double* __restrict__ y1_, double* __restrict__ y2_, double* __restrict__ y3_,
                              double* __restrict__ piv_, double* __restrict__ urows, int lane,
                              double* __restrict__ lout_ = nullptr) {
@@ -470,8 +485,8 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
   // Per tile: P the panel, R4 ring registers 0..3 (and the right-hand sides), RX ring register 4
   // and Y when they do not fit the 16x16x4 tile, F the groups read ahead.
   SlotRow<NG, false> st[T];
-  int crow[T];                                       // row being eliminated in the slot
-  int cfc[SL ? T : 1], coff[SL ? T : 1];             // its first column and profile offset (SL)
+  int crow[T], cfc[T];                               // row being eliminated in the slot, its first column
+  int coff[SL ? T : 1];                              // and profile offset (SL)
   double P[T], F[T][NG], RX[NX ? T : 1], Y[Y16 ? 1 : T];
   v4d R4[T];
 #pragma unroll
@@ -480,10 +495,8 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
     const int row = slot < g.nslots ? g.slot_first[slot] : -1;
     st[t].enter(rt, row, n, bw);
     crow[t] = row;
-    if constexpr (SL) {
-      cfc[t] = st[t].fc;
-      coff[t] = st[t].off8 >> 3;
-    }
+    cfc[t] = st[t].fc;
+    if constexpr (SL) coff[t] = st[t].off8 >> 3;
     const double y0 = (q < NRHS && row >= 0) ? (double)yq[row] : 0.0;
     P[t] = st[t].load(kb, q);
     R4[t] = v4d{0.0, 0.0, 0.0, 0.0};
@@ -501,6 +514,10 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
       F[t][s] = st[t].load(kb, 4 * (NG + 1 + s) + q);
     }
   }
+  // Wait for the loads so far here, once: with them in flight at the loop entry, in another order
+  // than on its edge, the compiler's wait analysis would put full waits into every round.
+  // (s_waitcnt fields: vmcnt 0, expcnt 7, lgkmcnt 15.)
+  __builtin_amdgcn_s_waitcnt(0x0F70);
   // Whole rounds of NG blocks (the ring positions are constants); a block past the last row
   // factorises the identity on empty tiles and its stores fall past the end.  An exit inside a
   // round would put register copies, and so a wait for every load ahead, on the loop edge.
@@ -518,26 +535,26 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
       }
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        if ((crow[t] >> 2) == gb) {
+        const bool mine = (crow[t] >> 2) == gb;
+        double y0 = 0.0;
+        if (mine) {
           lds_double* pk = piv + 4 * q + (crow[t] & 3);
           pk[0] = P[t];
 #pragma unroll
           for (int r = 0; r < NG; ++r) pk[16 * (r > u ? r - u : r - u + NG)] = r < 4 ? R4[t][r < 4 ? r : 0] : RX[NX ? t : 0];
           pk[16 * (NG + 1)] = Y16 ? R4[t][YR] : Y[Y16 ? 0 : t];
-          // the slot's next row (already the one being read): no column of it has arrived yet
+          // the slot's next row (already the one being read)
           const int nr = st[t].row;
+          if (q < NRHS && nr >= 0) y0 = yq[nr];
           crow[t] = nr;
-          P[t] = 0.0;
-          R4[t] = v4d{0.0, 0.0, 0.0, 0.0};
-          if constexpr (NX > 0) RX[t] = 0.0;
-          const double y0 = (q < NRHS && nr >= 0) ? (double)yq[nr] : 0.0;
-          if constexpr (Y16) R4[t][YR] = y0;
-          else Y[t] = y0;
-          if constexpr (SL) {
-            cfc[t] = st[t].fc;
-            coff[t] = st[t].off8 >> 3;
-          }
+          cfc[t] = st[t].fc;
+          if constexpr (SL) coff[t] = st[t].off8 >> 3;
         }
+        // No column of the next row has arrived yet; what the ring still holds is the old row's
+        // and is masked as it becomes the panel.
+        P[t] = mine ? 0.0 : P[t];
+        if constexpr (Y16) R4[t][YR] = mine ? y0 : R4[t][YR];
+        else Y[t] = mine ? y0 : Y[t];
       }
       // --- where the next group of every slot is read from
       int nx_o[T];
@@ -604,11 +621,12 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
 #pragma unroll
       for (int t = 0; t < T; ++t) {
         const int r = (u + 1) % RN;
+        const bool in = 4 * gb + 4 + q >= cfc[t];
         if (r < 4) {
-          P[t] = R4[t][r < 4 ? r : 0];
+          P[t] = in ? R4[t][r < 4 ? r : 0] : 0.0;
           R4[t][r < 4 ? r : 0] = F[t][u];
         } else {
-          P[t] = RX[NX ? t : 0];
+          P[t] = in ? RX[NX ? t : 0] : 0.0;
           RX[NX ? t : 0] = F[t][u];
         }
         F[t][u] = buf_load(kb, nx_o[t]);
@@ -622,7 +640,7 @@ __device__ void factor_tiles(const GridDev& g, const double* __restrict__ kprof,
 // blocks with the stored multipliers streamed as panels: per tile and block one load and one
 // 4x4x4 product.  The order of the operations on a row is the factorisation's.
 template <int W, int T>
-__device__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof, const int2* __restrict__ rt_,
+__device__ __forceinline__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof, const int2* __restrict__ rt_,
                               double* __restrict__ y_, double* __restrict__ piv_, int lane) {
   lane = fresh_lane(lane);
   constexpr int NG = trail_groups<W>(), PF = 4;
@@ -659,6 +677,7 @@ __device__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof
     }
     D[s] = diag(s);
   }
+  __builtin_amdgcn_s_waitcnt(0x0F70);                 // as in factor_tiles
   const int nb = (n + 3) >> 2;
   for (int g0 = 0; g0 < nb; g0 += PF) {
 #pragma unroll
@@ -704,7 +723,7 @@ __device__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof
 // of four rows: z_g = U11^-1 (y_g - sum_s U_(g,g+s) z_(g+s)), every product one 4x4x4 whose
 // result is the next one's operand as it stands; only two of them wait on the block before.
 template <int W, int NRHS>
-__device__ void back_tiles(const GridDev& g, const double* __restrict__ urows, double* __restrict__ Y1,
+__device__ __forceinline__ void back_tiles(const GridDev& g, const double* __restrict__ urows, double* __restrict__ Y1,
                            double* __restrict__ Y2, double* __restrict__ Y3, int lane) {
   lane = fresh_lane(lane);
   constexpr int NG = trail_groups<W>(), WP = (W + 1) & ~1, PD = NG <= 3 ? 2 * NG : NG;
@@ -727,12 +746,10 @@ __device__ void back_tiles(const GridDev& g, const double* __restrict__ urows, d
   for (int u = 0; u < PD; ++u)
 #pragma unroll
     for (int s = 0; s <= NG; ++s) A[u][s] = buf_load(ub, uo[s] + (nu - PD + u) * (4 * WP * 8));
-  auto rhs = [&](int gb) -> double {
-    const int j = 4 * gb + q;
-    const double v = yj[min(max(j, 0), n - 1)];
-    return (live && j < n) ? v : 0.0;
-  };
+  // Rows past the last have zero rows of U, U11^-1 among them, so any finite value does there.
+  auto rhs = [&](int gb) -> double { return yj[min(max(4 * gb + q, 0), n - 1)]; };
   double yn = rhs(nu - 1);
+  __builtin_amdgcn_s_waitcnt(0x0F70);                 // as in factor_tiles
   for (int g0 = nu - PD; g0 >= 0; g0 -= PD) {
 #pragma unroll
     for (int u = PD - 1; u >= 0; --u) {
@@ -753,7 +770,8 @@ __device__ void back_tiles(const GridDev& g, const double* __restrict__ urows, d
 
 // The radial mass Cholesky factor staged for mass_solve, rows of four: lc[4 q + d] for d <= q % 4
 // is entry (q, q - d) of the inverse of the 4 x 4 diagonal block that row q lies in, for d > q % 4
-// the factor's own entry L[q, q - d] (zero before the first column).  One lane per block.
+// the factor's own entry L[q, q - d] (zero before the first column); rows past the last are zero.
+// One lane per block, 16 doubles a block.
 __device__ void stage_mass(const GridDev& g, double* __restrict__ lc, int lane) {
   lane = fresh_lane(lane);
   const int nb = (g.npr + 3) >> 2;
@@ -781,9 +799,8 @@ __device__ void stage_mass(const GridDev& g, double* __restrict__ lc, int lane) 
                             {i3, x32, x31, x30}};
 #pragma unroll
     for (int i = 0; i < 4; ++i)
-      if (4 * b + i < g.npr)
 #pragma unroll
-        for (int d = 0; d < 4; ++d) lc[16 * b + 4 * i + d] = o[i][d];
+      for (int d = 0; d < 4; ++d) lc[16 * b + 4 * i + d] = 4 * b + i < g.npr ? o[i][d] : 0.0;
   }
 }
 
@@ -797,55 +814,51 @@ __device__ void mass_solve(int ns, int npr, const double* __restrict__ lc_, doub
   lane = fresh_lane(lane);
   const lds_double* lc = (const lds_double*)lc_;
   lds_double* b = (lds_double*)b_;
+  constexpr int CH = 8;                               // blocks whose operands are read together
   const int i = lane & 3, k = lane >> 4, col = lane & 15;
   const int nb = (npr + 3) >> 2;
-  // operands A[i][k]: -S_g (row 4 g + i, offset 4 + i - k, when i < k) and D_g (offset i - k)
-  auto opS = [&](int g) -> double {
-    const int r = 4 * g + i;
-    const double v = lc[4 * min(r, npr - 1) + ((4 + i - k) & 3)];
-    return (i < k && r < npr && g > 0) ? -v : 0.0;
-  };
-  auto opD = [&](int g) -> double {
-    const int r = 4 * g + i;
-    const double v = lc[4 * min(r, npr - 1) + ((i - k) & 3)];
-    return (i >= k && r < npr) ? v : 0.0;
-  };
-  // transposed: -S_(g+1)^T (row 4 g + 4 + k, offset 4 + k - i, when k < i) and D_g^T
-  auto opSt = [&](int g) -> double {
-    const int r = 4 * g + 4 + k;
-    const double v = lc[4 * min(r, npr - 1) + ((4 + k - i) & 3)];
-    return (k < i && r < npr) ? -v : 0.0;
-  };
-  auto opDt = [&](int g) -> double {
-    const int r = 4 * g + k;
-    const double v = lc[4 * min(r, npr - 1) + ((k - i) & 3)];
-    return (k >= i && r < npr) ? v : 0.0;
-  };
-  auto rhs = [&](int g) -> double {
-    const int r = 4 * g + k;
-    const double v = b[max(0, min(r, npr - 1)) * ns + min(col, ns - 1)];
-    return (r < npr && col < ns) ? v : 0.0;
-  };
+  // Operands A[i][k]: -S_g at (row i, offset 4 + i - k) where i < k, D_g at (i, i - k) where
+  // i >= k, and the transposes; rows past the last are zero, the first block's S is zero.
+  const int oS = 4 * i + ((4 + i - k) & 3), oD = 4 * i + ((i - k) & 3);
+  const int oSt = 4 * k + ((4 + k - i) & 3), oDt = 4 * k + ((k - i) & 3);
+  const double mS = i < k ? -1.0 : 0.0, mD = i >= k ? 1.0 : 0.0;
+  const double mSt = k < i ? -1.0 : 0.0, mDt = k >= i ? 1.0 : 0.0;
+  const int cc = min(col, ns - 1);
+  auto at = [&](int g) -> int { return max(0, min(4 * g + k, npr - 1)) * ns + cc; };
   auto put = [&](int g, double v) {
-    const int r = 4 * g + k;
-    if (r < npr && col < ns) b[r * ns + col] = v;
+    if (g >= 0 && 4 * g + k < npr && col < ns) b[(4 * g + k) * ns + col] = v;
   };
-  double y = 0.0, S = opS(0), D = opD(0), v = rhs(0);
-  for (int g = 0; g < nb; ++g) {
-    const int gn = min(g + 1, nb - 1);
-    const double Sn = opS(gn), Dn = opD(gn), vn = rhs(gn);
-    y = mfma4(D, mfma4(S, y, v), 0.0);
-    put(g, y);
-    S = Sn; D = Dn; v = vn;
+  double y = 0.0;
+  for (int g0 = 0; g0 < nb; g0 += CH) {
+    double S[CH], D[CH], v[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int g = min(g0 + u, nb - 1);
+      S[u] = lc[16 * g + oS];
+      D[u] = lc[16 * g + oD];
+      v[u] = b[at(g)];
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      y = mfma4(D[u] * mD, mfma4(S[u] * mS, y, v[u]), 0.0);
+      if (g0 + u < nb) put(g0 + u, y);
+    }
   }
   double z = 0.0;
-  S = opSt(nb - 1); D = opDt(nb - 1); v = rhs(nb - 1);
-  for (int g = nb - 1; g >= 0; --g) {
-    const int gn = max(g - 1, 0);
-    const double Sn = opSt(gn), Dn = opDt(gn), vn = rhs(gn);
-    z = mfma4(D, mfma4(S, z, v), 0.0);
-    put(g, z);
-    S = Sn; D = Dn; v = vn;
+  for (int g0 = nb - 1; g0 >= 0; g0 -= CH) {
+    double S[CH], D[CH], v[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      const int g = max(g0 - u, 0);
+      S[u] = lc[16 * min(g + 1, nb - 1) + oSt];       // the last block multiplies z = 0
+      D[u] = lc[16 * g + oDt];
+      v[u] = b[at(g)];
+    }
+#pragma unroll
+    for (int u = 0; u < CH; ++u) {
+      z = mfma4(D[u] * mDt, mfma4(S[u] * mSt, z, v[u]), 0.0);
+      put(g0 - u, z);
+    }
   }
 }
 
@@ -889,10 +902,13 @@ __global__ void k_prepare0d(GridDev g, BatchDev b) {
 }
 
 // LDS: the published pivot block PIV first (32-byte aligned), four n-vectors R0..R3, the staged
-// mass factor LC (4*npr doubles), then the row table (int2 per row).  Where LC would cost a
+// mass factor LC (mass_len doubles), then the row table (int2 per row).  Where LC would cost a
 // wavefront per CU or pass 64 KB it shares R1..R2 (with a pad after R2) and is staged again for
 // every residual.
-__host__ __device__ __forceinline__ int zpad(int n, int npr) { return (4 * npr > 2 * n) ? (4 * npr - 2 * n) : 0; }
+__host__ __device__ __forceinline__ int mass_len(int npr) { return 16 * ((npr + 3) / 4); }
+__host__ __device__ __forceinline__ int zpad(int n, int npr) {
+  return mass_len(npr) > 2 * n ? mass_len(npr) - 2 * n : 0;
+}
 
 template <int W>
 __host__ __device__ constexpr int piv_len() { return 16 * (trail_groups<W>() + 2); }
@@ -906,7 +922,7 @@ constexpr int tile_waves() { return T * (trail_groups<W>() + 2) <= 30 ? 2 : 1; }
 template <int W>
 size_t newton_lds_bytes(GridDev& g, int vecs) {
   const size_t rest = (size_t)((vecs + 2) * g.n + piv_len<W>()) * sizeof(double) + (size_t)g.n * sizeof(int2);
-  const size_t keep = rest + (size_t)4 * g.npr * sizeof(double), share = rest + (size_t)zpad(g.n, g.npr) * sizeof(double);
+  const size_t keep = rest + (size_t)mass_len(g.npr) * sizeof(double), share = rest + (size_t)zpad(g.n, g.npr) * sizeof(double);
   constexpr size_t cu = 160 * 1024;
   g.keep_mass = keep <= 64 * 1024 && (cu / keep >= 8 || cu / keep == cu / share);
   return g.keep_mass ? keep : share;
@@ -915,24 +931,17 @@ size_t newton_lds_bytes(GridDev& g, int vecs) {
 // Profiles and U rows are read through 32-bit byte offsets below kOutside.
 inline bool fits_offsets(const GridDev& g) { return g.P > 0 && g.P < kOutside / 8 && g.n < 32768; }
 
-// |(I - uhat uhat^T) v| for v = ca A + cx X + cp P (two passes: explicit projection, no
-// |v|^2 - (u.v)^2 cancellation); P may be null (cp ignored).
-__device__ double proj_norm3(const double* A, double ca, const double* X, double cx, const double* P, double cp,
-                             const double* __restrict__ uh, int n, int lane) {
+// |(I - uhat uhat^T) v|, v in LDS (two passes: explicit projection, no |v|^2 - (u.v)^2
+// cancellation).
+__device__ double proj_norm(const double* v, const ProfileBuf& uh, int n, int lane) {
   double su = 0.0;
-  for (int i = lane; i < n; i += 64) {
-    double v = fma(ca, A[i], cx * X[i]);
-    if (P) v = fma(cp, P[i], v);
-    su = fma(uh[i], v, su);
-  }
+  for_entries(uh, n, lane, [&](int i, double u) { su = fma(u, v[i], su); });
   su = wave_sum(su);
   double s2 = 0.0;
-  for (int i = lane; i < n; i += 64) {
-    double v = fma(ca, A[i], cx * X[i]);
-    if (P) v = fma(cp, P[i], v);
-    const double rp = v - su * uh[i];
+  for_entries(uh, n, lane, [&](int i, double u) {
+    const double rp = v[i] - su * u;
     s2 = fma(rp, rp, s2);
-  }
+  });
   return sqrt(wave_sum(s2));
 }
 
@@ -973,7 +982,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
   double* R1 = R0 + n;                                     // M uhat -> z1
   double* R2 = R1 + n;                                     // M x -> z2
   double* LC = g.keep_mass ? R2 + n : R1;                  // staged mass factor (R1..R2 free in a residual)
-  double* R3 = R2 + n + (g.keep_mass ? 4 * g.npr : zpad(n, g.npr));   // y3 -> T = M^-1 y3
+  double* R3 = R2 + n + (g.keep_mass ? mass_len(g.npr) : zpad(n, g.npr));   // y3 -> T = M^-1 y3
   int2* SC = reinterpret_cast<int2*>(R3 + n);
 
   double* kprof = b.kprof + (size_t)inst * g.P;           // K, then K - mu M on the band of M
@@ -991,7 +1000,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
   fill_rowtab(g, SC, lane);
   if (g.keep_mass) stage_mass(g, LC, lane);
   for (int i = lane; i < n; i += 64) R0[i] = b.x[(size_t)orig_index(i, g.ns, g.npr) * b.B + inst];
-  const ProfileBuf mb = profile_buf(mprof, g.P), kpb = profile_buf(kprof, g.P), kbb = profile_buf(KB0, 7 * n);
+  const ProfileBuf mb = profile_buf(mprof, g.P), kpb = profile_buf(kprof, g.P), kbb = profile_buf(KB0, 7 * n),
+                   muhb = profile_buf(g.muhat, n), uhb = profile_buf(UH, n), wvb = profile_buf(WV, n);
   __syncthreads();
 
   // residual at the point in R0 for the coefficient cq: x normalised in place, K' in the
@@ -1002,27 +1012,27 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
     for (int i = lane; i < n; i += 64) R0[i] = R0[i] / ux;
     __syncthreads();
     const double mu = dot_dd(WV, R0, n, lane);
-    // the band of M, lane d of eight on offset d - 3 of a row, eight rows to a pass and four
-    // passes' loads in flight
-    for (int i0 = lane >> 3; i0 - (lane >> 3) < n; i0 += 32) {
+    // the band of M, lane d of eight on offset d - 3 of a row, eight rows to a pass and the loads
+    // of NB passes in flight
+    constexpr int NB = 10;
+    for (int i0 = lane >> 3; i0 - (lane >> 3) < n; i0 += 8 * NB) {
       const int d = lane & 7;
-      double mv[4], kv[4];
-      int eo[4], bo[4];
+      double mv[NB], kv[NB];
+      int eo[NB];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < NB; ++u) {
         const int i = i0 + 8 * u, c = i + (d - 3) * g.ns;
         const bool ok = i < n && d < 7 && c >= 0 && c < n;
         eo[u] = ok ? 8 * (SC[min(i, n - 1)].y + c) : kOutside;
-        bo[u] = ok ? 8 * (7 * i + d) : kOutside;
         mv[u] = buf_load(mb, eo[u]);
-        kv[u] = first ? buf_load(kpb, eo[u]) : buf_load(kbb, bo[u]);
+        kv[u] = first ? buf_load(kpb, eo[u]) : buf_load(kbb, ok ? 8 * (7 * i + d) : kOutside);
       }
 #pragma unroll
-      for (int u = 0; u < 4; ++u) {
+      for (int u = 0; u < NB; ++u) {
 #pragma clang fp contract(off)
         const int i = i0 + 8 * u, c = i + (d - 3) * g.ns;
         const double xc = R0[max(0, min(c, n - 1))];         // weight zero outside the row
-        if (first) buf_store(kbb, bo[u], kv[u]);
+        if (first) buf_store(kbb, eo[u] != kOutside ? 8 * (7 * i + d) : kOutside, kv[u]);
         const double pm = mu * mv[u];
         const double pe = fma(mu, mv[u], -pm);
         const double hi = kv[u] - pm;                        // TwoSum(kv, -pm)
@@ -1038,7 +1048,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
         mx += dpp_move<kDppHalfMirror>(mx);
         corr += dpp_move<kDppHalfMirror>(corr);
         if (d == 0 && i < n) {
-          R3[i] = corr;
+          R2[i] = corr;
           MXG[i] = mx;
         }
       }
@@ -1046,17 +1056,23 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
     first = false;
     __syncthreads();                                       // K' of every row before any row is summed
     row_sums<true>(n, g.ns, g.npr, g.bw, g.P, SC, kprof, R0, lane, [&](int i, double s, double e) {
-      e -= R3[i];
-      two_sum_acc(cq, g.muhat[i], s, e);
+      R3[i] = s;
+      R1[i] = e;
+    });
+    __syncthreads();
+    for_entries(muhb, n, lane, [&](int i, double mh) {
+      double s = R3[i], e = R1[i] - R2[i];
+      two_sum_acc(cq, mh, s, e);
       const double y3 = s + e;
       R3[i] = y3;
       Y3G[i] = y3;
     });
+    __syncthreads();
     if (!g.keep_mass) stage_mass(g, LC, lane);
     __syncthreads();
     mass_solve(g.ns, g.npr, LC, R3, lane);
     __syncthreads();
-    return proj_norm3(R3, 1.0, R0, 0.0, nullptr, 0.0, UH, n, lane);
+    return proj_norm(R3, uhb, n, lane);
   };
 
   double cp = 0.0;
@@ -1076,12 +1092,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
     if (!(tval > tol)) { status = 0; break; }
     if (it >= b.max_iter) { status = 1; break; }
     // ---- right-hand sides and factorisation of K'
-    for (int i = lane; i < n; i += 64) {
+    for_entries(profile_buf(Y3G, n), n, lane, [&](int i, double v) {
       XG[i] = R0[i];
-      R0[i] = Y3G[i];
-      R1[i] = g.muhat[i];
-      R2[i] = MXG[i];
-    }
+      R0[i] = v;
+    });
+    for_entries(muhb, n, lane, [&](int i, double v) { R1[i] = v; });
+    for_entries(profile_buf(MXG, n), n, lane, [&](int i, double v) { R2[i] = v; });
     __syncthreads();
     factor_tiles<W, T, false, 3>(g, kprof, SC, R1, R2, R0, PIV, urows, lane);
     __syncthreads();
@@ -1089,14 +1105,16 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
     __syncthreads();
     // ---- step p = delta + a z1 + b z2
     double s11 = 0.0, s12 = 0.0, s13 = 0.0, wz1 = 0.0, wz2 = 0.0, wz3 = 0.0;
-    for (int i = lane; i < n; i += 64) {
-      s11 = fma(UH[i], R1[i], s11);
-      s12 = fma(UH[i], R2[i], s12);
-      s13 = fma(UH[i], R0[i], s13);
-      wz1 = fma(WV[i], R1[i], wz1);
-      wz2 = fma(WV[i], R2[i], wz2);
-      wz3 = fma(WV[i], R0[i], wz3);
-    }
+    for_entries(uhb, n, lane, [&](int i, double v) {
+      s11 = fma(v, R1[i], s11);
+      s12 = fma(v, R2[i], s12);
+      s13 = fma(v, R0[i], s13);
+    });
+    for_entries(wvb, n, lane, [&](int i, double v) {
+      wz1 = fma(v, R1[i], wz1);
+      wz2 = fma(v, R2[i], wz2);
+      wz3 = fma(v, R0[i], wz3);
+    });
     s11 = wave_sum(s11); s12 = wave_sum(s12); s13 = wave_sum(s13);
     wz1 = wave_sum(wz1); wz2 = wave_sum(wz2); wz3 = wave_sum(wz3);
     double a, bb;
@@ -1257,7 +1275,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
   double* Z1 = X + n;
   double* Z2 = Z1 + n;
   double* LC = g.keep_mass ? Z2 + n : Z1;
-  double* AV = Z2 + n + (g.keep_mass ? 4 * g.npr : zpad(n, g.npr));
+  double* AV = Z2 + n + (g.keep_mass ? mass_len(g.npr) : zpad(n, g.npr));
   double* U0 = AV + n;
   int2* SC = reinterpret_cast<int2*>(U0 + n);
 
@@ -1276,6 +1294,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
   }
   __syncthreads();
 
+  const ProfileBuf uhb = profile_buf(UH, n), wvb = profile_buf(WV, n);
   // frozen shift: the profile holds K; make it K - mu' M, mu' from the start state
   const double mu0 = dot(WV, U0, n, lane);
   const double mup = mu0 + 1.0 / cdt;
@@ -1296,20 +1315,22 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
     __syncthreads();
     mass_solve(g.ns, g.npr, LC, AV, lane);
     __syncthreads();
-    const double mu = dot(WV, X, n, lane);
+    double mu = 0.0;
+    for_entries(wvb, n, lane, [&](int i, double v) { mu = fma(v, X[i], mu); });
+    mu = wave_sum(mu);
     double su = 0.0;
-    for (int i = lane; i < n; i += 64) {
+    for_entries(uhb, n, lane, [&](int i, double uh) {
       const double a = fma(mup, X[i], AV[i]) - mu * X[i];      // M^-1 K x - mu x
       AV[i] = a;
-      su = fma(UH[i], a, su);
-    }
+      su = fma(uh, a, su);
+    });
     su = wave_sum(su);
     double s2 = 0.0;
-    for (int i = lane; i < n; i += 64) {
-      const double gi = (X[i] - U0[i]) - cdt * (AV[i] - su * UH[i]);
+    for_entries(uhb, n, lane, [&](int i, double uh) {
+      const double gi = (X[i] - U0[i]) - cdt * (AV[i] - su * uh);
       AV[i] = gi;
       s2 = fma(gi, gi, s2);
-    }
+    });
     __syncthreads();
     return sqrt(wave_sum(s2));
   };
@@ -1344,10 +1365,12 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W
       forward_tiles<W, T>(g, lp, SC, Z2, PIV, lane);
       __syncthreads();
       back_tiles<W, 1>(g, urows, Z2, nullptr, nullptr, lane);
-      for (int i = lane; i < n; i += 64) Z1[i] = ZU[i];
+      for_entries(profile_buf(ZU, n), n, lane, [&](int i, double v) { Z1[i] = v; });
       __syncthreads();
     }
-    const double gam = dot(UH, Z2, n, lane) / su;
+    double gam = 0.0;
+    for_entries(uhb, n, lane, [&](int i, double uh) { gam = fma(uh, Z2[i], gam); });
+    gam = wave_sum(gam) / su;
     const double ic = 1.0 / cdt;
     for (int i = lane; i < n; i += 64) X[i] = fma(ic, Z2[i] - gam * Z1[i], X[i]);
     __syncthreads();
