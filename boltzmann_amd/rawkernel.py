@@ -25,7 +25,7 @@ def bidiagonal_solve_batched(diag, sdiag, b, lower):
     assert _sdiag.shape[0] == _diag.shape[0] and _sdiag.shape[0] == _b.shape[0]
     assert _sdiag.shape[1] == _diag.shape[1] - 1 and _sdiag.shape[1] == _b.shape[1] - 1
     bsz, N = _diag.shape
-    out = torch.zeros_like(_b)
+    out = torch.empty_like(_b)                 # every entry is written
     _lib.call("bz_bidiag_solve_batched", _diag, _sdiag, _b, out, bsz, N, 1 if lower else 0)
     return out.reshape(diag.shape)
 
@@ -36,7 +36,7 @@ def banded_tri_solve_batched(diags, b, lower):
     _b = _c(b).reshape((-1, b.shape[-1]))
     assert _diags.shape[0] == _b.shape[0]
     bsz, nd, N = _diags.shape
-    out = torch.zeros_like(_b)
+    out = torch.empty_like(_b)                 # every entry is written
     _lib.call("bz_banded_tri_solve_batched", _diags, _b, out, bsz, nd, N, 1 if lower else 0)
     return out.reshape(b.shape)
 
@@ -47,7 +47,7 @@ def banded_tri_mv_batched(diags, b, lower):
     _b = _c(b).reshape((-1, b.shape[-1]))
     assert _diags.shape[0] == _b.shape[0]
     bsz, nd, N = _diags.shape
-    out = torch.zeros_like(_b)
+    out = torch.empty_like(_b)                 # every entry is written
     _lib.call("bz_banded_tri_mv_batched", _diags, _b, out, bsz, nd, N, 1 if lower else 0)
     return out.reshape(b.shape)
 
