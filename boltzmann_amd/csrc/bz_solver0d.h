@@ -234,6 +234,16 @@ __device__ __forceinline__ int fresh_lane(int lane) {
   return lane;
 }
 
+// The value taken out of its register at this point of the program, so that a load may refill the
+// register (else the compiler may take it later, load into another one and copy at the loop edge,
+// waiting for every load there).
+__device__ __forceinline__ double moved(double v) {
+  asm volatile("" : "+v"(v));
+  return v;
+}
+
+__device__ __forceinline__ bool wave_any(bool p) { return __builtin_amdgcn_ballot_w64(p) != 0; }
+
 __device__ __forceinline__ void wave_lds_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
   __builtin_amdgcn_wave_barrier();
@@ -374,32 +384,43 @@ __device__ __forceinline__ void fill_rowtab(const GridDev& g, int2* __restrict__
 
 // The row whose columns a slot is reading.  Row i reads the groups first_col >> 2 .. (i >> 2) +
 // NG; the schedule gives its successor no column before group (i >> 2) + NG + 1.  LEFT: only the
-// columns left of the row's pivot block (the stored L factor).
+// columns left of the row's pivot block (the stored L factor).  The table entry of the row after
+// it, and the entry value y of the row itself, are read from LDS when the row is taken up and
+// used only later, so no step waits for them.
 template <int NG, bool LEFT>
 struct SlotRow {
-  int fc, cnt, off8, lim, row, next;
-  __device__ __forceinline__ void enter(const lds_int* rt, int r, int n, int bw) {
-    row = r;
-    const int q = row >= 0 ? row : 0;
-    const int tx = rt[2 * q], ty = rt[2 * q + 1];
-    fc = tx & 0xffff;
-    cnt = LEFT ? max(0, (row & ~3) - fc) : min(row + bw, n - 1) - fc + 1;
+  int row, ent, off8, end8;            // kNone without a row; ent: first column, next row << 16
+  int tx, ty;                          // table entry of the next row
+  double y;
+  static constexpr int kNone = 0x7ffffff0;
+  __device__ __forceinline__ int fc() const { return row != kNone ? ent & 0xffff : kNone; }
+  __device__ __forceinline__ void take(const lds_int* rt, const lds_double* yl, int r, int n, int bw) {
+    const bool ok = r >= 0;
+    row = ok ? r : kNone;
+    ent = ok ? tx : -65536;
     off8 = ty * 8;
-    lim = (row >> 2) + NG;
-    next = tx >> 16;
-    if (row < 0) {
-      fc = 0x7fffffff;
-      cnt = 0;
-      lim = 0x7fffffff;
-      next = -1;
-    }
+    end8 = ok ? off8 + 8 * (LEFT ? r & ~3 : min(r + bw, n - 1) + 1) : (int)0x80000000;
+    y = yl[max(r, 0)];
+    tx = rt[2 * max(ent >> 16, 0)];
+    ty = rt[2 * max(ent >> 16, 0) + 1];
   }
-  __device__ __forceinline__ void advance(const lds_int* rt, int h, int n, int bw) {
-    if (h > lim) enter(rt, next, n, bw);
+  __device__ __forceinline__ void init(const lds_int* rt, const lds_double* yl, int r, int n, int bw) {
+    tx = rt[2 * max(r, 0)];
+    ty = rt[2 * max(r, 0) + 1];
+    take(rt, yl, r, n, bw);
   }
-  // byte offset of the row's entry in column c (past the end outside its profile)
-  __device__ __forceinline__ int at(int c) const { return (unsigned)(c - fc) < (unsigned)cnt ? off8 + 8 * c : kOutside; }
-  __device__ __forceinline__ double load(const ProfileBuf& kb, int c) const { return buf_load(kb, at(c)); }
+  __device__ __forceinline__ void advance(const lds_int* rt, const lds_double* yl, int h, int n, int bw) {
+    const bool past = row < 4 * (h - NG);
+    if (wave_any(past))
+      if (past) take(rt, yl, ent >> 16, n, bw);
+  }
+  // Byte offset of the row's entry in column c8 / 8, past the end of the profile outside the row.
+  // Without LEFT, columns left of the row's first read other rows' entries: their group is masked
+  // when it becomes the panel.
+  __device__ __forceinline__ int at(int c8) const {
+    const int o = off8 + c8;
+    return o < end8 && (!LEFT || c8 >= 8 * (ent & 0xffff)) ? o : kOutside;
+  }
 };
 
 // 4 x 4 LU without pivoting of the pivot block a[k][c], and what the block step needs of it.
@@ -493,16 +514,16 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
   for (int t = 0; t < T; ++t) {
     const int slot = 16 * t + a16;
     const int row = slot < g.nslots ? g.slot_first[slot] : -1;
-    st[t].enter(rt, row, n, bw);
-    crow[t] = row;
-    cfc[t] = st[t].fc;
+    st[t].init(rt, yq, row, n, bw);
+    crow[t] = st[t].row;
+    cfc[t] = st[t].fc();
     if constexpr (SL) coff[t] = st[t].off8 >> 3;
-    const double y0 = (q < NRHS && row >= 0) ? (double)yq[row] : 0.0;
-    P[t] = st[t].load(kb, q);
+    const double y0 = (q < NRHS && row >= 0) ? st[t].y : 0.0;
+    P[t] = q >= cfc[t] ? buf_load(kb, st[t].at(8 * q)) : 0.0;
     R4[t] = v4d{0.0, 0.0, 0.0, 0.0};
 #pragma unroll
     for (int s = 1; s <= NG; ++s) {
-      const double v = st[t].load(kb, 4 * s + q);
+      const double v = buf_load(kb, st[t].at(8 * (4 * s + q)));
       if (s % NG < 4) R4[t][s % NG < 4 ? s % NG : 0] = v;
       else RX[NX ? t : 0] = v;
     }
@@ -510,8 +531,8 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
     else Y[t] = y0;
 #pragma unroll
     for (int s = 0; s < NG; ++s) {
-      st[t].advance(rt, NG + 1 + s, n, bw);
-      F[t][s] = st[t].load(kb, 4 * (NG + 1 + s) + q);
+      st[t].advance(rt, yq, NG + 1 + s, n, bw);
+      F[t][s] = buf_load(kb, st[t].at(8 * (4 * (NG + 1 + s) + q)));
     }
   }
   // Wait for the loads so far here, once: with them in flight at the loop entry, in another order
@@ -535,33 +556,33 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
       }
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        const bool mine = (crow[t] >> 2) == gb;
-        double y0 = 0.0;
-        if (mine) {
-          lds_double* pk = piv + 4 * q + (crow[t] & 3);
-          pk[0] = P[t];
+        const int rel = crow[t] - 4 * gb;
+        const bool mine = (unsigned)rel < 4u;
+        if (wave_any(mine)) {
+          if (mine) {
+            lds_double* pk = piv + 4 * q + rel;
+            pk[0] = P[t];
 #pragma unroll
-          for (int r = 0; r < NG; ++r) pk[16 * (r > u ? r - u : r - u + NG)] = r < 4 ? R4[t][r < 4 ? r : 0] : RX[NX ? t : 0];
-          pk[16 * (NG + 1)] = Y16 ? R4[t][YR] : Y[Y16 ? 0 : t];
-          // the slot's next row (already the one being read)
-          const int nr = st[t].row;
-          if (q < NRHS && nr >= 0) y0 = yq[nr];
-          crow[t] = nr;
-          cfc[t] = st[t].fc;
-          if constexpr (SL) coff[t] = st[t].off8 >> 3;
+            for (int r = 0; r < NG; ++r) pk[16 * (r > u ? r - u : r - u + NG)] = r < 4 ? R4[t][r < 4 ? r : 0] : RX[NX ? t : 0];
+            pk[16 * (NG + 1)] = Y16 ? R4[t][YR] : Y[Y16 ? 0 : t];
+          }
+          // The slot's next row, already the one being read: no column of it has arrived yet;
+          // what the ring still holds is the old row's and is masked as it becomes the panel.
+          const double y0 = (q < NRHS && st[t].row != SlotRow<NG, false>::kNone) ? st[t].y : 0.0;
+          P[t] = mine ? 0.0 : P[t];
+          if constexpr (Y16) R4[t][YR] = mine ? y0 : R4[t][YR];
+          else Y[t] = mine ? y0 : Y[t];
+          crow[t] = mine ? st[t].row : crow[t];
+          cfc[t] = mine ? st[t].fc() : cfc[t];
+          if constexpr (SL) coff[t] = mine ? st[t].off8 >> 3 : coff[t];
         }
-        // No column of the next row has arrived yet; what the ring still holds is the old row's
-        // and is masked as it becomes the panel.
-        P[t] = mine ? 0.0 : P[t];
-        if constexpr (Y16) R4[t][YR] = mine ? y0 : R4[t][YR];
-        else Y[t] = mine ? y0 : Y[t];
       }
       // --- where the next group of every slot is read from
       int nx_o[T];
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        st[t].advance(rt, gb + 2 * NG + 1, n, bw);
-        nx_o[t] = st[t].at(4 * (gb + 2 * NG + 1) + q);
+        st[t].advance(rt, yq, gb + 2 * NG + 1, n, bw);
+        nx_o[t] = st[t].at(8 * (4 * (gb + 2 * NG + 1) + q));
       }
       wave_lds_fence();
       const lds_v4d* pc = (const lds_v4d*)piv;
@@ -605,7 +626,7 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
       if constexpr (SL) {
 #pragma unroll
         for (int t = 0; t < T; ++t)
-          if (crow[t] >= 0 && 4 * gb + q >= cfc[t]) lout[coff[t] + 4 * gb + q] = l[t];
+          if (4 * gb + q >= cfc[t]) lout[coff[t] + 4 * gb + q] = l[t];
         // the strict lower part of the pivot block's own factor
         if (a16 < q && j < n) {
           const int c = 4 * gb + a16;
@@ -624,10 +645,10 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
         const bool in = 4 * gb + 4 + q >= cfc[t];
         if (r < 4) {
           P[t] = in ? R4[t][r < 4 ? r : 0] : 0.0;
-          R4[t][r < 4 ? r : 0] = F[t][u];
+          R4[t][r < 4 ? r : 0] = moved(F[t][u]);
         } else {
           P[t] = in ? RX[NX ? t : 0] : 0.0;
-          RX[NX ? t : 0] = F[t][u];
+          RX[NX ? t : 0] = moved(F[t][u]);
         }
         F[t][u] = buf_load(kb, nx_o[t]);
       }
@@ -643,7 +664,7 @@ template <int W, int T>
 __device__ __forceinline__ void forward_tiles(const GridDev& g, const double* __restrict__ lprof, const int2* __restrict__ rt_,
                               double* __restrict__ y_, double* __restrict__ piv_, int lane) {
   lane = fresh_lane(lane);
-  constexpr int NG = trail_groups<W>(), PF = 4;
+  constexpr int NG = trail_groups<W>(), PF = NG + 2;        // at its pivot step a slot already reads its next row
   const int n = g.n, bw = g.bw;
   const int q = lane >> 4, a16 = lane & 15;
   const ProfileBuf lb = profile_buf(lprof, g.P);
@@ -664,16 +685,16 @@ __device__ __forceinline__ void forward_tiles(const GridDev& g, const double* __
   for (int t = 0; t < T; ++t) {
     const int slot = 16 * t + a16;
     const int row = slot < g.nslots ? g.slot_first[slot] : -1;
-    st[t].enter(rt, row, n, bw);
-    crow[t] = row;
-    Y[t] = row >= 0 ? (double)yl[row] : 0.0;
+    st[t].init(rt, yl, row, n, bw);
+    crow[t] = st[t].row;
+    Y[t] = row >= 0 ? st[t].y : 0.0;
   }
 #pragma unroll
   for (int s = 0; s < PF; ++s) {
 #pragma unroll
     for (int t = 0; t < T; ++t) {
-      st[t].advance(rt, s, n, bw);
-      F[t][s] = st[t].load(lb, 4 * s + q);
+      st[t].advance(rt, yl, s, n, bw);
+      F[t][s] = buf_load(lb, st[t].at(8 * (4 * s + q)));
     }
     D[s] = diag(s);
   }
@@ -686,18 +707,19 @@ __device__ __forceinline__ void forward_tiles(const GridDev& g, const double* __
       if (lane < 4 && 4 * gb + lane >= n) piv[lane] = 0.0;
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        if ((crow[t] >> 2) == gb) {
-          if (q == 0) piv[crow[t] & 3] = Y[t];
-          const int nr = rt[2 * crow[t]] >> 16;
-          crow[t] = nr;
-          Y[t] = nr >= 0 ? (double)yl[nr] : 0.0;
+        const int rel = crow[t] - 4 * gb;
+        const bool mine = (unsigned)rel < 4u;
+        if (wave_any(mine)) {
+          if (mine && q == 0) piv[rel] = Y[t];
+          Y[t] = mine ? (st[t].row != SlotRow<NG, true>::kNone ? st[t].y : 0.0) : Y[t];
+          crow[t] = mine ? st[t].row : crow[t];
         }
       }
       int nx_o[T];
 #pragma unroll
       for (int t = 0; t < T; ++t) {
-        st[t].advance(rt, gb + PF, n, bw);
-        nx_o[t] = st[t].at(4 * (gb + PF) + q);
+        st[t].advance(rt, yl, gb + PF, n, bw);
+        nx_o[t] = st[t].at(8 * (4 * (gb + PF) + q));
       }
       wave_lds_fence();
       const v4d v = *(const lds_v4d*)piv;
@@ -742,20 +764,23 @@ __device__ __forceinline__ void back_tiles(const GridDev& g, const double* __res
   double A[PD][NG + 1], Z[NG];
 #pragma unroll
   for (int s = 0; s < NG; ++s) Z[s] = 0.0;
+  // in the order of the loop, so that the compiler's wait analysis sees one order
 #pragma unroll
-  for (int u = 0; u < PD; ++u)
+  for (int u = PD - 1; u >= 0; --u) {
 #pragma unroll
-    for (int s = 0; s <= NG; ++s) A[u][s] = buf_load(ub, uo[s] + (nu - PD + u) * (4 * WP * 8));
+    for (int s = NG; s >= 0; --s) A[u][s] = buf_load(ub, uo[s] + (nu - PD + u) * (4 * WP * 8));
+    __builtin_amdgcn_sched_barrier(0);
+  }
   // Rows past the last have zero rows of U, U11^-1 among them, so any finite value does there.
   auto rhs = [&](int gb) -> double { return yj[min(max(4 * gb + q, 0), n - 1)]; };
-  double yn = rhs(nu - 1);
-  __builtin_amdgcn_s_waitcnt(0x0F70);                 // as in factor_tiles
+  double yn = rhs(nu - 1), yn2 = rhs(nu - 2);
   for (int g0 = nu - PD; g0 >= 0; g0 -= PD) {
 #pragma unroll
     for (int u = PD - 1; u >= 0; --u) {
       const int gb = g0 + u;
       double acc = yn;
-      yn = rhs(gb - 1);
+      yn = yn2;
+      yn2 = rhs(gb - 2);
 #pragma unroll
       for (int s = NG; s >= 1; --s) acc = mfma4(A[u][s], Z[(u + s) % NG], acc);
       const double z = mfma4(A[u][0], acc, 0.0);
@@ -763,7 +788,7 @@ __device__ __forceinline__ void back_tiles(const GridDev& g, const double* __res
       if (b4 == 0 && live && 4 * gb + q < n) yj[4 * gb + q] = z;
       // rows of block gb - PD; a negative block is past the end as an unsigned offset
 #pragma unroll
-      for (int s = 0; s <= NG; ++s) A[u][s] = buf_load(ub, gb >= PD ? uo[s] + (gb - PD) * (4 * WP * 8) : kOutside);
+      for (int s = NG; s >= 0; --s) A[u][s] = buf_load(ub, uo[s] + (gb - PD) * (4 * WP * 8));
     }
   }
 }
