@@ -459,8 +459,8 @@ class bte_1d3v:
         key = (float(dt), float(alpha))
         if self._dg is None or self._dg_key != key:
             op, E = self._op, self._Ebuf
-            mv = lambda src, dst: _lib.call("bz_fvm_rhs_mvec", op, E, key[0], src, dst)
-            pc = lambda src, dst: _lib.call("bz_fvm_precond_xvtvrc", op, E, key[1] * key[0], src, dst)
+            mv = lambda src, dst, done: _lib.call("bz_fvm_rhs_mvec_until", op, E, key[0], src, dst, done)
+            pc = lambda src, dst, done: _lib.call("bz_fvm_precond_xvtvrc_until", op, E, key[1] * key[0], src, dst, done)
             self._dg = DeviceGMRES(self.dof_v * self.dof_x, self.params.gmres_rsrt, self.dev, mv, pc,
                                    gs_passes=self.gs_passes)
             self._dg_key = key

@@ -23,7 +23,9 @@ constexpr int MAXB = 8;       // widest stencil (pvr, pvt, px <= 7)
 
 // s[r, x] = sum_t wq[t] v[(r Nvt + t) Nx + x]
 __global__ __launch_bounds__(256) void k_fvm_moment(const double* __restrict__ v, const double* __restrict__ wq,
-                                                    int Nr, int Nvt, int Nx, double* __restrict__ s) {
+                                                    int Nr, int Nvt, int Nx, double* __restrict__ s,
+                                                    const int* __restrict__ done) {
+  if (done && *done) return;
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= Nr * Nx) return;
   const int r = e / Nx, ix = e - r * Nx;
@@ -45,7 +47,8 @@ __global__ __launch_bounds__(256) void k_fvm_moment(const double* __restrict__ v
 // One element (r, t, x) of the step operator per thread.
 __global__ __launch_bounds__(256) void k_fvm_matvec(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                     const double* __restrict__ x, const double* __restrict__ s,
-                                                    double* __restrict__ y) {
+                                                    double* __restrict__ y, const int* __restrict__ done) {
+  if (done && *done) return;
   const int Nr = op.Nr, Nvt = op.Nvt, Nx = op.Nx;
   // 32-bit index arithmetic (the size is checked below 2^31 by the host)
   const unsigned eu = blockIdx.x * 256u + threadIdx.x;
@@ -107,7 +110,8 @@ __global__ __launch_bounds__(256) void k_fvm_matvec(BzFvm1d3v op, const double* 
 template <int NX, int NVR, int NVT, int GMAX>
 __global__ __launch_bounds__(256) void k_fvm_matvec_w(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                       const double* __restrict__ x, const double* __restrict__ s,
-                                                      double* __restrict__ y) {
+                                                      double* __restrict__ y, const int* __restrict__ done) {
+  if (done && *done) return;
   const int Nr = op.Nr, Nvt = op.Nvt, Nx = op.Nx;
   // Workgroups of one state row (r, t) each, threads over x: the row indices are workgroup-
   // uniform (no per-thread division).  Workgroups are dealt to the 8 XCDs in turn (workgroup
@@ -212,7 +216,9 @@ constexpr int CC_WAVES = 8;
 __global__ __launch_bounds__(64 * CC_WAVES) void k_fvm_coll_corr(const double* __restrict__ H,
                                                                  const int* __restrict__ h_lo,
                                                                  const double* __restrict__ s, int Nr, int Nx,
-                                                                 double* __restrict__ h) {
+                                                                 double* __restrict__ h,
+                                                                 const int* __restrict__ done) {
+  if (done && *done) return;
   __shared__ double red[CC_WAVES - 1][256];
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int i16 = lane & 15, k4 = lane >> 4;
@@ -270,7 +276,8 @@ constexpr int SW_LDS_DOUBLES = 8192;
 template <int MODE, int ND, bool LDS>
 __global__ __launch_bounds__(SWT) void k_fvm_sweep(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                    const double* b, double* out,   // may alias
-                                                   const double* __restrict__ h) {
+                                                   const double* __restrict__ h, const int* __restrict__ done) {
+  if (done && *done) return;
   extern __shared__ double sm[];
   constexpr int PF = (MODE == SW_VR && ND <= 4) ? 16 : 8;   // the radial sweep is the longest
   const int Nr = op.Nr, Nvt = op.Nvt, Nx = op.Nx;
@@ -389,7 +396,8 @@ constexpr int SCAN_SB = 8, NSEG = 32;
 template <int ND, int MAXL, int SB>
 __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                         const double* __restrict__ b, double* __restrict__ out,
-                                                        const double* __restrict__ h) {
+                                                        const double* __restrict__ h, const int* __restrict__ done) {
+  if (done && *done) return;
   constexpr int K = ND > 1 ? ND - 1 : 1;
   constexpr int NL = MAXL > 0 ? MAXL : 1;
   __shared__ double maps[SB * NSEG][K * K + K];
@@ -514,22 +522,22 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
 
 template <int ND, int SB>
 void launch_vr_scan(const BzFvm1d3v& op, const double* E, double dt, const double* b, double* out, const double* h,
-                    hipStream_t st) {
+                    const int* done, hipStream_t st) {
   const int nsys = op.Nvt * op.Nx;
   const int L = (op.Nr + NSEG - 1) / NSEG;
   const dim3 grid((nsys + SB - 1) / SB), block(SB * NSEG);
-  if (L <= 8) hipLaunchKernelGGL((k_fvm_vr_scan<ND, 8, SB>), grid, block, 0, st, op, E, dt, b, out, h);
-  else if (L <= 24) hipLaunchKernelGGL((k_fvm_vr_scan<ND, 24, SB>), grid, block, 0, st, op, E, dt, b, out, h);
-  else hipLaunchKernelGGL((k_fvm_vr_scan<ND, 0, SB>), grid, block, 0, st, op, E, dt, b, out, h);
+  if (L <= 8) hipLaunchKernelGGL((k_fvm_vr_scan<ND, 8, SB>), grid, block, 0, st, op, E, dt, b, out, h, done);
+  else if (L <= 24) hipLaunchKernelGGL((k_fvm_vr_scan<ND, 24, SB>), grid, block, 0, st, op, E, dt, b, out, h, done);
+  else hipLaunchKernelGGL((k_fvm_vr_scan<ND, 0, SB>), grid, block, 0, st, op, E, dt, b, out, h, done);
 }
 
 int launch_fvm_vr_scan(const BzFvm1d3v& op, const double* E, double dt, const double* b, double* out,
-                       const double* h, hipStream_t st) {
+                       const double* h, const int* done, hipStream_t st) {
   switch (op.nvr) {
-    case 2: launch_vr_scan<2, SCAN_SB>(op, E, dt, b, out, h, st); break;
-    case 3: launch_vr_scan<3, SCAN_SB>(op, E, dt, b, out, h, st); break;
-    case 4: launch_vr_scan<4, SCAN_SB>(op, E, dt, b, out, h, st); break;
-    case 5: launch_vr_scan<5, SCAN_SB>(op, E, dt, b, out, h, st); break;
+    case 2: launch_vr_scan<2, SCAN_SB>(op, E, dt, b, out, h, done, st); break;
+    case 3: launch_vr_scan<3, SCAN_SB>(op, E, dt, b, out, h, done, st); break;
+    case 4: launch_vr_scan<4, SCAN_SB>(op, E, dt, b, out, h, done, st); break;
+    case 5: launch_vr_scan<5, SCAN_SB>(op, E, dt, b, out, h, done, st); break;
     default: return BZ_EINVAL;
   }
   BZ_LAUNCH_CHECK();
@@ -543,7 +551,9 @@ int launch_fvm_vr_scan(const BzFvm1d3v& op, const double* E, double dt, const do
 // the lane re-runs them.  The maps are contractions (upwind), so the re-association changes
 // the result at rounding level.
 template <int PER>
-__global__ __launch_bounds__(64) void k_fvm_x_scan(BzFvm1d3v op, double dt, const double* b, double* out) {
+__global__ __launch_bounds__(64) void k_fvm_x_scan(BzFvm1d3v op, double dt, const double* b, double* out,
+                                                   const int* __restrict__ done) {
+  if (done && *done) return;
   const int s = blockIdx.x, lane = threadIdx.x;
   const int Nvt = op.Nvt, Nx = op.Nx;
   const int r = s / Nvt, t = s - r * Nvt;
@@ -590,30 +600,30 @@ __global__ __launch_bounds__(64) void k_fvm_x_scan(BzFvm1d3v op, double dt, cons
 
 template <int MODE, int ND>
 void launch_sweep_nd(const BzFvm1d3v& op, int N, int nsys, const double* E, double dt, const double* b, double* out,
-                     const double* h, hipStream_t st) {
+                     const double* h, const int* done, hipStream_t st) {
   const size_t lds = (size_t)(2 * ND + (MODE == SW_VR ? 1 : 0)) * N;
   const dim3 grid((nsys + SWT - 1) / SWT), block(SWT);
   if (lds <= SW_LDS_DOUBLES)
-    hipLaunchKernelGGL((k_fvm_sweep<MODE, ND, true>), grid, block, lds * sizeof(double), st, op, E, dt, b, out, h);
+    hipLaunchKernelGGL((k_fvm_sweep<MODE, ND, true>), grid, block, lds * sizeof(double), st, op, E, dt, b, out, h, done);
   else
-    hipLaunchKernelGGL((k_fvm_sweep<MODE, ND, false>), grid, block, 0, st, op, E, dt, b, out, h);
+    hipLaunchKernelGGL((k_fvm_sweep<MODE, ND, false>), grid, block, 0, st, op, E, dt, b, out, h, done);
 }
 
 template <int MODE>
 int launch_fvm_sweep(const BzFvm1d3v& op, const double* E, double dt, const double* b, double* out, const double* h,
-                     hipStream_t st) {
+                     const int* done, hipStream_t st) {
   const int N = MODE == SW_VR ? op.Nr : (MODE == SW_VT ? op.Nvt : op.Nx);
   const int nsys = MODE == SW_VR ? op.Nvt * op.Nx : (MODE == SW_VT ? op.Nr * op.Nx : op.Nr * op.Nvt);
   const int nd = MODE == SW_VR ? op.nvr : (MODE == SW_VT ? op.nvt : op.nx);
   switch (nd) {
-    case 1: launch_sweep_nd<MODE, 1>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 2: launch_sweep_nd<MODE, 2>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 3: launch_sweep_nd<MODE, 3>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 4: launch_sweep_nd<MODE, 4>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 5: launch_sweep_nd<MODE, 5>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 6: launch_sweep_nd<MODE, 6>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 7: launch_sweep_nd<MODE, 7>(op, N, nsys, E, dt, b, out, h, st); break;
-    case 8: launch_sweep_nd<MODE, 8>(op, N, nsys, E, dt, b, out, h, st); break;
+    case 1: launch_sweep_nd<MODE, 1>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 2: launch_sweep_nd<MODE, 2>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 3: launch_sweep_nd<MODE, 3>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 4: launch_sweep_nd<MODE, 4>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 5: launch_sweep_nd<MODE, 5>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 6: launch_sweep_nd<MODE, 6>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 7: launch_sweep_nd<MODE, 7>(op, N, nsys, E, dt, b, out, h, done, st); break;
+    case 8: launch_sweep_nd<MODE, 8>(op, N, nsys, E, dt, b, out, h, done, st); break;
     default: return BZ_EINVAL;
   }
   BZ_LAUNCH_CHECK();
@@ -633,8 +643,8 @@ int check_op(const BzFvm1d3v* op) {
 
 extern "C" {
 
-int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y,
-                    hipStream_t stream) {
+int bz_fvm_rhs_mvec_until(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y, const int* done,
+                          hipStream_t stream) {
   int rc = check_op(op);
   if (rc != BZ_OK) return rc;
   if (!E || !x || !y || x == y) return BZ_EINVAL;
@@ -644,7 +654,7 @@ int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
   const int nrx = op->Nr * op->Nx;
   double* s = op->work;
   hipLaunchKernelGGL(k_fvm_moment, dim3((nrx + 255) / 256), dim3(256), 0, stream, x, op->wq, op->Nr, op->Nvt, op->Nx,
-                     s);
+                     s, done);
   BZ_LAUNCH_CHECK();
   const long n = (long)nrx * op->Nvt;
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
@@ -653,17 +663,17 @@ int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
   const dim3 growx((unsigned)((nwg + 7) / 8 * 8)), browx(tx);
   const bool rows_fit = nwg < (1L << 30);
   if (rows_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
-    hipLaunchKernelGGL((k_fvm_matvec_w<2, 4, 4, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y);
+    hipLaunchKernelGGL((k_fvm_matvec_w<2, 4, 4, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
   else if (rows_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
-    hipLaunchKernelGGL((k_fvm_matvec_w<3, 3, 3, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y);
+    hipLaunchKernelGGL((k_fvm_matvec_w<3, 3, 3, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
   else
-    hipLaunchKernelGGL(k_fvm_matvec, grid, block, 0, stream, *op, E, dt, x, s, y);
+    hipLaunchKernelGGL(k_fvm_matvec, grid, block, 0, stream, *op, E, dt, x, s, y, done);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }
 
-int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
-                          hipStream_t stream) {
+int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
+                                const int* done, hipStream_t stream) {
   int rc = check_op(op);
   if (rc != BZ_OK) return rc;
   if (!E || !b || !y || b == y) return BZ_EINVAL;
@@ -675,30 +685,40 @@ int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt,
   double* h = op->work + nrx;
   // collisions: s_b, then h = H s_b (the sweep adds b / A + h)
   hipLaunchKernelGGL(k_fvm_moment, dim3((nrx + 255) / 256), dim3(256), 0, stream, b, op->wq, op->Nr, op->Nvt, op->Nx,
-                     s);
+                     s, done);
   BZ_LAUNCH_CHECK();
   hipLaunchKernelGGL(k_fvm_coll_corr, dim3((op->Nr + 15) / 16, (op->Nx + 15) / 16), dim3(64 * CC_WAVES), 0, stream,
-                     op->H, op->h_lo, s, op->Nr, op->Nx, h);
+                     op->H, op->h_lo, s, op->Nr, op->Nx, h, done);
   BZ_LAUNCH_CHECK();
   // the radial sweep: segmented scan for the common stencils and long radial lines, else one
   // thread per line
   if (op->nvr >= 2 && op->nvr <= 5 && op->Nr >= 2 * NSEG)
-    rc = launch_fvm_vr_scan(*op, E, alpha_dt, b, y, h, stream);
+    rc = launch_fvm_vr_scan(*op, E, alpha_dt, b, y, h, done, stream);
   else
-    rc = launch_fvm_sweep<SW_VR>(*op, E, alpha_dt, b, y, h, stream);
+    rc = launch_fvm_sweep<SW_VR>(*op, E, alpha_dt, b, y, h, done, stream);
   if (rc != BZ_OK) return rc;
-  rc = launch_fvm_sweep<SW_VT>(*op, E, alpha_dt, y, y, nullptr, stream);
+  rc = launch_fvm_sweep<SW_VT>(*op, E, alpha_dt, y, y, nullptr, done, stream);
   if (rc != BZ_OK) return rc;
   if (op->nx == 2 && op->Nx <= 64 * 8) {
     const dim3 grid(op->Nr * op->Nvt), block(64);
     const int per = (op->Nx + 63) / 64;
-    if (per <= 2) hipLaunchKernelGGL((k_fvm_x_scan<2>), grid, block, 0, stream, *op, alpha_dt, y, y);
-    else if (per <= 4) hipLaunchKernelGGL((k_fvm_x_scan<4>), grid, block, 0, stream, *op, alpha_dt, y, y);
-    else hipLaunchKernelGGL((k_fvm_x_scan<8>), grid, block, 0, stream, *op, alpha_dt, y, y);
+    if (per <= 2) hipLaunchKernelGGL((k_fvm_x_scan<2>), grid, block, 0, stream, *op, alpha_dt, y, y, done);
+    else if (per <= 4) hipLaunchKernelGGL((k_fvm_x_scan<4>), grid, block, 0, stream, *op, alpha_dt, y, y, done);
+    else hipLaunchKernelGGL((k_fvm_x_scan<8>), grid, block, 0, stream, *op, alpha_dt, y, y, done);
     BZ_LAUNCH_CHECK();
     return BZ_OK;
   }
-  return launch_fvm_sweep<SW_X>(*op, E, alpha_dt, y, y, nullptr, stream);
+  return launch_fvm_sweep<SW_X>(*op, E, alpha_dt, y, y, nullptr, done, stream);
+}
+
+int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y,
+                    hipStream_t stream) {
+  return bz_fvm_rhs_mvec_until(op, E, dt, x, y, nullptr, stream);
+}
+
+int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
+                          hipStream_t stream) {
+  return bz_fvm_precond_xvtvrc_until(op, E, alpha_dt, b, y, nullptr, stream);
 }
 
 }  // extern "C"

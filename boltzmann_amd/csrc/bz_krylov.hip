@@ -99,6 +99,274 @@ __global__ void k_hess_lstsq(const double* __restrict__ H, int ldh, int m, const
   }
 }
 
+// ---------------------------------------------------------------- one Arnoldi step in three launches
+// The vector part of a step (classical Gram-Schmidt, the norm, the scaling, the rotation of the new
+// column) as k_orth_dots, k_orth_update and k_orth_finish.  The reductions end in the kernel that
+// needs them: every workgroup adds the few hundred partial sums of the kernel before it, in one
+// order, so no launch and no gap is spent on a reduction, the rotation runs in the first workgroup
+// while the others scale, and |w|^2 is accumulated where w is written.  What bounds it: the rows of
+// V in the dots and the update (8 n bytes each), launch latency for small n.  Measured as whole
+// implicit steps against separate dot, reduce, update, dot, reduce, scale and rotation launches,
+// steps past convergence done in full: n = 1.07e6 4427 -> 3718 us, n = 21000 1064 -> 758 us.  A set
+// stop flag turns every launch into a no-op.
+constexpr int OT = 512;        // threads
+constexpr int OJ = 4;          // basis vectors per workgroup in the dots
+constexpr int OH = 256;        // basis vectors whose coefficients are held at a time in the update
+
+__device__ __forceinline__ double block_sum(double v, double* red) {   // OT threads, all get the sum
+  v = bz::wave_sum(v);
+  __syncthreads();
+  if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6] = v;
+  __syncthreads();
+  double s = 0.0;
+#pragma unroll
+  for (int w = 0; w < OT / 64; ++w) s += red[w];
+  return s;
+}
+
+// partial[j * gridDim.x + blockIdx.x] = sum over this block's chunk of V[j][e] u[e],
+// j = OJ blockIdx.y ...
+__global__ __launch_bounds__(OT) void k_orth_dots(const double* __restrict__ V, long ldv, int nv,
+                                                  const double* __restrict__ u, long n, long chunk,
+                                                  double* __restrict__ partial, const int* __restrict__ done) {
+  if (*done) return;
+  __shared__ double red[OT / 64][OJ];
+  const int j0 = blockIdx.y * OJ;
+  const long a = (long)blockIdx.x * chunk, b = std::min(n, a + chunk);
+  const double* v[OJ];
+#pragma unroll
+  for (int j = 0; j < OJ; ++j) v[j] = V + (long)std::min(j0 + j, nv - 1) * ldv;
+  double acc[OJ] = {0.0, 0.0, 0.0, 0.0};
+  long e = a + threadIdx.x;
+  for (; e + OT < b; e += 2 * OT) {
+    const double u0 = u[e], u1 = u[e + OT];
+    double v0[OJ], v1[OJ];
+#pragma unroll
+    for (int j = 0; j < OJ; ++j) {
+      v0[j] = v[j][e];
+      v1[j] = v[j][e + OT];
+    }
+#pragma unroll
+    for (int j = 0; j < OJ; ++j) acc[j] = fma(v1[j], u1, fma(v0[j], u0, acc[j]));
+  }
+  if (e < b) {
+    const double u0 = u[e];
+#pragma unroll
+    for (int j = 0; j < OJ; ++j) acc[j] = fma(v[j][e], u0, acc[j]);
+  }
+#pragma unroll
+  for (int j = 0; j < OJ; ++j) {
+    const double w = bz::wave_sum(acc[j]);
+    if ((threadIdx.x & 63) == 0) red[threadIdx.x >> 6][j] = w;
+  }
+  __syncthreads();
+  if (threadIdx.x < OJ && j0 + (int)threadIdx.x < nv) {
+    double t = 0.0;
+#pragma unroll
+    for (int w = 0; w < OT / 64; ++w) t += red[w][threadIdx.x];
+    partial[(long)(j0 + threadIdx.x) * gridDim.x + blockIdx.x] = t;
+  }
+}
+
+// h_j = sum of the nblk partials of vector j (to column H[., col], added to it when accumulate);
+// w -= sum_j h_j V_j; with norm_partial also the block's part of |w|^2
+__global__ __launch_bounds__(OT) void k_orth_update(const double* __restrict__ V, long ldv, int nv,
+                                                    const double* __restrict__ partial, int nblk,
+                                                    double* __restrict__ w, long n, long chunk,
+                                                    double* __restrict__ H, int ldh, int col, int accumulate,
+                                                    double* __restrict__ norm_partial, const int* __restrict__ done) {
+  if (*done) return;
+  __shared__ double h[OH], red[OT / 64];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const long a = (long)blockIdx.x * chunk, b = std::min(n, a + chunk);
+  double sq = 0.0;
+  for (int j0 = 0; j0 < nv; j0 += OH) {
+    const int nj = std::min(OH, nv - j0);
+    for (int j = wave; j < nj; j += OT / 64) {
+      double t = 0.0;
+      for (int k = lane; k < nblk; k += 64) t += partial[(long)(j0 + j) * nblk + k];
+      t = bz::wave_sum(t);
+      if (lane == 0) {
+        h[j] = t;
+        if (blockIdx.x == 0) {
+          double* hp = H + (long)(j0 + j) * ldh + col;
+          *hp = accumulate ? *hp + t : t;
+        }
+      }
+    }
+    __syncthreads();
+    const bool last = j0 + OH >= nv;
+    const double* Vj = V + (long)j0 * ldv;
+    for (long e0 = a + threadIdx.x; e0 < b; e0 += 2 * OT) {
+      const long e1 = e0 + OT < b ? e0 + OT : e0;
+      double s0 = 0.0, s1 = 0.0;
+      int j = 0;
+      for (; j + 4 <= nj; j += 4) {
+        double v0[4], v1[4];
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          v0[i] = Vj[(long)(j + i) * ldv + e0];
+          v1[i] = Vj[(long)(j + i) * ldv + e1];
+        }
+#pragma unroll
+        for (int i = 0; i < 4; ++i) {
+          s0 = fma(h[j + i], v0[i], s0);
+          s1 = fma(h[j + i], v1[i], s1);
+        }
+      }
+      for (; j < nj; ++j) {
+        s0 = fma(h[j], Vj[(long)j * ldv + e0], s0);
+        s1 = fma(h[j], Vj[(long)j * ldv + e1], s1);
+      }
+      const double w0 = w[e0] - s0, w1 = w[e1] - s1;
+      w[e0] = w0;
+      if (e1 != e0) w[e1] = w1;
+      if (last) sq = fma(w0, w0, e1 != e0 ? fma(w1, w1, sq) : sq);
+    }
+    __syncthreads();
+  }
+  if (norm_partial) {
+    const double t = block_sum(sq, red);
+    if (threadIdx.x == 0) norm_partial[blockIdx.x] = t;
+  }
+}
+
+// The new column h[0..i] of the triangular factor (h[r] at h[r * hs]) under the rotations before
+// it, its own rotation, the rotated right-hand side and the stop test; hn = H[i+1][i].
+__device__ void rotate_column(double* h, long hs, const double* cs, const double* sn, int i, double hn, double* cs_out,
+                              double* sn_out, double* g, double tol, int* done, int* kdone) {
+  double a = h[0];
+  for (int k = 0; k < i; ++k) {
+    const double b = h[(k + 1) * hs], c = cs[k], s = sn[k];
+    h[k * hs] = c * a + s * b;
+    a = -s * a + c * b;
+  }
+  const double r = hypot(a, hn);
+  const double c = (r > 0.0) ? a / r : 1.0, s = (r > 0.0) ? hn / r : 0.0;
+  *cs_out = c;
+  *sn_out = s;
+  h[i * hs] = r;
+  const double gi = g[i], gn = -s * gi;
+  g[i] = c * gi;
+  g[i + 1] = gn;
+  if (fabs(gn) <= tol || hn == 0.0) {
+    *kdone = i + 1;
+    *done = 1;
+  }
+}
+
+// hn = |w| from the partial sums, V_(i+1) = w / hn (not written when hn = 0); the first workgroup
+// rotates column i of H.  A workgroup that starts after the flag is set skips its part of
+// V_(i+1), which nothing reads then.
+__global__ __launch_bounds__(OT) void k_orth_finish(const double* __restrict__ norm_partial, int nblk,
+                                                    const double* __restrict__ w, double* __restrict__ Vn, long n,
+                                                    double* __restrict__ H, int ldh, int i, double* __restrict__ cs,
+                                                    double* __restrict__ sn, double* __restrict__ g,
+                                                    const double* __restrict__ tol, int* done, int* kdone) {
+  if (*done) return;
+  constexpr int CL = 512;                            // columns up to this length are rotated in LDS
+  __shared__ double red[OT / 64], hc[CL], sc[CL], ss[CL];
+  double t = 0.0;
+  for (int k = threadIdx.x; k < nblk; k += OT) t += norm_partial[k];
+  const double hn = sqrt(block_sum(t, red));
+  if (hn != 0.0)
+    for (long e = (long)blockIdx.x * OT + threadIdx.x; e < n; e += (long)gridDim.x * OT) Vn[e] = w[e] / hn;
+  if (blockIdx.x != 0) return;
+  if (i < CL) {
+    if ((int)threadIdx.x <= i) {
+      hc[threadIdx.x] = H[(long)threadIdx.x * ldh + i];
+      sc[threadIdx.x] = cs[threadIdx.x];
+      ss[threadIdx.x] = sn[threadIdx.x];
+    }
+    __syncthreads();
+    if (threadIdx.x == 0) rotate_column(hc, 1, sc, ss, i, hn, cs + i, sn + i, g, tol[0], done, kdone);
+    __syncthreads();
+    if ((int)threadIdx.x <= i) H[(long)threadIdx.x * ldh + i] = hc[threadIdx.x];
+  } else if (threadIdx.x == 0) {
+    rotate_column(H + i, ldh, cs, sn, i, hn, cs + i, sn + i, g, tol[0], done, kdone);
+  }
+  if (threadIdx.x == 0) H[(long)(i + 1) * ldh + i] = 0.0;
+}
+
+// r = b - ax (ax NULL: r = b) and the block's part of |r|^2
+__global__ __launch_bounds__(OT) void k_gmres_residual(const double* __restrict__ b, const double* ax, double* r, long n,
+                                                       long chunk, double* __restrict__ partial) {
+  __shared__ double red[OT / 64];
+  const long a = (long)blockIdx.x * chunk, z = std::min(n, a + chunk);
+  double sq = 0.0;
+  for (long e = a + threadIdx.x; e < z; e += OT) {
+    const double v = ax ? b[e] - ax[e] : b[e];
+    if (r) r[e] = v;
+    sq = fma(v, v, sq);
+  }
+  const double t = block_sum(sq, red);
+  if (threadIdx.x == 0) partial[blockIdx.x] = t;
+}
+
+// stat: |r|, |b|, tol = max(atol, rtol |b|), steps of the cycle.  out = |r| or |b| (of = 0, 1);
+// of = 0 also fills in the tolerance and the step count.
+__global__ __launch_bounds__(OT) void k_gmres_stat(const double* __restrict__ partial, int nblk, int of, double atol,
+                                                   double rtol, const int* __restrict__ kdone, double* stat) {
+  __shared__ double red[OT / 64];
+  double t = 0.0;
+  for (int k = threadIdx.x; k < nblk; k += OT) t += partial[k];
+  const double v = sqrt(block_sum(t, red));
+  if (threadIdx.x == 0) {
+    stat[of] = v;
+    if (of == 0) {
+      stat[2] = fmax(atol, rtol * stat[1]);
+      stat[3] = (double)*kdone;
+    }
+  }
+}
+
+// Start of a cycle from r, |r| in stat[0]: V_0 = r / |r|, g = (|r|, 0, ...), the flags
+__global__ __launch_bounds__(OT) void k_gmres_begin(const double* __restrict__ r, const double* __restrict__ stat,
+                                                    double* __restrict__ V0, long n, int m, double* __restrict__ g,
+                                                    double* __restrict__ tol, int* done, int* kdone) {
+  const double beta = stat[0];
+  if (beta != 0.0)
+    for (long e = (long)blockIdx.x * OT + threadIdx.x; e < n; e += (long)gridDim.x * OT) V0[e] = r[e] / beta;
+  if (blockIdx.x != 0) return;
+  for (int k = threadIdx.x; k <= m; k += OT) g[k] = k == 0 ? beta : 0.0;
+  if (threadIdx.x == 0) {
+    tol[0] = stat[2];
+    *done = beta < stat[2] ? 1 : 0;
+    *kdone = beta < stat[2] ? 0 : m;
+  }
+}
+
+// x += V y, R y = g over the k = *kdone steps of the cycle.  Every workgroup solves for y itself,
+// column by column (64 rows at a time in flight), from an LDS copy of R up to order 64.
+__global__ __launch_bounds__(OT) void k_gmres_solution(const double* __restrict__ V, long ldv,
+                                                       const double* __restrict__ H, int ldh,
+                                                       const double* __restrict__ g, const int* __restrict__ kdone,
+                                                       double* __restrict__ x, long n, int kmax) {
+  extern __shared__ double y[];                      // m, then R up to order 64
+  double* R = y + kmax;
+  const int k = *kdone;
+  const bool lds = kmax <= 64;
+  for (int j = threadIdx.x; j < k; j += OT) y[j] = g[j];
+  if (lds)
+    for (int e = threadIdx.x; e < k * k; e += OT) R[e] = H[(long)(e / k) * ldh + e % k];
+  __syncthreads();
+  for (int r = k - 1; r >= 0; --r) {
+    const double yr = y[r] / (lds ? R[r * k + r] : H[(long)r * ldh + r]);
+    __syncthreads();
+    for (int j = threadIdx.x; j <= r; j += OT)
+      y[j] = j == r ? yr : y[j] - (lds ? R[j * k + r] : H[(long)j * ldh + r]) * yr;
+    __syncthreads();
+  }
+  for (long e = (long)blockIdx.x * OT + threadIdx.x; e < n; e += (long)gridDim.x * OT) {
+    double s = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < k; ++j) s = fma(y[j], V[(long)j * ldv + e], s);
+    x[e] += s;
+  }
+}
+
+int orth_blocks(long n, long per) { return (int)std::max<long>(1, std::min<long>(256, (n + per - 1) / per)); }
+
 int grid_for(long n) { return (int)std::min<long>((n + NT - 1) / NT, 8192); }
 
 // bin[x] = argmin_i |E[x] - Ev[i]| (first minimum), the preconditioner membership of
@@ -269,6 +537,60 @@ int bz_vt_axpy(const double* V, long ldv, int nv, const double* coef, int cstrid
 int bz_scale_inv(const double* x, const double* s, double* y, long n, hipStream_t stream) {
   if (n < 1 || !x || !s || !y) return BZ_EINVAL;
   hipLaunchKernelGGL(k_scale_inv, dim3(grid_for(n)), dim3(NT), 0, stream, x, s, y, n);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
+// partial: (m + 1) * 256 doubles.  The last 256 hold |w|^2.
+int bz_gmres_orthogonalise(double* V, long ldv, int m, int i, double* w, long n, int passes, double* partial, double* H,
+                           int ldh, double* cs, double* sn, double* g, const double* tol, int* done, int* kdone,
+                           hipStream_t stream) {
+  if (n < 1 || ldv < n || m < 1 || i < 0 || i >= m || passes < 1 || ldh <= i || !V || !w || !partial || !H || !cs ||
+      !sn || !g || !tol || !done || !kdone)
+    return BZ_EINVAL;
+  if ((i + OJ) / OJ > 65535) return BZ_EINVAL;
+  const int nblk = orth_blocks(n, 2 * OT);
+  const long chunk = (n + nblk - 1) / nblk;
+  double* np = partial + (long)m * 256;
+  for (int p = 0; p < passes; ++p) {
+    hipLaunchKernelGGL(k_orth_dots, dim3(nblk, (i + OJ) / OJ), dim3(OT), 0, stream, V, ldv, i + 1, w, n, chunk, partial,
+                       done);
+    BZ_LAUNCH_CHECK();
+    hipLaunchKernelGGL(k_orth_update, dim3(nblk), dim3(OT), 0, stream, V, ldv, i + 1, partial, nblk, w, n, chunk, H, ldh,
+                       i, p > 0 ? 1 : 0, p + 1 == passes ? np : nullptr, done);
+    BZ_LAUNCH_CHECK();
+  }
+  hipLaunchKernelGGL(k_orth_finish, dim3(orth_blocks(n, OT) * 2), dim3(OT), 0, stream, np, nblk, w,
+                     V + (long)(i + 1) * ldv, n, H, ldh, i, cs, sn, g, tol, done, kdone);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
+int bz_gmres_norm(const double* b, const double* ax, double* r, long n, double* partial, int of, double atol, double rtol,
+                  const int* kdone, double* stat, hipStream_t stream) {
+  if (n < 1 || !b || !partial || !kdone || !stat || of < 0 || of > 1) return BZ_EINVAL;
+  const int nblk = orth_blocks(n, 2 * OT);
+  hipLaunchKernelGGL(k_gmres_residual, dim3(nblk), dim3(OT), 0, stream, b, ax, r, n, (n + nblk - 1) / nblk, partial);
+  BZ_LAUNCH_CHECK();
+  hipLaunchKernelGGL(k_gmres_stat, dim3(1), dim3(OT), 0, stream, partial, nblk, of, atol, rtol, kdone, stat);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
+int bz_gmres_begin(const double* r, const double* stat, double* V0, long n, int m, double* g, double* tol, int* done,
+                   int* kdone, hipStream_t stream) {
+  if (n < 1 || m < 1 || !r || !stat || !V0 || !g || !tol || !done || !kdone) return BZ_EINVAL;
+  hipLaunchKernelGGL(k_gmres_begin, dim3(orth_blocks(n, OT) * 2), dim3(OT), 0, stream, r, stat, V0, n, m, g, tol, done,
+                     kdone);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
+int bz_gmres_solution(const double* V, long ldv, int m, const double* H, int ldh, const double* g, const int* kdone,
+                      double* x, long n, hipStream_t stream) {
+  if (n < 1 || ldv < n || m < 1 || m > 8000 || ldh < m || !V || !H || !g || !kdone || !x) return BZ_EINVAL;
+  hipLaunchKernelGGL(k_gmres_solution, dim3(orth_blocks(n, OT) * 2), dim3(OT),
+                     (size_t)(m <= 64 ? m + m * m : m) * sizeof(double), stream, V, ldv, H, ldh, g, kdone, x, n, m);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }

@@ -134,67 +134,37 @@ class capture_guard:
         return False
 
 
-class DeviceGMRES:
-    """Restarted, right-preconditioned GMRES with the whole Arnoldi step on the device, for an
-    operator and a preconditioner given as launchers `matvec(src, dst)` and
-    `precond(src, dst)` (device addresses of flat float64 vectors of length n; each writes
-    dst only).
+class ArnoldiCycle:
+    """The device state of a restarted GMRES cycle and its vector operations (bz_krylov.hip):
+    basis, Hessenberg column rotation, residual estimate, stop flag.  A subclass supplies
+    `product(src, out, done)`: t = P src and out = A t (device addresses; nothing when the device
+    flag `done` is set).  After the first cycle the steps are replayed from HIP graphs of `chunk`
+    steps; the host reads the stop flag between them.  Steps past convergence are no-ops."""
 
-    The method of utils.gmres_pcr (utils.py:1172-1268: right preconditioning, restart,
-    tol = max(atol, rtol |b|)) with the host out of the inner loop: the stop test of a step
-    is the least-squares residual |g_(i+1)| of the Givens-rotated Hessenberg system (the
-    true residual in exact arithmetic, bz_gmres_givens), and the true residual is evaluated
-    once per cycle, at its end, before the solution is accepted.  Per step: preconditioner,
-    operator, classical Gram-Schmidt (bz_multi_dot, bz_vt_axpy; two passes by default, one
-    with gs_passes=1), the norm and scaling, one rotation.  After the first cycle the steps are replayed from HIP graphs of `chunk`
-    steps; the host reads the device stop flag between graphs.  The launchers' scalar
-    arguments and buffers are captured with the graphs, so they must stay the same between
-    solves (inputs are copied into fixed buffers)."""
-
-    def __init__(self, n, restart, dev, matvec, precond, chunk=4, use_graph=True, gs_passes=2):
+    def __init__(self, n, restart, dev, chunk, gs_passes, use_graph=True):
         f64, i32 = torch.float64, torch.int32
         self.n, self.m, self.chunk = int(n), int(restart), int(chunk)
         self.gs_passes = int(gs_passes)                             # classical Gram-Schmidt passes
-        self.matvec, self.precond = matvec, precond
         self.use_graph = use_graph
-        self.nblk = max(1, min(1024, (self.n + 4095) // 4096))
         m = self.m
-        # zero-filled: rows past the last step of a cycle enter the solution update with zero
-        # coefficients, which must not meet uninitialised NaN patterns
         self.V = torch.zeros((m + 1, self.n), dtype=f64, device=dev)
         self.H = torch.zeros((m + 2, m + 1), dtype=f64, device=dev)
         self.ldh = m + 1
-        self.partial = torch.empty(((m + 1) * self.nblk,), dtype=f64, device=dev)
-        self.h = torch.zeros(m + 2, dtype=f64, device=dev)
+        self.partial = torch.empty(((m + 1) * 256,), dtype=f64, device=dev)
         self.cs = torch.zeros(m + 1, dtype=f64, device=dev)
         self.sn = torch.zeros(m + 1, dtype=f64, device=dev)
         self.g = torch.zeros(m + 2, dtype=f64, device=dev)
-        self.y = torch.zeros(m + 1, dtype=f64, device=dev)
         self.tol = torch.zeros(1, dtype=f64, device=dev)
-        self.scal = torch.zeros(4, dtype=f64, device=dev)
+        self.stat = torch.zeros(4, dtype=f64, device=dev)           # |r|, |b|, tolerance, steps
         self.flags = torch.zeros(2, dtype=i32, device=dev)          # done, steps of the cycle
-        self.w = torch.empty(self.n, dtype=f64, device=dev)
-        self.t = torch.empty(self.n, dtype=f64, device=dev)
-        self.x = torch.empty(self.n, dtype=f64, device=dev)
-        self.b = torch.empty(self.n, dtype=f64, device=dev)
-        self.r = torch.empty(self.n, dtype=f64, device=dev)
+        self.w, self.t, self.x, self.b, self.r = (torch.empty(self.n, dtype=f64, device=dev) for _ in range(5))
         self.graphs = None
 
-    def _dot(self, V, nv, u, out, ostride=1, accumulate=0, take_sqrt=0, out2=None):
-        _lib.call("bz_multi_dot", _at(V), self.n, nv, _at(u), self.n, self.partial, self.nblk, out, ostride,
-                  accumulate, take_sqrt, out2)
-
     def _step(self, i):
-        n, ldh = self.n, self.ldh
-        self.precond(_at(self.V, i * n), _at(self.t))
-        self.matvec(_at(self.t), _at(self.w))
-        for rep in range(self.gs_passes):
-            self._dot(self.V, i + 1, self.w, _at(self.H, i), ostride=ldh, accumulate=rep, out2=self.h)
-            _lib.call("bz_vt_axpy", _at(self.V), n, i + 1, self.h, 1, -1.0, self.w, self.w, n)
-        self._dot(self.w, 1, self.w, _at(self.H, (i + 1) * ldh + i), take_sqrt=1)
-        _lib.call("bz_scale_inv", self.w, _at(self.H, (i + 1) * ldh + i), _at(self.V, (i + 1) * n), n)
-        _lib.call("bz_gmres_givens", self.H, ldh, i, self.cs, self.sn, self.g, self.tol, _ptr(self.flags, 0),
-                  _ptr(self.flags, 1))
+        done, kdone = _ptr(self.flags, 0), _ptr(self.flags, 1)
+        self.product(_at(self.V, i * self.n), _at(self.w), done)
+        _lib.call("bz_gmres_orthogonalise", self.V, self.n, self.m, i, self.w, self.n, self.gs_passes, self.partial,
+                  self.H, self.ldh, self.cs, self.sn, self.g, self.tol, done, kdone)
 
     def _capture(self):
         with capture_guard():
@@ -206,34 +176,41 @@ class DeviceGMRES:
                         self._step(i)
                 self.graphs.append(gr)
 
-    def _residual(self, out_scal):
-        """r = b - A P x, |r| into scal[out_scal]; leaves P x in t."""
-        self.precond(_at(self.x), _at(self.t))
-        self.matvec(_at(self.t), _at(self.r))
-        torch.sub(self.b, self.r, out=self.r)
-        self._dot(self.r, 1, self.r, _at(self.scal, out_scal), take_sqrt=1)
+    def _norm(self, of, b, ax, r, atol=0.0, rtol=0.0):
+        _lib.call("bz_gmres_norm", b, ax, r, self.n, self.partial, of, float(atol), float(rtol), _ptr(self.flags, 1),
+                  self.stat)
 
-    def solve(self, b, atol, rtol, max_cycles, x0=None, callback=None):
-        """Returns (P x, total steps); raises RuntimeError after max_cycles cycles."""
-        self.b.copy_(b.reshape(-1))
-        if x0 is None:
-            self.x.zero_()
+    def _residual(self, atol, rtol):
+        """r = b - A P x with its norm; leaves P x in t."""
+        self.product(_at(self.x), _at(self.r), None)
+        self._norm(0, self.b, self.r, self.r, atol, rtol)
+
+    def _solution(self):
+        """x += V y over the steps of the cycle."""
+        if self.m > 8000:                                           # more rows of y than fit the kernel's LDS
+            y = torch.zeros(self.m, dtype=torch.float64, device=self.x.device)
+            _lib.call("bz_gmres_back_solve", self.H, self.ldh, self.g, _ptr(self.flags, 1), y, self.m)
+            _lib.call("bz_vt_axpy", self.V, self.n, self.m, y, 1, 1.0, self.x, self.x, self.n)
+            return
+        _lib.call("bz_gmres_solution", self.V, self.n, self.m, self.H, self.ldh, self.g, _ptr(self.flags, 1), self.x,
+                  self.n)
+
+    def cycles(self, atol, rtol, max_cycles, zero_start, callback=None):
+        """Cycles from x (zero_start: x = 0) for the right-hand side b, until the true residual
+        is below tol = max(atol, rtol |b|).  Returns (converged, total steps); P x is in t."""
+        self._norm(1, self.b, None, None)
+        if zero_start:
+            self.t.zero_()
+            self._norm(0, self.b, None, self.r, atol, rtol)
         else:
-            self.x.copy_(x0.reshape(-1))
-        self._dot(self.b, 1, self.b, _at(self.scal, 1), take_sqrt=1)
-        self._residual(0)                                  # r = b - A P x0, |r| -> scal[0]
+            self._residual(atol, rtol)
         iters = 0
-        for cyc in range(max_cycles):
-            # r and |r| are those of the current x: computed above, or at the end of the
-            # previous cycle (where the host found |r| >= tol), so only the first cycle reads
-            # the start test back
-            self.H.zero_()
-            _lib.call("bz_gmres_cycle_start", self.scal, float(atol), float(rtol), self.m, self.g, self.tol,
+        for _ in range(max_cycles):
+            # r and its norm are those of the current x: computed above, or at the end of the
+            # previous cycle.  When |r| is below the tolerance at the start the cycle is empty.
+            _lib.call("bz_gmres_begin", self.r, self.stat, self.V, self.n, self.m, self.g, self.tol,
                       _ptr(self.flags, 0), _ptr(self.flags, 1))
-            if cyc == 0 and int(self.flags[0].item()):
-                return self.t.clone(), iters
-            _lib.call("bz_scale_inv", self.r, self.scal, _at(self.V, 0), self.n)
-            if self.graphs is None or not self.use_graph:
+            if self.graphs is None:
                 # eager cycle (the first one loads and runs every kernel once), then capture
                 for i in range(self.m):
                     self._step(i)
@@ -246,16 +223,49 @@ class DeviceGMRES:
                     gr.replay()
                     if int(self.flags[0].item()):
                         break
-            _lib.call("bz_gmres_back_solve", self.H, self.ldh, self.g, _ptr(self.flags, 1), self.y, self.m)
-            _lib.call("bz_vt_axpy", _at(self.V), self.n, self.m, self.y, 1, 1.0, self.x, self.x, self.n)
-            self._residual(2)
+            self._solution()
+            self._residual(atol, rtol)
             # one read-back per cycle: the true residual, |b|, the tolerance and the step count
-            rn, bn, tol, k = torch.stack([self.scal[2], self.scal[1], self.tol[0],
-                                          self.flags[1].to(torch.float64)]).tolist()
+            rn, bn, tol, k = self.stat.tolist()
             iters += int(k)
             if callback is not None:
                 callback(rn / bn if bn > 0 else 0.0)
             if rn < tol:
-                return self.t.clone(), iters
-            self.scal[0].copy_(self.scal[2])              # the next cycle starts from this r
-        raise RuntimeError(f"GMRES did not converge in {max_cycles} cycles of {self.m}")
+                return True, iters
+        return False, iters
+
+
+class DeviceGMRES(ArnoldiCycle):
+    """Restarted, right-preconditioned GMRES with the whole Arnoldi step on the device, for an
+    operator and a preconditioner given as launchers `matvec(src, dst, done)` and
+    `precond(src, dst, done)` (device addresses of flat float64 vectors of length n; each writes
+    dst only, and nothing when the device flag `done`, if not None, is set).
+
+    The method of utils.gmres_pcr (utils.py:1172-1268: right preconditioning, restart,
+    tol = max(atol, rtol |b|)) with the host out of the inner loop: the stop test of a step
+    is the least-squares residual |g_(i+1)| of the Givens-rotated Hessenberg system (the
+    true residual in exact arithmetic), and the true residual is evaluated once per cycle, at its
+    end, before the solution is accepted.  Per step: preconditioner, operator and
+    bz_gmres_orthogonalise (classical Gram-Schmidt, two passes by default, one with gs_passes=1).
+    The launchers' scalar arguments and buffers are captured with the graphs, so they must stay
+    the same between solves (inputs are copied into fixed buffers)."""
+
+    def __init__(self, n, restart, dev, matvec, precond, chunk=4, use_graph=True, gs_passes=2):
+        super().__init__(n, restart, dev, chunk, gs_passes, use_graph)
+        self.matvec, self.precond = matvec, precond
+
+    def product(self, src, out, done):
+        self.precond(src, _at(self.t), done)
+        self.matvec(_at(self.t), out, done)
+
+    def solve(self, b, atol, rtol, max_cycles, x0=None, callback=None):
+        """Returns (P x, total steps); raises RuntimeError after max_cycles cycles."""
+        self.b.copy_(b.reshape(-1))
+        if x0 is None:
+            self.x.zero_()
+        else:
+            self.x.copy_(x0.reshape(-1))
+        converged, iters = self.cycles(atol, rtol, max_cycles, x0 is None, callback)
+        if not converged:
+            raise RuntimeError(f"GMRES did not converge in {max_cycles} cycles of {self.m}")
+        return self.t.clone(), iters

@@ -337,6 +337,30 @@ int bz_scale_inv(const double* x, const double* s, double* y, long n, hipStream_
  * xp.linalg.lstsq call of utils.gmres_pcr (utils.py:1228). */
 int bz_hess_lstsq(const double* H, int ldh, int m, const double* beta, double* work, double* y, hipStream_t stream);
 
+/* The vector part of Arnoldi step i (0 <= i < m) of a restart cycle: w (n) = A M^-1 V_i is
+ * orthogonalised against V_0..V_i by `passes` classical Gram-Schmidt passes, V_(i+1) = w / |w|,
+ * column i of H (row stride ldh) is rotated into the triangular factor and g, cs, sn are extended
+ * as by bz_gmres_givens; done, kdone as there.  Three launches (two more per further pass), none of
+ * which does anything once *done is set.  partial: (m + 1) * 256 doubles. */
+int bz_gmres_orthogonalise(double* V, long ldv, int m, int i, double* w, long n, int passes, double* partial, double* H,
+                           int ldh, double* cs, double* sn, double* g, const double* tol, int* done, int* kdone,
+                           hipStream_t stream);
+
+/* r = b - ax (r = b for ax NULL; r may be NULL or ax) and its norm: stat[of], of = 0 for a residual
+ * (then also stat[2] = max(atol, rtol stat[1]) and stat[3] = *kdone), of = 1 for |b|.
+ * partial: 256 doubles. */
+int bz_gmres_norm(const double* b, const double* ax, double* r, long n, double* partial, int of, double atol, double rtol,
+                  const int* kdone, double* stat, hipStream_t stream);
+
+/* Start of a cycle of m steps from r: V0 = r / stat[0], g = (stat[0], 0, ...), tol = stat[2],
+ * done = |r| < tol, kdone = m (0 when done). */
+int bz_gmres_begin(const double* r, const double* stat, double* V0, long n, int m, double* g, double* tol, int* done,
+                   int* kdone, hipStream_t stream);
+
+/* x += V y with R y = g over the *kdone (<= m <= 8000) steps of the cycle. */
+int bz_gmres_solution(const double* V, long ldv, int m, const double* H, int ldh, const double* g, const int* kdone,
+                      double* x, long n, hipStream_t stream);
+
 /* GMRES over B independent systems of size n (one per 0D instance), basis
  * V[(j*B + b)*n + e], j = 0..m (m <= 64).  Arnoldi step i: w (B, n) = A M^-1 V_i; classical
  * Gram-Schmidt twice, V_{i+1}, the Givens-rotated column into R[b][i*m + 0..i], cs, sn
@@ -571,6 +595,12 @@ int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
  * the dense PmatC or SpSM. */
 int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
                           hipStream_t stream);
+
+/* The same two products, no-ops when the device flag *done is set (done may be NULL). */
+int bz_fvm_rhs_mvec_until(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y, const int* done,
+                          hipStream_t stream);
+int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
+                                const int* done, hipStream_t stream);
 
 #ifdef __cplusplus
 }

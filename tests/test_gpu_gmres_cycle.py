@@ -1,0 +1,102 @@
+"""The three-launch Arnoldi step of bz_krylov.hip: block and chunk edges of the reductions, more than
+64 steps (the triangular solve past its LDS copy), more than 256 basis vectors, restarts, a start
+that is already converged, replays of the captured graphs.
+
+The solver stops on its own true residual |b - A P x| < tol, evaluated on the device; the same
+residual from the returned vector on the host differs by the rounding of the product, n eps |A| |x|,
+far below the tolerances of 1e-8 |b| asked for here, so the host's must be below 1.01 tol."""
+import numpy as np
+import pytest
+import torch
+
+from boltzmann_amd import _lib
+from boltzmann_amd.krylov import DeviceGMRES
+
+pytestmark = pytest.mark.gpu
+
+
+def _solver(n, restart, seed, spread, **kw):
+    g = torch.Generator(device="cuda").manual_seed(seed)
+    A = torch.randn((n, n), dtype=torch.float64, device="cuda", generator=g) * (spread / n ** 0.5)
+    A += torch.eye(n, dtype=torch.float64, device="cuda")
+    b = torch.randn(n, dtype=torch.float64, device="cuda", generator=g)
+    scale = torch.full((n,), 0.5, dtype=torch.float64, device="cuda")
+
+    def tensor(ptr):
+        for t in (s.V.view(-1), s.t, s.x, s.w, s.r):
+            off = (ptr.value - t.data_ptr()) // 8
+            if 0 <= off < t.numel():
+                return t[off:off + n]
+        raise AssertionError("unknown vector")
+
+    def matvec(src, dst, done):
+        torch.mv(A, tensor(src), out=tensor(dst))
+
+    def precond(src, dst, done):
+        torch.mul(tensor(src), scale, out=tensor(dst))
+
+    s = DeviceGMRES(n, restart, torch.device("cuda"), matvec, precond, use_graph=False, **kw)
+    return s, A, b
+
+
+@pytest.mark.parametrize("n,restart,spread,gs_passes", [(1, 1, 0.0, 1), (2, 2, 0.1, 2), (511, 20, 0.3, 1),
+                                                        (513, 7, 0.4, 2), (1025, 90, 0.85, 1), (700, 300, 0.99, 2)])
+def test_solution_meets_its_tolerance(n, restart, spread, gs_passes):
+    s, A, b = _solver(n, restart, n, spread, gs_passes=gs_passes)
+    x, k = s.solve(b, 0.0, 1e-8, 200)
+    assert float(torch.linalg.vector_norm(A.cpu() @ x.cpu() - b.cpu())) < 1.01e-8 * float(torch.linalg.vector_norm(b))
+    assert 1 <= k
+    again, k2 = s.solve(b, 0.0, 1e-8, 200, x0=2.0 * x)         # P x0 = x: nothing left to do
+    assert k2 == 0 and torch.equal(again, x * 1.0)
+
+
+@pytest.mark.parametrize("n,i", [(1, 0), (1023, 3), (1025, 4), (300000, 5), (600, 259)])
+def test_orthogonalise_against_the_host(n, i):
+    """One step against the same operations in NumPy; errors of a sum of n products of order one
+    against unit vectors are below n eps, the rotation adds a few eps."""
+    rng = np.random.default_rng(n)
+    m = i + 1
+    V = np.zeros((m + 1, n))
+    q, _ = np.linalg.qr(rng.normal(size=(n, min(n, m)))) if n < 5000 else (None, None)
+    if q is None:
+        V[:m] = rng.normal(size=(m, n))
+        V[:m] /= np.linalg.norm(V[:m], axis=1)[:, None]
+    else:
+        V[:q.shape[1]] = q.T
+    w = rng.normal(size=n) / np.sqrt(n)
+    d = lambda a, t=torch.float64: torch.tensor(a, dtype=t, device="cuda")
+    Vd, wd, H = d(V), d(w), d(np.zeros((m + 2, m + 1)))
+    th = rng.uniform(0, 6, m + 1)
+    cs, sn, g = d(np.cos(th)), d(np.sin(th)), d(np.append(rng.normal(size=i + 1), np.zeros(m + 1 - i)))
+    g0 = float(g[i])
+    tol, flags = d(np.zeros(1)), d(np.zeros(2), torch.int32)
+    part = torch.empty((m + 1) * 256, dtype=torch.float64, device="cuda")
+    ptr = lambda k: __import__("ctypes").c_void_p(flags.data_ptr() + 4 * k)
+    _lib.call("bz_gmres_orthogonalise", Vd, n, m, i, wd, n, 1, part, H, m + 1, cs, sn, g, tol, ptr(0), ptr(1))
+    h = V[:i + 1] @ w
+    r = w - h @ V[:i + 1]
+    hn = np.linalg.norm(r)
+    eps = 4 * max(n, 64) * np.finfo(float).eps
+    assert np.abs(wd.cpu().numpy() - r).max() <= eps
+    if n > 1:
+        assert np.abs(Vd[i + 1].cpu().numpy() - r / hn).max() <= eps / hn
+    c, s_ = np.cos(th), np.sin(th)
+    col, a = h.copy(), h[0]
+    full = np.append(h, hn)
+    for k in range(i):
+        col[k], a = c[k] * a + s_[k] * full[k + 1], -s_[k] * a + c[k] * full[k + 1]
+    col[i] = np.hypot(a, hn)
+    assert np.abs(H[:i + 1, i].cpu().numpy() - col).max() <= (i + 4) * eps
+    assert abs(float(g[i + 1]) - (-hn / col[i] * g0)) <= (i + 4) * eps * abs(g0) / col[i]
+
+
+def test_nothing_moves_once_done():
+    n, m = 3000, 4
+    g = torch.Generator(device="cuda").manual_seed(1)
+    t = lambda *s: torch.randn(s, dtype=torch.float64, device="cuda", generator=g)
+    V, w, H, cs, sn, gg, tol = t(m + 1, n), t(n), t(m + 2, m + 1), t(m + 1), t(m + 1), t(m + 2), t(1)
+    flags = torch.tensor([1, 2], dtype=torch.int32, device="cuda")
+    before = [x.clone() for x in (V, w, H, cs, sn, gg, flags)]
+    ptr = lambda k: __import__("ctypes").c_void_p(flags.data_ptr() + 4 * k)
+    _lib.call("bz_gmres_orthogonalise", V, n, m, 2, w, n, 2, t((m + 1) * 256), H, m + 1, cs, sn, gg, tol, ptr(0), ptr(1))
+    assert all(torch.equal(x, y) for x, y in zip((V, w, H, cs, sn, gg, flags), before))
