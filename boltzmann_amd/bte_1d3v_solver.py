@@ -238,6 +238,14 @@ class gmres_counter:
         self.residuals.append(float(rk))
 
 
+class _StepGMRES(DeviceGMRES):
+    """DeviceGMRES with the preconditioner and the step operator in one call, which shares the
+    isotropic moment of t = P src between them: launch(src, t, out, done)."""
+
+    def product(self, src, out, done):
+        self.launch(src, self.t, out, done)
+
+
 class bte_1d3v:
     def __init__(self, args):
         self.params = p = args.params if getattr(args, "params", None) is not None else params(args.par_file)
@@ -459,10 +467,10 @@ class bte_1d3v:
         key = (float(dt), float(alpha))
         if self._dg is None or self._dg_key != key:
             op, E = self._op, self._Ebuf
-            mv = lambda src, dst, done: _lib.call("bz_fvm_rhs_mvec_until", op, E, key[0], src, dst, done)
-            pc = lambda src, dst, done: _lib.call("bz_fvm_precond_xvtvrc_until", op, E, key[1] * key[0], src, dst, done)
-            self._dg = DeviceGMRES(self.dof_v * self.dof_x, self.params.gmres_rsrt, self.dev, mv, pc,
-                                   gs_passes=self.gs_passes)
+            self._dg = _StepGMRES(self.dof_v * self.dof_x, self.params.gmres_rsrt, self.dev, None, None,
+                                  gs_passes=self.gs_passes)
+            self._dg.launch = lambda src, t, out, done: _lib.call("bz_fvm_step_product", op, E, key[0], key[1] * key[0],
+                                                                  src, t, out, done)
             self._dg_key = key
         return self._dg
 

@@ -102,103 +102,107 @@ __global__ __launch_bounds__(256) void k_fvm_matvec(BzFvm1d3v op, const double* 
   y[e] = out;
 }
 
-// The step operator for fixed stencil widths (the common ones): every neighbour load is issued
-// unconditionally from a clamped address and weighted by zero where the stencil has no entry,
-// so all loads of an element go out together instead of one loop iteration at a time; the
-// gain row is read the same way, GMAX entries at once.  Same sums, in the same order, as
-// k_fvm_matvec (the zero terms add exactly nothing).
-template <int NX, int NVR, int NVT, int GMAX>
-__global__ __launch_bounds__(256) void k_fvm_matvec_w(BzFvm1d3v op, const double* __restrict__ E, double dt,
+// The step operator for fixed stencil widths (the common ones), TB ordinates of one (r, x) per
+// thread: the element alone takes 24 vector loads (8 state values, 6 gains, 10 stencil weights);
+// with TB together the gains, the x weights and most angular neighbours are shared and the radial
+// and angular weights are uniform (scalar loads, both directions, chosen per lane), 8 vector loads
+// an element.  Every neighbour load is issued unconditionally from a clamped address and weighted
+// by zero where the stencil has no entry.  Same sums, in the same order, as k_fvm_matvec (the zero
+// terms add exactly nothing).  Measured at 671 x 16 x 100: MVFIG.
+template <int NX, int NVR, int NVT, int GMAX, int TB>
+__global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                       const double* __restrict__ x, const double* __restrict__ s,
                                                       double* __restrict__ y, const int* __restrict__ done) {
   if (done && *done) return;
   const int Nr = op.Nr, Nvt = op.Nvt, Nx = op.Nx;
-  // Workgroups of one state row (r, t) each, threads over x: the row indices are workgroup-
-  // uniform (no per-thread division).  Workgroups are dealt to the 8 XCDs in turn (workgroup
-  // b to XCD b % 8); the grid is a multiple of 8 and XCD k takes the k-th eighth of the rows,
-  // so the radial neighbours (Nvt rows away) of a row are read through the same L2.
+  // Workgroups of one radius and one group of ordinates each, threads over x: the row indices are
+  // workgroup-uniform.  Workgroups are dealt to the 8 XCDs in turn (workgroup b to XCD b % 8); the
+  // grid is a multiple of 8 and XCD k takes the k-th eighth of the rows, so the radial neighbours
+  // of a row are read through the same L2.
   const int bx = (Nx + blockDim.x - 1) / blockDim.x;            // workgroups per row
+  const int ntg = (Nvt + TB - 1) / TB;
   const unsigned per = gridDim.x >> 3;
   const unsigned lb = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   const int row = (int)(lb / (unsigned)bx);
   const int ix = (int)(lb - (unsigned)row * bx) * blockDim.x + threadIdx.x;
-  if (row >= Nr * Nvt || ix >= Nx) return;
-  const int r = row / Nvt, t = row - r * Nvt;
-  const long e = (long)row * Nx + ix;
+  if (row >= Nr * ntg || ix >= Nx) return;
+  const int r = row / ntg, t0 = (row - r * ntg) * TB;
   const int mp = Nvt / 2;
-  const double cs = op.cos_vt[t];
-  const bool low = t >= mp;
-  const double cx = op.dt_x * op.adx[r] * cs;
-  const double* DX = low ? op.dxL : op.dxR;
-  const double x0 = x[e];
-  double xv[NX], dx[NX];
+  const long rs = (long)Nvt * Nx;
+  const double* xr0 = x + (long)r * rs + ix;
+  const double Ex = E[ix];
+  const bool ep = Ex >= 0;
+  // the ordinates of the group and NVT - 1 on either side
+  constexpr int HC = NVT - 1, NC = TB + 2 * HC;
+  double xc[NC], xn[TB][NX], xr[TB][NVR];
+#pragma unroll
+  for (int k = 0; k < NC; ++k) xc[k] = xr0[(long)min(max(t0 - HC + k, 0), Nvt - 1) * Nx];
+#pragma unroll
+  for (int i = 0; i < TB; ++i) {
+    const int t = min(t0 + i, Nvt - 1);
+    const bool low = t >= mp, up = (ep == low);
+#pragma unroll
+    for (int k = 1; k < NX; ++k) xn[i][k] = xr0[(long)t * Nx + min(max(low ? ix - k : ix + k, 0), Nx - 1) - ix];
+#pragma unroll
+    for (int d = 1; d < NVR; ++d) xr[i][d] = xr0[(long)t * Nx + (long)(min(max(up ? r + d : r - d, 0), Nr - 1) - r) * rs];
+  }
+  double dxl[NX], dxr[NX];
 #pragma unroll
   for (int k = 0; k < NX; ++k) {
-    const int j = min(max(low ? ix - k : ix + k, 0), Nx - 1);
-    xv[k] = k == 0 ? x0 : x[e + (j - ix)];
-    dx[k] = DX[k * Nx + ix];
+    dxl[k] = op.dxL[k * Nx + ix];
+    dxr[k] = op.dxR[k * Nx + ix];
   }
-  double yx = 0.0;
+  const int q0 = op.g_ptr[r], q1 = op.g_ptr[r + 1];
+  const int qmax = max(op.g_ptr[Nr] - 1, 0);
+  double gv[GMAX], gs[GMAX];
 #pragma unroll
-  for (int k = 0; k < NX; ++k) {
-    const int j = low ? ix - k : ix + k;
-    const double d = cx * dx[k] + (k == 0 ? 1.0 : 0.0);
-    yx += (j >= 0 && j < Nx) ? d * xv[k] : 0.0;
+  for (int k = 0; k < GMAX; ++k) {
+    const int q = min(q0 + k, qmax);
+    gv[k] = op.g_val[q];
+    gs[k] = s[(size_t)op.g_col[q] * Nx + ix];
   }
-  const bool inflow = low ? (ix == 0) : (ix == Nx - 1);
-  double out = yx;
-  if (!inflow) {
-    const int q0 = op.g_ptr[r], q1 = op.g_ptr[r + 1];
-    const int qmax = max(op.g_ptr[Nr] - 1, 0);
-    double gv[GMAX], gs[GMAX];
+  double g = 0.0;
 #pragma unroll
-    for (int k = 0; k < GMAX; ++k) {
-      const int q = min(q0 + k, qmax);
-      gv[k] = op.g_val[q];
-      gs[k] = s[(size_t)op.g_col[q] * Nx + ix];
+  for (int k = 0; k < GMAX; ++k) g += (q0 + k < q1) ? gv[k] * gs[k] : 0.0;
+  for (int q = q0 + GMAX; q < q1; ++q) g += op.g_val[q] * s[(size_t)op.g_col[q] * Nx + ix];
+  const double loss = op.loss[r], vr = op.vr[r], adx = op.dt_x * op.adx[r];
+  double out[TB];
+#pragma unroll
+  for (int i = 0; i < TB; ++i) {
+    const int t = min(t0 + i, Nvt - 1);
+    const double cs = op.cos_vt[t];
+    const bool low = t >= mp, up = (ep == low);
+    const double x0 = xc[HC + i];
+    const double cx = adx * cs;
+    double yx = 0.0;
+#pragma unroll
+    for (int k = 0; k < NX; ++k) {
+      const int j = low ? ix - k : ix + k;
+      const double d = cx * (low ? dxl[k] : dxr[k]) + (k == 0 ? 1.0 : 0.0);
+      yx += (j >= 0 && j < Nx) ? d * (k == 0 ? x0 : xn[i][k]) : 0.0;
     }
-    double g = 0.0;
-#pragma unroll
-    for (int k = 0; k < GMAX; ++k) g += (q0 + k < q1) ? gv[k] * gs[k] : 0.0;
-    for (int q = q0 + GMAX; q < q1; ++q) g += op.g_val[q] * s[(size_t)op.g_col[q] * Nx + ix];
-    const double xc = x0;
-    const double cv = g - op.loss[r] * xc;
-    const double Ex = E[ix];
-    const bool ep = Ex >= 0;
-    const bool vr_up = (ep == low);
-    const double* Dr = vr_up ? op.dvrR : op.dvrL;
-    const long rs = (long)Nvt * Nx;
-    double xr[NVR], dr[NVR];
-#pragma unroll
-    for (int d = 0; d < NVR; ++d) {
-      const int j = min(max(vr_up ? r + d : r - d, 0), Nr - 1);
-      xr[d] = d == 0 ? x0 : x[e + (long)(j - r) * rs];
-      dr[d] = Dr[d * Nr + r];
-    }
+    const bool inflow = low ? (ix == 0) : (ix == Nx - 1);
+    const double cv = g - loss * x0;
     double ar = 0.0;
 #pragma unroll
     for (int d = 0; d < NVR; ++d) {
-      const int j = vr_up ? r + d : r - d;
-      ar += (j >= 0 && j < Nr) ? dr[d] * xr[d] : 0.0;
-    }
-    const double* Dt = ep ? op.dvtR : op.dvtL;
-    double xt[NVT], dtt[NVT];
-#pragma unroll
-    for (int d = 0; d < NVT; ++d) {
-      const int j = min(max(ep ? t + d : t - d, 0), Nvt - 1);
-      xt[d] = d == 0 ? x0 : x[e + (long)(j - t) * Nx];
-      dtt[d] = Dt[d * Nvt + t];
+      const int j = up ? r + d : r - d;
+      const double wr = up ? op.dvrR[d * Nr + r] : op.dvrL[d * Nr + r];
+      ar += (j >= 0 && j < Nr) ? wr * (d == 0 ? x0 : xr[i][d]) : 0.0;
     }
     double at = 0.0;
 #pragma unroll
     for (int d = 0; d < NVT; ++d) {
       const int j = ep ? t + d : t - d;
-      at += (j >= 0 && j < Nvt) ? dtt[d] * xt[d] : 0.0;
+      const double wt = ep ? op.dvtR[d * Nvt + t] : op.dvtL[d * Nvt + t];
+      at += (j >= 0 && j < Nvt) ? wt * (ep ? xc[HC + i + d] : xc[HC + i - d]) : 0.0;
     }
-    const double ae = cs * ar - (op.sin_vt[t] / op.vr[r]) * at;
-    out = yx - dt * (op.tau_n0np0 * cv + op.tau * (Ex * (op.eq * ae)));
+    const double ae = cs * ar - (op.sin_vt[t] / vr) * at;
+    out[i] = inflow ? yx : yx - dt * (op.tau_n0np0 * cv + op.tau * (Ex * (op.eq * ae)));
   }
-  y[e] = out;
+#pragma unroll
+  for (int i = 0; i < TB; ++i)
+    if (t0 + i < Nvt) y[(long)r * rs + (long)(t0 + i) * Nx + ix] = out[i];
 }
 
 // h = H s on the matrix cores: one workgroup of CC_WAVES wavefronts per 16 x 16 tile of h
@@ -598,6 +602,148 @@ __global__ __launch_bounds__(64) void k_fvm_x_scan(BzFvm1d3v op, double dt, cons
   }
 }
 
+// The angular sweep, the x sweep for two-point stencils and the isotropic moment of the result for
+// one radius, whose plane (Nvt x Nx, contiguous) stays in LDS from one load to one store: apart they
+// are three passes over the state, each of one dependent chain.  One thread per x point for the
+// angular sweep (SW_VT of k_fvm_sweep), one wavefront per ordinate for the x scan (k_fvm_x_scan).
+constexpr int PT = 256;
+
+template <int ND, int PER>
+__global__ __launch_bounds__(PT) void k_fvm_plane(BzFvm1d3v op, const double* __restrict__ E, double dt, double* y,
+                                                  double* __restrict__ s, const int* __restrict__ done) {
+  if (done && *done) return;
+  extern __shared__ double pl[];                      // the plane, then the band tables
+  const int Nvt = op.Nvt, Nx = op.Nx, r = blockIdx.x;
+  const int cells = Nvt * Nx;
+  double* tv = pl + cells;                            // angular: left to right, right to left
+  double* tx = tv + 2 * ND * Nvt;                     // x: the same
+  double* yr = y + (size_t)r * cells;
+  for (int e = threadIdx.x; e < cells; e += PT) pl[e] = yr[e];
+  for (int e = threadIdx.x; e < ND * Nvt; e += PT) {
+    tv[e] = op.vt_l2r[e];
+    tv[ND * Nvt + e] = op.vt_r2l[e];
+  }
+  for (int e = threadIdx.x; e < 2 * Nx; e += PT) {
+    tx[e] = op.x_l2r[e];
+    tx[2 * Nx + e] = op.x_r2l[e];
+  }
+  __syncthreads();
+  const double vr = op.vr[r];
+  for (int ix = threadIdx.x; ix < Nx; ix += PT) {
+    const double aE = op.eaE * E[ix];
+    const double av = aE / vr;
+    const bool fwd = -av >= 0;
+    const double dtav = dt * av;
+    const double* D = tv + (fwd ? 0 : ND * Nvt);
+    double z[ND > 1 ? ND - 1 : 1];
+#pragma unroll
+    for (int d = 0; d < (ND > 1 ? ND - 1 : 1); ++d) z[d] = 0.0;
+#pragma unroll 4
+    for (int p = 0; p < Nvt; ++p) {
+      const int c = fwd ? p : Nvt - 1 - p;
+      double dd[ND];
+#pragma unroll
+      for (int d = 0; d < ND; ++d) dd[d] = D[d * Nvt + (fwd ? max(c - d, 0) : min(c + d, Nvt - 1))];
+      double sv = 0.0;
+#pragma unroll
+      for (int d = ND - 1; d >= 1; --d) sv += dd[d] * z[d - 1];
+      const double rden = 1.0 / (1.0 + av * dt * dd[0]);   // off the recurrence
+      const double val = (pl[c * Nx + ix] - sv * dtav) * rden;
+#pragma unroll
+      for (int d = (ND > 1 ? ND - 2 : 0); d >= 1; --d) z[d] = z[d - 1];
+      z[0] = val;
+      pl[c * Nx + ix] = val;
+    }
+  }
+  __syncthreads();
+  // LN lines of a wavefront at a time, so that their scans overlap
+  constexpr int LN = PER <= 4 ? 4 : 2;
+  const int lane = threadIdx.x & 63;
+  const double ax = op.axvr[r];
+  for (int t0 = threadIdx.x >> 6; t0 < Nvt; t0 += LN * (PT / 64)) {
+    double al[LN][PER], be[LN][PER], A[LN], B[LN];
+    bool fw[LN];
+#pragma unroll
+    for (int l = 0; l < LN; ++l) {
+      const int t = min(t0 + l * (PT / 64), Nvt - 1);
+      const double* line = pl + t * Nx;
+      const double av = ax * op.cos_vt[t];
+      fw[l] = av >= 0;
+      const double* D = tx + (fw[l] ? 0 : 2 * Nx);
+      const double dtav = dt * av;
+      A[l] = 1.0;
+      B[l] = 0.0;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int p = lane * PER + i;
+        al[l][i] = 0.0;
+        be[l][i] = 1.0;                            // identity beyond the end
+        if (p < Nx) {
+          const int c = fw[l] ? p : Nx - 1 - p;
+          const double rden = 1.0 / (1.0 + dtav * D[c]);
+          al[l][i] = p == 0 ? 0.0 : line[c] * rden;
+          be[l][i] = p == 0 ? 0.0 : -dtav * D[Nx + (fw[l] ? c - 1 : c + 1)] * rden;
+        }
+        B[l] = fma(be[l][i], B[l], al[l][i]);
+        A[l] *= be[l][i];
+      }
+    }
+#pragma unroll
+    for (int off = 1; off < 64; off <<= 1) {
+      double Ap[LN], Bp[LN];
+#pragma unroll
+      for (int l = 0; l < LN; ++l) {
+        Ap[l] = __shfl_up(A[l], off, 64);
+        Bp[l] = __shfl_up(B[l], off, 64);
+      }
+#pragma unroll
+      for (int l = 0; l < LN; ++l)
+        if (lane >= off) {
+          B[l] = fma(A[l], Bp[l], B[l]);
+          A[l] *= Ap[l];
+        }
+    }
+#pragma unroll
+    for (int l = 0; l < LN; ++l) {
+      const int t = t0 + l * (PT / 64);
+      double v = __shfl_up(B[l], 1, 64);
+      if (lane == 0) v = 0.0;
+#pragma unroll
+      for (int i = 0; i < PER; ++i) {
+        const int p = lane * PER + i;
+        v = fma(be[l][i], v, al[l][i]);
+        if (p < Nx && t < Nvt) pl[t * Nx + (fw[l] ? p : Nx - 1 - p)] = v;
+      }
+    }
+  }
+  __syncthreads();
+  for (int e = threadIdx.x; e < cells; e += PT) yr[e] = pl[e];
+  for (int ix = threadIdx.x; ix < Nx; ix += PT) {
+    double acc = 0.0;
+    for (int t = 0; t < Nvt; ++t) acc += op.wq[t] * pl[t * Nx + ix];
+    s[(size_t)r * Nx + ix] = acc;
+  }
+}
+
+// Whether the plane of a radius takes k_fvm_plane: two-point x stencil with at most 8 points per
+// lane, one of the common angular stencils, and a plane that fits 64 KB of LDS with its tables.
+size_t plane_doubles(const BzFvm1d3v& op) {
+  return (size_t)op.Nvt * op.Nx + 2 * (size_t)op.nvt * op.Nvt + 4 * (size_t)op.Nx;
+}
+bool plane_fits(const BzFvm1d3v& op) {
+  return op.nx == 2 && op.Nx <= 64 * 8 && op.nvt >= 2 && op.nvt <= 5 && plane_doubles(op) <= 8192;
+}
+
+template <int ND>
+void launch_plane(const BzFvm1d3v& op, const double* E, double dt, double* y, double* s, const int* done,
+                  hipStream_t st) {
+  const int per = (op.Nx + 63) / 64;
+  const size_t lds = plane_doubles(op) * sizeof(double);
+  if (per <= 2) hipLaunchKernelGGL((k_fvm_plane<ND, 2>), dim3(op.Nr), dim3(PT), lds, st, op, E, dt, y, s, done);
+  else if (per <= 4) hipLaunchKernelGGL((k_fvm_plane<ND, 4>), dim3(op.Nr), dim3(PT), lds, st, op, E, dt, y, s, done);
+  else hipLaunchKernelGGL((k_fvm_plane<ND, 8>), dim3(op.Nr), dim3(PT), lds, st, op, E, dt, y, s, done);
+}
+
 template <int MODE, int ND>
 void launch_sweep_nd(const BzFvm1d3v& op, int N, int nsys, const double* E, double dt, const double* b, double* out,
                      const double* h, const int* done, hipStream_t st) {
@@ -639,12 +785,9 @@ int check_op(const BzFvm1d3v* op) {
   return BZ_OK;
 }
 
-}  // namespace
-
-extern "C" {
-
-int bz_fvm_rhs_mvec_until(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y, const int* done,
-                          hipStream_t stream) {
+// The step operator on x; have_moment: work already holds the moment of x.
+int launch_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y, bool have_moment,
+                    const int* done, hipStream_t stream) {
   int rc = check_op(op);
   if (rc != BZ_OK) return rc;
   if (!E || !x || !y || x == y) return BZ_EINVAL;
@@ -653,27 +796,31 @@ int bz_fvm_rhs_mvec_until(const BzFvm1d3v* op, const double* E, double dt, const
     return BZ_EINVAL;
   const int nrx = op->Nr * op->Nx;
   double* s = op->work;
-  hipLaunchKernelGGL(k_fvm_moment, dim3((nrx + 255) / 256), dim3(256), 0, stream, x, op->wq, op->Nr, op->Nvt, op->Nx,
-                     s, done);
-  BZ_LAUNCH_CHECK();
+  if (!have_moment) {
+    hipLaunchKernelGGL(k_fvm_moment, dim3((nrx + 255) / 256), dim3(256), 0, stream, x, op->wq, op->Nr, op->Nvt, op->Nx,
+                       s, done);
+    BZ_LAUNCH_CHECK();
+  }
   const long n = (long)nrx * op->Nvt;
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
   const int tx = op->Nx <= 64 ? 64 : (op->Nx <= 128 ? 128 : 256);       // row kernels: x per workgroup
-  const long nwg = (long)op->Nr * op->Nvt * ((op->Nx + tx - 1) / tx);
+  constexpr int TB = 4;
+  const long nwg = (long)op->Nr * ((op->Nvt + TB - 1) / TB) * ((op->Nx + tx - 1) / tx);
   const dim3 growx((unsigned)((nwg + 7) / 8 * 8)), browx(tx);
   const bool rows_fit = nwg < (1L << 30);
   if (rows_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
-    hipLaunchKernelGGL((k_fvm_matvec_w<2, 4, 4, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
+    hipLaunchKernelGGL((k_fvm_matvec_t<2, 4, 4, 6, TB>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
   else if (rows_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
-    hipLaunchKernelGGL((k_fvm_matvec_w<3, 3, 3, 6>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
+    hipLaunchKernelGGL((k_fvm_matvec_t<3, 3, 3, 6, TB>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
   else
     hipLaunchKernelGGL(k_fvm_matvec, grid, block, 0, stream, *op, E, dt, x, s, y, done);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }
 
-int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
-                                const int* done, hipStream_t stream) {
+// The preconditioner; *moment: whether work holds the moment of y afterwards.
+int launch_precond(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y, bool* moment,
+                   const int* done, hipStream_t stream) {
   int rc = check_op(op);
   if (rc != BZ_OK) return rc;
   if (!E || !b || !y || b == y) return BZ_EINVAL;
@@ -697,6 +844,18 @@ int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alp
   else
     rc = launch_fvm_sweep<SW_VR>(*op, E, alpha_dt, b, y, h, done, stream);
   if (rc != BZ_OK) return rc;
+  if (plane_fits(*op)) {
+    switch (op->nvt) {
+      case 2: launch_plane<2>(*op, E, alpha_dt, y, s, done, stream); break;
+      case 3: launch_plane<3>(*op, E, alpha_dt, y, s, done, stream); break;
+      case 4: launch_plane<4>(*op, E, alpha_dt, y, s, done, stream); break;
+      default: launch_plane<5>(*op, E, alpha_dt, y, s, done, stream); break;
+    }
+    BZ_LAUNCH_CHECK();
+    *moment = true;
+    return BZ_OK;
+  }
+  *moment = false;
   rc = launch_fvm_sweep<SW_VT>(*op, E, alpha_dt, y, y, nullptr, done, stream);
   if (rc != BZ_OK) return rc;
   if (op->nx == 2 && op->Nx <= 64 * 8) {
@@ -711,14 +870,27 @@ int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alp
   return launch_fvm_sweep<SW_X>(*op, E, alpha_dt, y, y, nullptr, done, stream);
 }
 
+}  // namespace
+
+extern "C" {
+
 int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y,
                     hipStream_t stream) {
-  return bz_fvm_rhs_mvec_until(op, E, dt, x, y, nullptr, stream);
+  return launch_rhs_mvec(op, E, dt, x, y, false, nullptr, stream);
 }
 
 int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
                           hipStream_t stream) {
-  return bz_fvm_precond_xvtvrc_until(op, E, alpha_dt, b, y, nullptr, stream);
+  bool moment;
+  return launch_precond(op, E, alpha_dt, b, y, &moment, nullptr, stream);
+}
+
+int bz_fvm_step_product(const BzFvm1d3v* op, const double* E, double dt, double alpha_dt, const double* v, double* t,
+                        double* w, const int* done, hipStream_t stream) {
+  if (w == v) return BZ_EINVAL;
+  bool moment = false;
+  const int rc = launch_precond(op, E, alpha_dt, v, t, &moment, done, stream);
+  return rc != BZ_OK ? rc : launch_rhs_mvec(op, E, dt, t, w, moment, done, stream);
 }
 
 }  // extern "C"

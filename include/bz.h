@@ -596,11 +596,10 @@ int bz_fvm_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
 int bz_fvm_precond_xvtvrc(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
                           hipStream_t stream);
 
-/* The same two products, no-ops when the device flag *done is set (done may be NULL). */
-int bz_fvm_rhs_mvec_until(const BzFvm1d3v* op, const double* E, double dt, const double* x, double* y, const int* done,
-                          hipStream_t stream);
-int bz_fvm_precond_xvtvrc_until(const BzFvm1d3v* op, const double* E, double alpha_dt, const double* b, double* y,
-                                const int* done, hipStream_t stream);
+/* t = P v (the preconditioner with step alpha_dt) and w = A t (the step operator with step dt);
+ * nothing when the device flag *done is set (done may be NULL).  v, t and w do not alias. */
+int bz_fvm_step_product(const BzFvm1d3v* op, const double* E, double dt, double alpha_dt, const double* v, double* t,
+                        double* w, const int* done, hipStream_t stream);
 
 #ifdef __cplusplus
 }
