@@ -102,13 +102,19 @@ __global__ __launch_bounds__(256) void k_fvm_matvec(BzFvm1d3v op, const double* 
   y[e] = out;
 }
 
+// A load at a workgroup-uniform row plus a byte offset of the lane (one instruction, no address
+// arithmetic in the vector unit).
+__device__ __forceinline__ double row_load(const double* row, unsigned off) {
+  return *(const double*)((const char*)row + off);
+}
+
 // The step operator for fixed stencil widths (the common ones), TB ordinates of one (r, x) per
-// thread: the element alone takes 24 vector loads (8 state values, 6 gains, 10 stencil weights);
-// with TB together the gains, the x weights and most angular neighbours are shared and the radial
-// and angular weights are uniform (scalar loads, both directions, chosen per lane), 8 vector loads
-// an element.  Every neighbour load is issued unconditionally from a clamped address and weighted
-// by zero where the stencil has no entry.  Same sums, in the same order, as k_fvm_matvec (the zero
-// terms add exactly nothing).  Measured at 671 x 16 x 100: MVFIG.
+// thread, all on one side of theta = pi / 2, so that only the sign of E differs between lanes.
+// What bounds it is the vector unit: one element per thread with every index, clamp and weight
+// worked out per lane took about 1000 instructions for four elements.  Here rows are addressed by
+// scalars, weights outside the domain are zeroed as scalars (their clamped operands are values the
+// stencil uses anyway), the gains and the x weights are shared by the TB ordinates, and the
+// angular sum is taken both ways and chosen once.  Measured at 671 x 16 x 100: 19.3 -> 11.6 us.
 template <int NX, int NVR, int NVT, int GMAX, int TB>
 __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                       const double* __restrict__ x, const double* __restrict__ s,
@@ -120,89 +126,98 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
   // grid is a multiple of 8 and XCD k takes the k-th eighth of the rows, so the radial neighbours
   // of a row are read through the same L2.
   const int bx = (Nx + blockDim.x - 1) / blockDim.x;            // workgroups per row
-  const int ntg = (Nvt + TB - 1) / TB;
+  const int ntg = Nvt / TB;
   const unsigned per = gridDim.x >> 3;
   const unsigned lb = (blockIdx.x & 7u) * per + (blockIdx.x >> 3);
   const int row = (int)(lb / (unsigned)bx);
   const int ix = (int)(lb - (unsigned)row * bx) * blockDim.x + threadIdx.x;
   if (row >= Nr * ntg || ix >= Nx) return;
   const int r = row / ntg, t0 = (row - r * ntg) * TB;
-  const int mp = Nvt / 2;
-  const long rs = (long)Nvt * Nx;
-  const double* xr0 = x + (long)r * rs + ix;
+  const bool low = t0 >= Nvt / 2;
+  const unsigned rs8 = (unsigned)Nvt * Nx * 8u, ix8 = ix * 8u;
   const double Ex = E[ix];
-  const bool ep = Ex >= 0;
+  const bool ep = Ex >= 0, up = ep == low;
+  const double* xr0 = x + (size_t)r * Nvt * Nx;
   // the ordinates of the group and NVT - 1 on either side
   constexpr int HC = NVT - 1, NC = TB + 2 * HC;
   double xc[NC], xn[TB][NX], xr[TB][NVR];
 #pragma unroll
-  for (int k = 0; k < NC; ++k) xc[k] = xr0[(long)min(max(t0 - HC + k, 0), Nvt - 1) * Nx];
+  for (int k = 0; k < NC; ++k) xc[k] = row_load(xr0 + (size_t)min(max(t0 - HC + k, 0), Nvt - 1) * Nx, ix8);
 #pragma unroll
-  for (int i = 0; i < TB; ++i) {
-    const int t = min(t0 + i, Nvt - 1);
-    const bool low = t >= mp, up = (ep == low);
+  for (int d = 1; d < NVR; ++d) {
+    const unsigned off = ix8 + (up ? min(r + d, Nr - 1) * rs8 : max(r - d, 0) * rs8);
 #pragma unroll
-    for (int k = 1; k < NX; ++k) xn[i][k] = xr0[(long)t * Nx + min(max(low ? ix - k : ix + k, 0), Nx - 1) - ix];
-#pragma unroll
-    for (int d = 1; d < NVR; ++d) xr[i][d] = xr0[(long)t * Nx + (long)(min(max(up ? r + d : r - d, 0), Nr - 1) - r) * rs];
+    for (int i = 0; i < TB; ++i) xr[i][d] = row_load(x + (size_t)(t0 + i) * Nx, off);
   }
-  double dxl[NX], dxr[NX];
+  double dx[NX];
 #pragma unroll
   for (int k = 0; k < NX; ++k) {
-    dxl[k] = op.dxL[k * Nx + ix];
-    dxr[k] = op.dxR[k * Nx + ix];
+    const int j = low ? ix - k : ix + k;
+    const bool in = j >= 0 && j < Nx;
+    dx[k] = row_load((low ? op.dxL : op.dxR) + (size_t)k * Nx, ix8);
+    if (!in) dx[k] = 0.0;
+    if (k > 0)
+#pragma unroll
+      for (int i = 0; i < TB; ++i) xn[i][k] = row_load(xr0 + (size_t)(t0 + i) * Nx, in ? 8u * j : ix8);
   }
   const int q0 = op.g_ptr[r], q1 = op.g_ptr[r + 1];
   const int qmax = max(op.g_ptr[Nr] - 1, 0);
-  double gv[GMAX], gs[GMAX];
+  double gs[GMAX];
 #pragma unroll
-  for (int k = 0; k < GMAX; ++k) {
-    const int q = min(q0 + k, qmax);
-    gv[k] = op.g_val[q];
-    gs[k] = s[(size_t)op.g_col[q] * Nx + ix];
+  for (int k = 0; k < GMAX; ++k) gs[k] = row_load(s + (size_t)op.g_col[min(q0 + k, qmax)] * Nx, ix8);
+  double wr[NVR];
+#pragma unroll
+  for (int d = 0; d < NVR; ++d) {
+    const double wu = r + d < Nr ? op.dvrR[d * Nr + r] : 0.0, wd = r - d >= 0 ? op.dvrL[d * Nr + r] : 0.0;
+    wr[d] = up ? wu : wd;
   }
   double g = 0.0;
 #pragma unroll
-  for (int k = 0; k < GMAX; ++k) g += (q0 + k < q1) ? gv[k] * gs[k] : 0.0;
+  for (int k = 0; k < GMAX; ++k)
+    if (q0 + k < q1) g += op.g_val[q0 + k] * gs[k];
   for (int q = q0 + GMAX; q < q1; ++q) g += op.g_val[q] * s[(size_t)op.g_col[q] * Nx + ix];
-  const double loss = op.loss[r], vr = op.vr[r], adx = op.dt_x * op.adx[r];
+  const double loss = op.loss[r], rvr = 1.0 / op.vr[r], adx = op.dt_x * op.adx[r];
+  const bool inflow = low ? (ix == 0) : (ix == Nx - 1);
   double out[TB];
 #pragma unroll
   for (int i = 0; i < TB; ++i) {
-    const int t = min(t0 + i, Nvt - 1);
+    const int t = t0 + i;
     const double cs = op.cos_vt[t];
-    const bool low = t >= mp, up = (ep == low);
     const double x0 = xc[HC + i];
     const double cx = adx * cs;
-    double yx = 0.0;
+    double yx = (cx * dx[0] + 1.0) * x0;
 #pragma unroll
-    for (int k = 0; k < NX; ++k) {
-      const int j = low ? ix - k : ix + k;
-      const double d = cx * (low ? dxl[k] : dxr[k]) + (k == 0 ? 1.0 : 0.0);
-      yx += (j >= 0 && j < Nx) ? d * (k == 0 ? x0 : xn[i][k]) : 0.0;
-    }
-    const bool inflow = low ? (ix == 0) : (ix == Nx - 1);
+    for (int k = 1; k < NX; ++k) yx += cx * dx[k] * xn[i][k];
     const double cv = g - loss * x0;
-    double ar = 0.0;
+    double ar = wr[0] * x0;
 #pragma unroll
-    for (int d = 0; d < NVR; ++d) {
-      const int j = up ? r + d : r - d;
-      const double wr = up ? op.dvrR[d * Nr + r] : op.dvrL[d * Nr + r];
-      ar += (j >= 0 && j < Nr) ? wr * (d == 0 ? x0 : xr[i][d]) : 0.0;
-    }
-    double at = 0.0;
+    for (int d = 1; d < NVR; ++d) ar += wr[d] * xr[i][d];
+    double au = 0.0, ad = 0.0;
 #pragma unroll
     for (int d = 0; d < NVT; ++d) {
-      const int j = ep ? t + d : t - d;
-      const double wt = ep ? op.dvtR[d * Nvt + t] : op.dvtL[d * Nvt + t];
-      at += (j >= 0 && j < Nvt) ? wt * (ep ? xc[HC + i + d] : xc[HC + i - d]) : 0.0;
+      au += (t + d < Nvt ? op.dvtR[d * Nvt + t] : 0.0) * xc[HC + i + d];
+      ad += (t - d >= 0 ? op.dvtL[d * Nvt + t] : 0.0) * xc[HC + i - d];
     }
-    const double ae = cs * ar - (op.sin_vt[t] / vr) * at;
+    const double ae = cs * ar - (op.sin_vt[t] * rvr) * (ep ? au : ad);
     out[i] = inflow ? yx : yx - dt * (op.tau_n0np0 * cv + op.tau * (Ex * (op.eq * ae)));
   }
 #pragma unroll
-  for (int i = 0; i < TB; ++i)
-    if (t0 + i < Nvt) y[(long)r * rs + (long)(t0 + i) * Nx + ix] = out[i];
+  for (int i = 0; i < TB; ++i) y[((size_t)r * Nvt + t0 + i) * Nx + ix] = out[i];
+}
+
+// Four ordinates per thread where they fit a half range, two for the remaining even half ranges
+// (6, 10, ...), one for odd ones.
+template <int NX, int NVR, int NVT>
+void launch_matvec_t(const BzFvm1d3v& op, const double* E, double dt, const double* x, const double* s, double* y,
+                     const int* done, hipStream_t st) {
+  const int mp = op.Nvt / 2;
+  const int tb = mp % 4 == 0 ? 4 : (mp % 2 == 0 ? 2 : 1);
+  const int tx = op.Nx <= 64 ? 64 : (op.Nx <= 128 ? 128 : 256);         // x per workgroup
+  const long nwg = (long)op.Nr * (op.Nvt / tb) * ((op.Nx + tx - 1) / tx);
+  const dim3 grid((unsigned)((nwg + 7) / 8 * 8)), block(tx);
+  if (tb == 4) hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 4>), grid, block, 0, st, op, E, dt, x, s, y, done);
+  else if (tb == 2) hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 2>), grid, block, 0, st, op, E, dt, x, s, y, done);
+  else hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 1>), grid, block, 0, st, op, E, dt, x, s, y, done);
 }
 
 // h = H s on the matrix cores: one workgroup of CC_WAVES wavefronts per 16 x 16 tile of h
@@ -387,16 +402,19 @@ __global__ __launch_bounds__(SWT) void k_fvm_sweep(BzFvm1d3v op, const double* _
 // y_new = alpha - sum_d beta_d y_(d-1) (alpha = b rden, beta_d = av dt D_d rden); pass 1 composes
 // the maps of its segment (K x K matrix A and offset c), the entering state of a segment is
 // the composition of the earlier segments applied to the zero state the sweep starts from
-// (through LDS), and pass 2 re-runs the segment with the sequential formula from that state.
-// The maps are contractions (upwind, 1 + av dt D_0 >= 1 in the direction of the sweep), so
-// the re-association changes the result at rounding level.  A workgroup holds SB systems
-// (consecutive x) times NSEG segments, so loads of one segment are coalesced over x.
+// (through LDS; groups of eight segments are composed first, so a segment applies at most
+// NSEG / 8 + 7 maps), and pass 2 re-runs the segment from that state.  The maps are contractions
+// (upwind, 1 + av dt D_0 >= 1 in the direction of the sweep), so the re-association changes the
+// result at rounding level.  A workgroup holds SB systems (consecutive x) times NSEG segments.
+// What bounds it is the instructions and latency of one thread, with less than a wavefront per
+// SIMD: so pass 2 reuses the coefficients of pass 1 (one division per position) and addresses are
+// 32-bit offsets.  64 segments of half the length were slower (their maps and coefficients do not
+// fit the registers of a 512-thread workgroup).  Measured at 671 x 16 x 100: 18.7 -> 15.8 us.
 constexpr int SCAN_SB = 8, NSEG = 32;
 
-// MAXL > 0: a segment has at most MAXL positions, and all of its loads (right-hand sides and
-// stencil weights, from clamped in-bounds positions) are issued up front into registers and kept
-// for pass 2, so each pass waits on memory once instead of once per position; the arithmetic,
-// and its order, are those of the MAXL = 0 form, which loads one position at a time.
+// MAXL > 0: a segment has at most MAXL positions; its loads (right-hand sides and stencil weights,
+// from clamped in-bounds positions) are issued eight positions at a time and the coefficients stay
+// in registers for pass 2; the MAXL = 0 form loads one position at a time, twice.
 template <int ND, int MAXL, int SB>
 __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                         const double* __restrict__ b, double* __restrict__ out,
@@ -404,7 +422,10 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
   if (done && *done) return;
   constexpr int K = ND > 1 ? ND - 1 : 1;
   constexpr int NL = MAXL > 0 ? MAXL : 1;
-  __shared__ double maps[SB * NSEG][K * K + K];
+  constexpr int GS = 8, NGRP = NSEG / GS;             // segments per group, groups
+  static_assert(K + 1 <= GS, "one thread per column of a group's map");
+  __shared__ double maps[SB * NSEG][K * K + K];       // column q < K of A, then c: entry [q * K + r]
+  __shared__ double gmap[SB * NGRP][K * K + K];
   const int Nr = op.Nr, Nvt = op.Nvt, Nx = op.Nx;
   const int N = Nr;
   const int j = threadIdx.x % SB, seg = threadIdx.x / SB;
@@ -416,21 +437,29 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
   const double av = -aE * op.cos_vt[t];
   const bool fwd = av >= 0;
   const double dtav = dt * av;
-  const long base = (long)t * Nx + ix, stride = (long)Nvt * Nx;
+  // byte offsets of column 0 of a row, of a row step and of a point's entry in the tables
+  const unsigned base8 = (unsigned)(t * Nx + ix) * 8u, stride8 = (unsigned)(Nvt * Nx) * 8u;
   const double* D = fwd ? op.vr_l2r : op.vr_r2l;
   const int L = (N + NSEG - 1) / NSEG;
   const int p_lo = min(seg * L, N), p_hi = min(p_lo + L, N);
-  auto coeffs = [&](int p, double& bi, double dd[ND]) __attribute__((always_inline)) {
-    const int c = fwd ? p : N - 1 - p;
-    bi = b[base + c * stride] * op.ainv[c] + h[(size_t)c * Nx + ix];
+  // (clamp: positions whose neighbours may lie before the first)
+  auto coeffs = [&](int p, double& bi, double dd[ND], bool clamp) __attribute__((always_inline)) {
+    const unsigned c = fwd ? p : N - 1 - p;
+    bi = row_load(b, base8 + c * stride8) * row_load(op.ainv, 8u * c) + row_load(h, (c * Nx + ix) * 8u);
 #pragma unroll
-    for (int d = 0; d < ND; ++d) dd[d] = D[d * N + (fwd ? max(c - d, 0) : min(c + d, N - 1))];
+    for (int d = 0; d < ND; ++d) {
+      const int e = fwd ? (int)c - d : (int)c + d;
+      dd[d] = D[d * N + (clamp ? max(0, min(e, N - 1)) : e)];
+    }
+  };
+  // bi, dd -> alpha, beta (in place; dd[0] is not used again)
+  auto affine = [&](double& bi, double dd[ND]) __attribute__((always_inline)) {
+    const double rden = 1.0 / (1.0 + av * dt * dd[0]);
+    bi *= rden;
+#pragma unroll
+    for (int d = 1; d < ND; ++d) dd[d] *= dtav * rden;
   };
   double bv[NL], dv[NL][ND];
-  if constexpr (MAXL > 0) {
-#pragma unroll
-    for (int i = 0; i < MAXL; ++i) coeffs(min(p_lo + i, N - 1), bv[i], dv[i]);
-  }
   // pass 1: the segment's map, state (y0 .. y_(K-1)), y0 the newest value
   double A[K][K], cv[K];
 #pragma unroll
@@ -439,17 +468,15 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
 #pragma unroll
     for (int q = 0; q < K; ++q) A[r][q] = (r == q) ? 1.0 : 0.0;
   }
-  auto compose = [&](double bi, const double dd[ND]) __attribute__((always_inline)) {
-    const double rden = 1.0 / (1.0 + av * dt * dd[0]);
-    double a0[K], c0 = bi * rden;
+  auto compose = [&](double alpha, const double be[ND]) __attribute__((always_inline)) {
+    double a0[K], c0 = alpha;
 #pragma unroll
     for (int q = 0; q < K; ++q) a0[q] = 0.0;
 #pragma unroll
     for (int d = ND - 1; d >= 1; --d) {
-      const double beta = dtav * dd[d] * rden;
-      c0 -= beta * cv[d - 1];
+      c0 -= be[d] * cv[d - 1];
 #pragma unroll
-      for (int q = 0; q < K; ++q) a0[q] -= beta * A[d - 1][q];
+      for (int q = 0; q < K; ++q) a0[q] -= be[d] * A[d - 1][q];
     }
 #pragma unroll
     for (int r = K - 1; r >= 1; --r) {
@@ -461,64 +488,88 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
 #pragma unroll
     for (int q = 0; q < K; ++q) A[0][q] = a0[q];
   };
-  if (active) {
-    if constexpr (MAXL > 0) {
+  if constexpr (MAXL > 0) {
+    constexpr int BT = 8;
+    static_assert(MAXL % BT == 0, "whole batches");
 #pragma unroll
-      for (int i = 0; i < MAXL; ++i)
-        if (p_lo + i < p_hi) compose(bv[i], dv[i]);
-    } else {
-      for (int p = p_lo; p < p_hi; ++p) {
-        double bi, dd[ND];
-        coeffs(p, bi, dd);
-        compose(bi, dd);
-      }
+    for (int i0 = 0; i0 < MAXL; i0 += BT) {
+#pragma unroll
+      for (int i = i0; i < i0 + BT; ++i) coeffs(min(p_lo + i, N - 1), bv[i], dv[i], i < ND - 1);
+      // a map past the last position enters only segments that hold no position
+#pragma unroll
+      for (int i = i0; i < i0 + BT; ++i)
+        if (i < L) {
+          affine(bv[i], dv[i]);
+          compose(bv[i], dv[i]);
+        }
+    }
+  } else {
+    for (int p = p_lo; p < p_hi; ++p) {
+      double bi, dd[ND];
+      coeffs(p, bi, dd, true);
+      affine(bi, dd);
+      compose(bi, dd);
     }
   }
 #pragma unroll
   for (int r = 0; r < K; ++r) {
     maps[threadIdx.x][K * K + r] = cv[r];
 #pragma unroll
-    for (int q = 0; q < K; ++q) maps[threadIdx.x][r * K + q] = A[r][q];
+    for (int q = 0; q < K; ++q) maps[threadIdx.x][q * K + r] = A[r][q];
   }
   __syncthreads();
-  if (!active || p_lo >= p_hi) return;
-  // entering state: the earlier segments' maps applied in order to the zero state
-  double y[K];
-#pragma unroll
-  for (int r = 0; r < K; ++r) y[r] = 0.0;
-  for (int sg = 0; sg < seg; ++sg) {
-    const double* m = maps[sg * SB + j];
+  // y <- A y (+ c) of one map
+  auto apply = [&](const double* m, double y[K], bool offset) __attribute__((always_inline)) {
     double yn[K];
 #pragma unroll
     for (int r = 0; r < K; ++r) {
-      double acc = m[K * K + r];
+      double acc = offset ? m[K * K + r] : 0.0;
 #pragma unroll
-      for (int q = 0; q < K; ++q) acc += m[r * K + q] * y[q];
+      for (int q = 0; q < K; ++q) acc += m[q * K + r] * y[q];
       yn[r] = acc;
     }
 #pragma unroll
     for (int r = 0; r < K; ++r) y[r] = yn[r];
-  }
-  // pass 2: the sequential recurrence over the segment
-  auto advance = [&](int p, double bi, const double dd[ND]) __attribute__((always_inline)) {
-    double sv = 0.0;
+  };
+  const int grp = seg / GS, col = seg % GS;
+  double y[K];
+  if (col <= K) {                                      // one column of the group's map per thread
 #pragma unroll
-    for (int d = ND - 1; d >= 1; --d) sv += dd[d] * y[d - 1];
-    const double rden = 1.0 / (1.0 + av * dt * dd[0]);
-    const double val = (bi - sv * dtav) * rden;
+    for (int r = 0; r < K; ++r) y[r] = col == r ? 1.0 : 0.0;
+    if (col == K)
+#pragma unroll
+      for (int r = 0; r < K; ++r) y[r] = 0.0;
+    for (int i = 0; i < GS; ++i) apply(maps[(grp * GS + i) * SB + j], y, col == K);
+#pragma unroll
+    for (int r = 0; r < K; ++r) gmap[grp * SB + j][col * K + r] = y[r];
+  }
+  __syncthreads();
+  if (!active || p_lo >= p_hi) return;
+  // entering state: the earlier groups' and segments' maps applied in order to the zero state
+#pragma unroll
+  for (int r = 0; r < K; ++r) y[r] = 0.0;
+  for (int i = 0; i < grp; ++i) apply(gmap[i * SB + j], y, true);
+  for (int i = 0; i < col; ++i) apply(maps[(grp * GS + i) * SB + j], y, true);
+  // pass 2: the recurrence over the segment
+  auto advance = [&](int p, double alpha, const double be[ND]) __attribute__((always_inline)) {
+    double val = alpha;
+#pragma unroll
+    for (int d = ND - 1; d >= 1; --d) val -= be[d] * y[d - 1];
 #pragma unroll
     for (int d = K - 1; d >= 1; --d) y[d] = y[d - 1];
     y[0] = val;
-    out[base + (fwd ? p : N - 1 - p) * stride] = val;
+    const unsigned c = fwd ? p : N - 1 - p;
+    if (p < p_hi) *(double*)((char*)out + (base8 + c * stride8)) = val;
   };
   if constexpr (MAXL > 0) {
 #pragma unroll
     for (int i = 0; i < MAXL; ++i)
-      if (p_lo + i < p_hi) advance(p_lo + i, bv[i], dv[i]);
+      if (i < L) advance(p_lo + i, bv[i], dv[i]);
   } else {
     for (int p = p_lo; p < p_hi; ++p) {
       double bi, dd[ND];
-      coeffs(p, bi, dd);
+      coeffs(p, bi, dd, true);
+      affine(bi, dd);
       advance(p, bi, dd);
     }
   }
@@ -803,15 +854,11 @@ int launch_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
   }
   const long n = (long)nrx * op->Nvt;
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
-  const int tx = op->Nx <= 64 ? 64 : (op->Nx <= 128 ? 128 : 256);       // row kernels: x per workgroup
-  constexpr int TB = 4;
-  const long nwg = (long)op->Nr * ((op->Nvt + TB - 1) / TB) * ((op->Nx + tx - 1) / tx);
-  const dim3 growx((unsigned)((nwg + 7) / 8 * 8)), browx(tx);
-  const bool rows_fit = nwg < (1L << 30);
-  if (rows_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
-    hipLaunchKernelGGL((k_fvm_matvec_t<2, 4, 4, 6, TB>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
-  else if (rows_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
-    hipLaunchKernelGGL((k_fvm_matvec_t<3, 3, 3, 6, TB>), growx, browx, 0, stream, *op, E, dt, x, s, y, done);
+  const bool offsets_fit = n < (1L << 29);            // row_load's 32-bit byte offsets
+  if (offsets_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
+    launch_matvec_t<2, 4, 4>(*op, E, dt, x, s, y, done, stream);
+  else if (offsets_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
+    launch_matvec_t<3, 3, 3>(*op, E, dt, x, s, y, done, stream);
   else
     hipLaunchKernelGGL(k_fvm_matvec, grid, block, 0, stream, *op, E, dt, x, s, y, done);
   BZ_LAUNCH_CHECK();
@@ -837,9 +884,9 @@ int launch_precond(const BzFvm1d3v* op, const double* E, double alpha_dt, const 
   hipLaunchKernelGGL(k_fvm_coll_corr, dim3((op->Nr + 15) / 16, (op->Nx + 15) / 16), dim3(64 * CC_WAVES), 0, stream,
                      op->H, op->h_lo, s, op->Nr, op->Nx, h, done);
   BZ_LAUNCH_CHECK();
-  // the radial sweep: segmented scan for the common stencils and long radial lines, else one
-  // thread per line
-  if (op->nvr >= 2 && op->nvr <= 5 && op->Nr >= 2 * NSEG)
+  // the radial sweep: segmented scan for the common stencils, long radial lines and states within
+  // its 32-bit byte offsets, else one thread per line
+  if (op->nvr >= 2 && op->nvr <= 5 && op->Nr >= 2 * NSEG && (long)nrx * op->Nvt < (1L << 29))
     rc = launch_fvm_vr_scan(*op, E, alpha_dt, b, y, h, done, stream);
   else
     rc = launch_fvm_sweep<SW_VR>(*op, E, alpha_dt, b, y, h, done, stream);
