@@ -13,10 +13,12 @@
 //
 // The ion fluid lives on Np <= 200 Chebyshev points.  Its backward-Euler Jacobian is a dense
 // Np x Np matrix that changes with the field every half step, and the reference inverts it.
-// One workgroup of 1024 threads holds the matrix in registers (thread (r, g) owns row r and
-// the columns g Sc .. g Sc + Sc - 1, g < CG = 1024 / Np, Sc = ceil(Np / CG)) and inverts it
-// in place by Gauss-Jordan elimination with partial pivoting.  Pivot rows are chosen, never moved: the inverse comes out with
-// permuted rows and columns and is applied through the permutation.  The Newton loop of the
+// One workgroup of 512 threads holds the matrix in registers: as tiles where its columns are
+// diagonally dominant (Jacobi iterations, or elimination without row exchanges), else by rows
+// (thread (r, g) owns row r and the columns g Sc .. g Sc + Sc - 1, g < CG = min(512 / Np, Np),
+// Sc = ceil(Np / CG)), inverted in place by Gauss-Jordan elimination with partial pivoting.  Pivot
+// rows are chosen, never moved: the inverse comes out with permuted rows and columns and is applied
+// through the permutation.  The Newton loop of the
 // reference, its residuals (two products with the Chebyshev derivative matrix, which stays
 // in L2) and the Poisson fields run in the same launch, so a half step is one launch with no
 // host round trip.  The whole step is FP64.
@@ -25,11 +27,11 @@
 
 namespace {
 
-constexpr int GF_THREADS = 1024;
+constexpr int GF_THREADS = 512;
 constexpr int GF_WAVES = GF_THREADS / 64;
 constexpr int GF_NMAX = 200;
-constexpr int GF_NPAD = 384;       // >= CG ceil(Np / CG) for every Np <= 200: padded vectors
-constexpr int BZ_GLOW_TILE_THREADS = 512;   // block size of the tile layouts
+constexpr int GF_NPAD = 384;       // >= CG ceil(Np / CG) and CG SMAX for every Np <= 200: padded vectors
+constexpr int BZ_GLOW_TILE_THREADS = 512;   // = GF_THREADS: tables are laid out by thread
 constexpr int GF_TILE_RED = 5000;  // >= max(TR, TC) Npad of the tile layouts below (25 x 200 at 8 x 10)
 
 enum { V_NE = 0, V_NI, V_E, V_X, V_RR, V_R0, V_W, V_Z, V_DX, V_DI, V_COUNT };
@@ -57,20 +59,48 @@ struct GfCtx {
   bool act;
 };
 
+// s + sum_i f(i), i = i0, i0 + di, ... < n in order, U operand loads in flight: with a single
+// workgroup nothing else hides their latency.
+template <int U, typename F>
+__device__ __forceinline__ double gf_sum(double s, int i0, int di, int n, F term) {
+  int i = i0;
+  for (; i + (U - 1) * di < n; i += U * di) {
+    double v[U], w[U];
+#pragma unroll
+    for (int u = 0; u < U; ++u) term(i + u * di, v[u], w[u]);
+#pragma unroll
+    for (int u = 0; u < U; ++u) s = fma(v[u], w[u], s);
+  }
+  for (; i < n; i += di) {
+    double v, w;
+    term(i, v, w);
+    s = fma(v, w, s);
+  }
+  return s;
+}
+
+// sum over g < count of p[g * stride], in order (LDS)
+__device__ __forceinline__ double gf_strided_sum(const double* p, int stride, int count) {
+  return gf_sum<8>(0.0, 0, 1, count, [&](int g, double& v, double& w) {
+    v = p[g * stride];
+    w = 1.0;
+  });
+}
+
 // y[r] = sum_c M[r][c] x[c] for M given transposed (MT[c n + r] = M[r][c], so the lanes of a
 // wave read consecutive entries); x and y in LDS and distinct.
+template <int U>
 __device__ __forceinline__ void gf_matvec(const GfCtx& q, GfShared& S, const double* __restrict__ MT,
                                           const double* x, double* y) {
   if (q.act) {
-    double acc = 0.0;
-    for (int c = q.cg; c < q.n; c += q.CG) acc = fma(MT[(size_t)c * q.n + q.r], x[c], acc);
-    S.red[q.cg * q.n + q.r] = acc;
+    S.red[q.cg * q.n + q.r] = gf_sum<U>(0.0, q.cg, q.CG, q.n, [&](int c, double& v, double& w) {
+      v = MT[(size_t)c * q.n + q.r];
+      w = x[c];
+    });
   }
   __syncthreads();
   if (q.t < q.n) {
-    double s = 0.0;
-    for (int g = 0; g < q.CG; ++g) s += S.red[g * q.n + q.t];
-    y[q.t] = s;
+    y[q.t] = gf_strided_sum(S.red + q.t, q.n, q.CG);
   }
   __syncthreads();
 }
@@ -99,24 +129,25 @@ __device__ __forceinline__ void gf_field(const GfCtx& q, GfShared& S, const BzGl
     S.vec[V_W][t] = (t == 0) ? bc : (t == q.n - 1 ? 0.0 : -g.alpha * (S.vec[V_NI][t] - S.vec[V_NE][t]));
   }
   __syncthreads();
-  gf_matvec(q, S, g.GT, S.vec[V_W], out);
+  gf_matvec<16>(q, S, g.GT, S.vec[V_W], out);
 }
 
 // rr = x - h (ki n0 ne - Dp flux),  flux = mu ni1 E - Di Dp ni1 (weak flux mu ni1 E at both
 // ends), ni1 = ni + x.
+template <int U>
 __device__ __forceinline__ void gf_residual(const GfCtx& q, GfShared& S, const BzGlowFluid& g, double h,
                                             const double* x, double* rr) {
   const int t = q.t;
   if (t < q.n) S.vec[V_W][t] = S.vec[V_NI][t] + x[t];
   __syncthreads();
-  gf_matvec(q, S, g.DpT, S.vec[V_W], S.vec[V_Z]);
+  gf_matvec<U>(q, S, g.DpT, S.vec[V_W], S.vec[V_Z]);
   if (t < q.n) {
     const double ni1 = S.vec[V_W][t];
     const double adv = g.mu_i * ni1 * S.vec[V_E][t];
     S.vec[V_Z][t] = (t == 0 || t == q.n - 1) ? adv : adv - g.Di * S.vec[V_Z][t];
   }
   __syncthreads();
-  gf_matvec(q, S, g.DpT, S.vec[V_Z], S.vec[V_W]);
+  gf_matvec<U>(q, S, g.DpT, S.vec[V_Z], S.vec[V_W]);
   if (t < q.n) rr[t] = x[t] - h * (g.ki[t] * g.n0 * S.vec[V_NE][t] - S.vec[V_W][t]);
   __syncthreads();
 }
@@ -138,9 +169,7 @@ __device__ __forceinline__ void gf_apply_inverse(const GfCtx& q, GfShared& S, co
   }
   __syncthreads();
   if (q.t < q.n) {
-    double s = 0.0;
-    for (int g = 0; g < q.CG; ++g) s += S.red[g * q.n + q.t];
-    dx[S.qinv[q.t]] = s;
+    dx[S.qinv[q.t]] = gf_strided_sum(S.red + q.t, q.n, q.CG);
   }
   __syncthreads();
 }
@@ -260,7 +289,7 @@ __device__ __forceinline__ int gf_gauss_jordan(const GfCtx& q, GfShared& S, doub
 
 // Newton with the frozen inverse and the damping restarts of glow1d_utils.newton_solver
 // (glow1d_utils.py:131-207): apply(rr, dx) writes dx = J^-1 rr.  Writes ni and the status.
-template <typename Apply>
+template <int U, typename Apply>
 __device__ __forceinline__ void gf_newton(const GfCtx& q, GfShared& S, const BzGlowFluid& g, double h, int singular,
                                           Apply apply) {
   const int n = q.n, t = q.t;
@@ -269,7 +298,7 @@ __device__ __forceinline__ void gf_newton(const GfCtx& q, GfShared& S, const BzG
   double* r0 = S.vec[V_R0];
   if (t < n) x[t] = 0.0;
   __syncthreads();
-  gf_residual(q, S, g, h, x, r0);
+  gf_residual<U>(q, S, g, h, x, r0);
   const double nr0 = gf_norm(q, S, r0);
   double nr = nr0;
   bool conv = (nr / nr0 < g.rtol) || (nr < g.atol);
@@ -286,7 +315,7 @@ __device__ __forceinline__ void gf_newton(const GfCtx& q, GfShared& S, const BzG
       apply(rr, S.vec[V_DX]);
       if (t < n) x[t] = x[t] - alpha * S.vec[V_DX][t];
       __syncthreads();
-      gf_residual(q, S, g, h, x, rr);
+      gf_residual<U>(q, S, g, h, x, rr);
       nr = gf_norm(q, S, rr);
       ++count;
       conv = (nr / nr0 < g.rtol) || (nr < g.atol);
@@ -383,16 +412,16 @@ __device__ __forceinline__ bool gf_tile_build(const GfCtx& q, GfShared& S, const
   if (q.t == 0) S.flag = 1;
   __syncthreads();
   if (q.t < tl.Npad) {
-    double sum = 0.0;
-    for (int r = 0; r < tl.TR; ++r) sum += S.red2[r * tl.Npad + q.t];
+    const double sum = gf_strided_sum(S.red2 + q.t, tl.Npad, tl.TR);
     if (!(S.tprow[0][q.t] > sum)) S.flag = 0;
     S.red[q.t] = sum / S.tprow[0][q.t];            // column ratio (padding columns: 0)
   }
   __syncthreads();
-  if (q.t == 0) {
+  if (q.t < 64) {
     double rmax = 0.0;
-    for (int c = 0; c < tl.Npad; ++c) rmax = fmax(rmax, S.red[c]);
-    S.sc[0] = rmax;
+    for (int c = q.t; c < tl.Npad; c += 64) rmax = fmax(rmax, S.red[c]);
+    for (int off = 32; off > 0; off >>= 1) rmax = fmax(rmax, __shfl_xor(rmax, off, 64));
+    if (q.t == 0) S.sc[0] = rmax;
   }
   __syncthreads();
   const bool dom = S.flag != 0;
@@ -431,8 +460,7 @@ __device__ __forceinline__ void gf_tile_jacobi(const GfCtx& q, GfShared& S, cons
     }
     __syncthreads();
     if (t < q.n) {
-      double w = 0.0;
-      for (int c = 0; c < tl.TC; ++c) w += S.red2[c * tl.Npad + t];
+      const double w = gf_strided_sum(S.red2 + t, tl.Npad, tl.TC);
       dx[t] = fma(di[t], rr[t] - w, dx[t]);
     }
     __syncthreads();
@@ -517,9 +545,7 @@ __device__ __forceinline__ void gf_tile_apply(const GfCtx& q, GfShared& S, const
   }
   __syncthreads();
   if (q.t < q.n) {
-    double s = 0.0;
-    for (int c = 0; c < tl.TC; ++c) s += S.red2[c * tl.Npad + q.t];
-    dx[q.t] = s;
+    dx[q.t] = gf_strided_sum(S.red2 + q.t, tl.Npad, tl.TC);
   }
   __syncthreads();
 }
@@ -531,7 +557,7 @@ __global__ __launch_bounds__(NT) void k_glow_fluid(BzGlowFluid g, int flags, dou
   GfCtx q;
   q.n = g.n;
   q.t = threadIdx.x;
-  q.CG = NT / q.n;
+  q.CG = min(NT / q.n, q.n);                         // at most 22 groups: CG SMAX entries of prow
   q.nw = NT / 64;
   q.r = q.t % q.n;
   q.cg = q.t / q.n;
@@ -551,14 +577,15 @@ __global__ __launch_bounds__(NT) void k_glow_fluid(BzGlowFluid g, int flags, dou
     double m[3];
     for (int k = 0; k < 3; ++k) {
       if (q.act) {
-        double acc = 0.0;
-        for (int sp = q.cg; sp < g.nsplit; sp += q.CG) acc += g.partial[((size_t)sp * 3 + k) * n + q.r];
-        S.red[q.cg * n + q.r] = acc;
+        S.red[q.cg * n + q.r] = gf_sum<8>(0.0, q.cg, q.CG, g.nsplit, [&](int sp, double& v, double& w) {
+          v = g.partial[((size_t)sp * 3 + k) * n + q.r];
+          w = 1.0;
+        });
       }
       __syncthreads();
       m[k] = 0.0;
       if (t < n)
-        for (int gg = 0; gg < q.CG; ++gg) m[k] += S.red[gg * n + t];
+        m[k] = gf_strided_sum(S.red + t, n, q.CG);
       __syncthreads();
     }
     if (t < n) {
@@ -580,16 +607,17 @@ __global__ __launch_bounds__(NT) void k_glow_fluid(BzGlowFluid g, int flags, dou
       // pivot-free tile path when J is column diagonally dominant
       const GfTile tl = gf_tile_ctx<BR, BC>(q);
       double Xt[BR][BC];
+      constexpr int UT = BR * BC <= 36 ? 16 : 6;     // products' loads in flight beside the tile
       if (gf_tile_build<BR, BC>(q, S, g, h, tl, Xt)) {
         const double rho = S.sc[0];
         if (rho <= 0.5) {
           // strongly dominant (the glow's half steps: rho about 0.14): Jacobi iterations on J
           const int K = rho > 0.0 ? (int)ceil(36.7368005696771 / -log(rho)) + 1 : 1;   // 53 ln 2
-          gf_newton(q, S, g, h, 4,                                   // bit 2: Jacobi path
+          gf_newton<UT>(q, S, g, h, 4,                                   // bit 2: Jacobi path
                     [&](const double* rr, double* dx) { gf_tile_jacobi<BR, BC>(q, S, tl, Xt, K, rr, dx); });
         } else {
           const int singular = gf_tile_gauss_jordan<BR, BC>(q, S, tl, Xt);
-          gf_newton(q, S, g, h, singular,
+          gf_newton<UT>(q, S, g, h, singular,
                     [&](const double* rr, double* dx) { gf_tile_apply<BR, BC>(q, S, tl, Xt, rr, dx); });
         }
         done = true;
@@ -612,7 +640,7 @@ __global__ __launch_bounds__(NT) void k_glow_fluid(BzGlowFluid g, int flags, dou
         }
       }
       const int singular = gf_gauss_jordan<SMAX>(q, S, X, Sc) | 2;     // bit 1: pivoted path
-      gf_newton(q, S, g, h, singular,
+      gf_newton<SMAX <= 32 ? 8 : 2>(q, S, g, h, singular,
                 [&](const double* rr, double* dx) { gf_apply_inverse<SMAX>(q, S, X, Sc, rr, dx); });
     }
   }
@@ -655,14 +683,12 @@ __global__ __launch_bounds__(256) void k_glow_moments(const double* __restrict__
 
 }  // namespace
 
-// The kernel variant (register layout) bz_glow_fluid_step uses for n points: 0, 1: row
-// layouts of 2 and 8 columns per thread at 1024 threads; 2: 6 x 6 tiles at 512; 3: 8 x 10.
-static int gf_variant(int n) {
-  const int CG = GF_THREADS / n, Sc = (n + CG - 1) / CG;
-  if (Sc <= 2) return 0;
-  if (Sc <= 8) return 1;
-  return n <= 128 ? 2 : 3;
-}
+// The kernel variant (register layout) bz_glow_fluid_step uses for n points.
+// Tile layouts: 4 x 4 up to 88 points (at most 22 x 22 threads), 6 x 6 up to 128 (Npad <= 132,
+// 22 x 22), 8 x 10 up to 200 (25 x 20).  Below 90 points a layout of rows over 1024 threads, which
+// can only eliminate (two barriers of 16 wavefronts a pivot), took 114 us a launch on average at 75
+// points, tiles 26; with the operands of the products batched, 200 points went from 120 to 71.
+static int gf_variant(int n) { return n <= 88 ? 1 : (n <= 128 ? 2 : 3); }
 
 template <int BR, int BC>
 __global__ __launch_bounds__(256) void k_glow_tile_order(const double* __restrict__ DpT,
@@ -690,14 +716,15 @@ extern "C" int bz_glow_tile_tables(int n, const double* DpT, const double* DppT,
                                    hipStream_t stream) {
   if (n < 3 || n > GF_NMAX || !DpT || !DppT || !DpTile || !DppTile) return BZ_EINVAL;
   const int v = gf_variant(n);
-  if (v == 2) {
+  if (v == 1) {
+    hipLaunchKernelGGL((k_glow_tile_order<4, 4>), dim3((16 * BZ_GLOW_TILE_THREADS + 255) / 256), dim3(256), 0,
+                       stream, DpT, DppT, n, DpTile, DppTile);
+  } else if (v == 2) {
     hipLaunchKernelGGL((k_glow_tile_order<6, 6>), dim3((36 * BZ_GLOW_TILE_THREADS + 255) / 256), dim3(256), 0,
                        stream, DpT, DppT, n, DpTile, DppTile);
-  } else if (v == 3) {
+  } else {
     hipLaunchKernelGGL((k_glow_tile_order<8, 10>), dim3((80 * BZ_GLOW_TILE_THREADS + 255) / 256), dim3(256), 0,
                        stream, DpT, DppT, n, DpTile, DppTile);
-  } else {
-    return BZ_OK;
   }
   BZ_LAUNCH_CHECK();
   return BZ_OK;
@@ -721,20 +748,16 @@ extern "C" int bz_glow_fluid_step(const BzGlowFluid* g, int flags, double h, dou
                                  g->max_iter < 0))
     return BZ_EINVAL;
   if ((flags & BZ_GLOW_FIELD_AFTER) && (!g->GT || !g->bsE)) return BZ_EINVAL;
-  // tile layouts: 8 x 10 for 128 < n <= 200 (Npad <= 200, 25 x 20 threads), 6 x 6 for
-  // 90 < n <= 128 (Npad <= 132, 22 x 22 threads): LDS reductions of max(TR, TC) Npad entries
+  // LDS reductions of max(TR, TC) Npad entries
   static_assert(25 * 200 <= GF_TILE_RED && 22 * 132 <= GF_TILE_RED, "tile reduction buffer");
   static_assert(25 * 20 <= 512 && 22 * 22 <= 512, "tile threads");
+  static_assert((88 + 512 / 88 - 1) / (512 / 88) <= 18, "row layout");
   const BzGlowFluid gv = *g;
-  // register layout: the matrix fits in registers either at 1024 threads (4 waves per SIMD,
-  // 128 registers each) with up to 8 columns per thread, or at 512 threads (256 registers)
-  // with up to 32 (n <= 128) or 100 columns per thread
+  // the row layout of the eliminating path: up to 18 columns a thread at 88 points, 32 at 128 and
+  // 100 at 200 in the 256 registers that 512 threads leave each
   switch (gf_variant(g->n)) {
-    case 0:
-      hipLaunchKernelGGL((k_glow_fluid<1024, 2, 0, 0>), dim3(1), dim3(1024), 0, stream, gv, flags, h, bc_before, bc_after);
-      break;
     case 1:
-      hipLaunchKernelGGL((k_glow_fluid<1024, 8, 0, 0>), dim3(1), dim3(1024), 0, stream, gv, flags, h, bc_before, bc_after);
+      hipLaunchKernelGGL((k_glow_fluid<512, 18, 4, 4>), dim3(1), dim3(512), 0, stream, gv, flags, h, bc_before, bc_after);
       break;
     case 2:
       hipLaunchKernelGGL((k_glow_fluid<512, 32, 6, 6>), dim3(1), dim3(512), 0, stream, gv, flags, h, bc_before, bc_after);
