@@ -303,8 +303,8 @@ __global__ __launch_bounds__(OT) void k_gmres_residual(const double* __restrict_
   if (threadIdx.x == 0) partial[blockIdx.x] = t;
 }
 
-// stat: |r|, |b|, tol = max(atol, rtol |b|), steps of the cycle.  out = |r| or |b| (of = 0, 1);
-// of = 0 also fills in the tolerance and the step count.
+// stat: |r|, |b|, tol = max(atol, rtol |b|), steps of the cycle.  of: 0 the residual's norm (and
+// the step count), 1 the right-hand side's (and the tolerance), 2 both at once (r = b).
 __global__ __launch_bounds__(OT) void k_gmres_stat(const double* __restrict__ partial, int nblk, int of, double atol,
                                                    double rtol, const int* __restrict__ kdone, double* stat) {
   __shared__ double red[OT / 64];
@@ -312,10 +312,13 @@ __global__ __launch_bounds__(OT) void k_gmres_stat(const double* __restrict__ pa
   for (int k = threadIdx.x; k < nblk; k += OT) t += partial[k];
   const double v = sqrt(block_sum(t, red));
   if (threadIdx.x == 0) {
-    stat[of] = v;
-    if (of == 0) {
-      stat[2] = fmax(atol, rtol * stat[1]);
+    if (of != 1) {
+      stat[0] = v;
       stat[3] = (double)*kdone;
+    }
+    if (of != 0) {
+      stat[1] = v;
+      stat[2] = fmax(atol, rtol * v);
     }
   }
 }
@@ -568,7 +571,7 @@ int bz_gmres_orthogonalise(double* V, long ldv, int m, int i, double* w, long n,
 
 int bz_gmres_norm(const double* b, const double* ax, double* r, long n, double* partial, int of, double atol, double rtol,
                   const int* kdone, double* stat, hipStream_t stream) {
-  if (n < 1 || !b || !partial || !kdone || !stat || of < 0 || of > 1) return BZ_EINVAL;
+  if (n < 1 || !b || !partial || !kdone || !stat || of < 0 || of > 2) return BZ_EINVAL;
   const int nblk = orth_blocks(n, 2 * OT);
   hipLaunchKernelGGL(k_gmres_residual, dim3(nblk), dim3(OT), 0, stream, b, ax, r, n, (n + nblk - 1) / nblk, partial);
   BZ_LAUNCH_CHECK();

@@ -138,8 +138,10 @@ class ArnoldiCycle:
     """The device state of a restarted GMRES cycle and its vector operations (bz_krylov.hip):
     basis, Hessenberg column rotation, residual estimate, stop flag.  A subclass supplies
     `product(src, out, done)`: t = P src and out = A t (device addresses; nothing when the device
-    flag `done` is set).  After the first cycle the steps are replayed from HIP graphs of `chunk`
-    steps; the host reads the stop flag between them.  Steps past convergence are no-ops."""
+    flag `done` is set).  After the first cycle everything between two read-backs is one HIP graph:
+    the residual of a start vector, the beginning of a cycle with its first `chunk` steps, each
+    further chunk, and the end of a cycle (solution and true residual).  The host reads the stop
+    flag after a chunk and the residual after a cycle.  Steps past convergence are no-ops."""
 
     def __init__(self, n, restart, dev, chunk, gs_passes, use_graph=True):
         f64, i32 = torch.float64, torch.int32
@@ -166,24 +168,29 @@ class ArnoldiCycle:
         _lib.call("bz_gmres_orthogonalise", self.V, self.n, self.m, i, self.w, self.n, self.gs_passes, self.partial,
                   self.H, self.ldh, self.cs, self.sn, self.g, self.tol, done, kdone)
 
-    def _capture(self):
+    def _steps(self, i0):
+        for i in range(i0, min(self.m, i0 + self.chunk)):
+            self._step(i)
+
+    def _capture(self, parts):
+        """The replays of one graph for every sequence of launches in `parts`."""
+        run = {}
         with capture_guard():
-            self.graphs = []
-            for i0 in range(0, self.m, self.chunk):
+            for name, launch in parts.items():
                 gr = torch.cuda.CUDAGraph()
                 with torch.cuda.graph(gr):
-                    for i in range(i0, min(self.m, i0 + self.chunk)):
-                        self._step(i)
-                self.graphs.append(gr)
+                    launch()
+                run[name] = gr.replay
+        return run
 
     def _norm(self, of, b, ax, r, atol=0.0, rtol=0.0):
         _lib.call("bz_gmres_norm", b, ax, r, self.n, self.partial, of, float(atol), float(rtol), _ptr(self.flags, 1),
                   self.stat)
 
-    def _residual(self, atol, rtol):
+    def _residual(self):
         """r = b - A P x with its norm; leaves P x in t."""
         self.product(_at(self.x), _at(self.r), None)
-        self._norm(0, self.b, self.r, self.r, atol, rtol)
+        self._norm(0, self.b, self.r, self.r)
 
     def _solution(self):
         """x += V y over the steps of the cycle."""
@@ -198,33 +205,36 @@ class ArnoldiCycle:
     def cycles(self, atol, rtol, max_cycles, zero_start, callback=None):
         """Cycles from x (zero_start: x = 0) for the right-hand side b, until the true residual
         is below tol = max(atol, rtol |b|).  Returns (converged, total steps); P x is in t."""
-        self._norm(1, self.b, None, None)
-        if zero_start:
-            self.t.zero_()
-            self._norm(0, self.b, None, self.r, atol, rtol)
-        else:
-            self._residual(atol, rtol)
-        iters = 0
-        for _ in range(max_cycles):
-            # r and its norm are those of the current x: computed above, or at the end of the
+        def begin():
+            # r and its norm are those of the current x: from the start, or from the end of the
             # previous cycle.  When |r| is below the tolerance at the start the cycle is empty.
             _lib.call("bz_gmres_begin", self.r, self.stat, self.V, self.n, self.m, self.g, self.tol,
                       _ptr(self.flags, 0), _ptr(self.flags, 1))
-            if self.graphs is None:
-                # eager cycle (the first one loads and runs every kernel once), then capture
-                for i in range(self.m):
-                    self._step(i)
-                    if (i + 1) % self.chunk == 0 and int(self.flags[0].item()):
-                        break
-                if self.use_graph:
-                    self._capture()
-            else:
-                for gr in self.graphs:
-                    gr.replay()
-                    if int(self.flags[0].item()):
-                        break
+            self._steps(0)
+
+        def end():
             self._solution()
-            self._residual(atol, rtol)
+            self._residual()
+
+        parts = {"residual": self._residual, "end": end, 0: begin}
+        parts.update({i0: lambda i0=i0: self._steps(i0) for i0 in range(self.chunk, self.m, self.chunk)})
+        run = self.graphs or parts
+        if zero_start:
+            self.t.zero_()
+            self._norm(2, self.b, None, self.r, atol, rtol)        # r = b
+        else:
+            self._norm(1, self.b, None, None, atol, rtol)
+            run["residual"]()
+        iters = 0
+        for _ in range(max_cycles):
+            for i0 in range(0, self.m, self.chunk):
+                run[i0]()
+                if int(self.flags[0].item()):
+                    break
+            run["end"]()
+            if self.graphs is None and self.use_graph:
+                # the eager cycle has loaded and run every kernel once
+                self.graphs = run = self._capture(parts)
             # one read-back per cycle: the true residual, |b|, the tolerance and the step count
             rn, bn, tol, k = self.stat.tolist()
             iters += int(k)

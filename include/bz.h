@@ -346,9 +346,9 @@ int bz_gmres_orthogonalise(double* V, long ldv, int m, int i, double* w, long n,
                            int ldh, double* cs, double* sn, double* g, const double* tol, int* done, int* kdone,
                            hipStream_t stream);
 
-/* r = b - ax (r = b for ax NULL; r may be NULL or ax) and its norm: stat[of], of = 0 for a residual
- * (then also stat[2] = max(atol, rtol stat[1]) and stat[3] = *kdone), of = 1 for |b|.
- * partial: 256 doubles. */
+/* r = b - ax (r = b for ax NULL; r may be NULL or ax) and its norm: of = 0 the residual's, to stat[0]
+ * with stat[3] = *kdone; of = 1 the right-hand side's, to stat[1] with the tolerance
+ * stat[2] = max(atol, rtol stat[1]); of = 2 all of them (r = b).  partial: 256 doubles. */
 int bz_gmres_norm(const double* b, const double* ax, double* r, long n, double* partial, int of, double atol, double rtol,
                   const int* kdone, double* stat, hipStream_t stream);
 

@@ -100,3 +100,17 @@ def test_nothing_moves_once_done():
     ptr = lambda k: __import__("ctypes").c_void_p(flags.data_ptr() + 4 * k)
     _lib.call("bz_gmres_orthogonalise", V, n, m, 2, w, n, 2, t((m + 1) * 256), H, m + 1, cs, sn, gg, tol, ptr(0), ptr(1))
     assert all(torch.equal(x, y) for x, y in zip((V, w, H, cs, sn, gg, flags), before))
+
+
+@pytest.mark.parametrize("nx,nbins", [(1, 1), (7, 3), (200, 30), (4096, 256), (4089, 5)])
+def test_points_grouped_by_bin(nx, nbins):
+    """The stable grouping of points by bin, exactly (whole numbers), with empty bins."""
+    rng = np.random.default_rng(nx)
+    b = rng.integers(0, max(1, nbins - 1), nx)
+    i32 = lambda a: torch.tensor(a, dtype=torch.int32, device="cuda")
+    start, count, order = i32(np.full(nbins, -1)), i32(np.full(nbins, -1)), i32(np.full(nx, -1))
+    _lib.call("bz_group_bins", i32(b), nx, nbins, start, count, order)
+    want = np.bincount(b, minlength=nbins)
+    np.testing.assert_array_equal(count.cpu().numpy(), want)
+    np.testing.assert_array_equal(start.cpu().numpy(), np.cumsum(want) - want)
+    np.testing.assert_array_equal(order.cpu().numpy(), np.argsort(b, kind="stable"))
