@@ -204,7 +204,22 @@ __global__ void k_ee_potentials(const double* __restrict__ H, const double* __re
     const double* Hr = H + ((long)s * npr + r) * npr;
     const double* Gr = G + ((long)s * npr + r) * npr;
     double sh = 0.0, sg = 0.0;
-    for (int k = 0; k < npr; ++k) {
+    int k = 0;
+    for (; k + 8 <= npr; k += 8) {                     // the loads of eight terms together
+      double xv[8], hk[8], gk[8];
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        xv[u] = x[(long)((k + u) * ns + s) * B + b];
+        hk[u] = Hr[k + u];
+        gk[u] = Gr[k + u];
+      }
+#pragma unroll
+      for (int u = 0; u < 8; ++u) {
+        sh = fma(hk[u], xv[u], sh);
+        sg = fma(gk[u], xv[u], sg);
+      }
+    }
+    for (; k < npr; ++k) {
       const double xv = x[(long)(k * ns + s) * B + b];
       sh = fma(Hr[k], xv, sh);
       sg = fma(Gr[k], xv, sg);
@@ -265,11 +280,13 @@ __global__ __launch_bounds__(256) void k_ee_t2(int npr, int B, const double* __r
                                                const double* __restrict__ hv, const double* __restrict__ gv,
                                                const double* __restrict__ negam, const int* __restrict__ active,
                                                double* __restrict__ t2) {
-  // one workgroup: radial row p, 256 instances; the tensor blocks of row p for one q at a
-  // time in LDS (read by every thread), the instance's potentials at r = p-3..p+3 in registers
+  // one workgroup: radial row p, harmonic q, 256 instances; the tensor blocks of (p, q) in LDS
+  // (read by every thread), the instance's potentials at r = p-3..p+3 in registers.  With q in the
+  // grid a batch of up to 256 instances has npr NS workgroups instead of npr, each with one of the
+  // NS serial sums.
   constexpr int NC2 = NS * NS, NC = NS * NS * NS;
   __shared__ double SA[49 * NC2], SB[49 * NC2];
-  const int p = blockIdx.y, tid = threadIdx.x;
+  const int p = blockIdx.y, q = blockIdx.z, tid = threadIdx.x;
   const int inst = blockIdx.x * 256 + tid;
   const int n = NS * npr;
   const bool ok = inst < B && (!active || active[inst]);
@@ -285,39 +302,36 @@ __global__ __launch_bounds__(256) void k_ee_t2(int npr, int B, const double* __r
     }
   }
   const double ng = ok ? negam[inst] : 0.0;
-  for (int q = 0; q < NS; ++q) {
-    __syncthreads();
-    for (int e = tid; e < 49 * NC2; e += 256) {
-      const int dkdr = e / NC2, ls = e - dkdr * NC2;
-      const long src = ((long)p * 49 + dkdr) * NC + q * NC2 + ls;
-      SA[e] = ccA[src];
-      SB[e] = ccB[src];
-    }
-    __syncthreads();
-    if (!ok) continue;
-    double sum = 0.0;
-#pragma unroll
-    for (int dk = 0; dk < 7; ++dk) {
-      const int k = p + dk - 3;
-      if (k < 0 || k >= npr) continue;
-#pragma unroll
-      for (int l = 0; l < NS; ++l) {
-        const double xv = x[(long)(k * NS + l) * B + inst];
-        double a = 0.0;
-#pragma unroll
-        for (int dr = 0; dr < 7; ++dr) {
-#pragma unroll
-          for (int ss = 0; ss < NS; ++ss) {
-            const int e = (dk * 7 + dr) * NC2 + l * NS + ss;
-            a = fma(SA[e], h[dr][ss], a);
-            a = fma(SB[e], g[dr][ss], a);
-          }
-        }
-        sum = fma(a, xv, sum);
-      }
-    }
-    t2[(long)inst * n + p * NS + q] = ng * sum;
+  for (int e = tid; e < 49 * NC2; e += 256) {
+    const int dkdr = e / NC2, ls = e - dkdr * NC2;
+    const long src = ((long)p * 49 + dkdr) * NC + q * NC2 + ls;
+    SA[e] = ccA[src];
+    SB[e] = ccB[src];
   }
+  __syncthreads();
+  if (!ok) return;
+  double sum = 0.0;
+#pragma unroll
+  for (int dk = 0; dk < 7; ++dk) {
+    const int k = p + dk - 3;
+    if (k < 0 || k >= npr) continue;
+#pragma unroll
+    for (int l = 0; l < NS; ++l) {
+      const double xv = x[(long)(k * NS + l) * B + inst];
+      double a = 0.0;
+#pragma unroll
+      for (int dr = 0; dr < 7; ++dr) {
+#pragma unroll
+        for (int ss = 0; ss < NS; ++ss) {
+          const int e = (dk * 7 + dr) * NC2 + l * NS + ss;
+          a = fma(SA[e], h[dr][ss], a);
+          a = fma(SB[e], g[dr][ss], a);
+        }
+      }
+      sum = fma(a, xv, sum);
+    }
+  }
+  t2[(long)inst * n + p * NS + q] = ng * sum;
 }
 
 // negam[b] = ne[b] * gamma_a(x_b): m0 = c_m0 (mass . x), kT = |c_kt (top . x) / m0|,
@@ -414,7 +428,7 @@ int bz_ee_potentials_cols(const double* H, const double* G, int ns, int npr, con
 int bz_ee_jacobian_t2(int ns, int npr, int B, const double* ccA, const double* ccB, const double* x, const double* hv,
                       const double* gv, const double* negam, const int* active, double* t2, hipStream_t stream) {
   if (ns < 1 || ns > 5 || npr < 1 || B < 1 || !ccA || !ccB || !x || !hv || !gv || !negam || !t2) return BZ_EINVAL;
-  const dim3 grid((B + 255) / 256, npr);
+  const dim3 grid((B + 255) / 256, npr, ns);
   switch (ns) {
     case 1: hipLaunchKernelGGL(k_ee_t2<1>, grid, dim3(256), 0, stream, npr, B, ccA, ccB, x, hv, gv, negam, active, t2); break;
     case 2: hipLaunchKernelGGL(k_ee_t2<2>, grid, dim3(256), 0, stream, npr, B, ccA, ccB, x, hv, gv, negam, active, t2); break;

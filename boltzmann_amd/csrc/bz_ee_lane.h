@@ -45,28 +45,54 @@ __device__ void flat_matvec(int P, const double* __restrict__ kp, const unsigned
 // (d = 0 entry stored inverted, out-of-band entries zero) held in LDS; lanes
 // 0..ns-1 each own one block and carry the last three values in registers.
 __device__ void lane_mass_solve(int ns, int npr, const double* __restrict__ lc, double* __restrict__ b, int lane) {
+  // the LDS operands of U rows are read together, ahead of the recurrence
+  constexpr int U = 4;
   if (lane < ns) {
     const int l = lane;
     double y1 = 0.0, y2 = 0.0, y3 = 0.0;
-    for (int q = 0; q < npr; ++q) {
-      const double* L = lc + q * 4;
-      double s = b[q * ns + l];
-      s = fma(-L[1], y1, s);
-      s = fma(-L[2], y2, s);
-      s = fma(-L[3], y3, s);
-      const double y = s * L[0];
-      b[q * ns + l] = y;
-      y3 = y2; y2 = y1; y1 = y;
+    for (int q0 = 0; q0 < npr; q0 += U) {
+      double v[U], L[U][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = min(q0 + u, npr - 1);
+        v[u] = b[q * ns + l];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) L[u][d] = lc[q * 4 + d];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+        if (q0 + u < npr) {
+          double s = fma(-L[u][1], y1, v[u]);
+          s = fma(-L[u][2], y2, s);
+          s = fma(-L[u][3], y3, s);
+          const double y = s * L[u][0];
+          b[(q0 + u) * ns + l] = y;
+          y3 = y2; y2 = y1; y1 = y;
+        }
     }
     double z1 = 0.0, z2 = 0.0, z3 = 0.0;
-    for (int q = npr - 1; q >= 0; --q) {
-      double s = b[q * ns + l];
-      if (q + 1 < npr) s = fma(-lc[(q + 1) * 4 + 1], z1, s);
-      if (q + 2 < npr) s = fma(-lc[(q + 2) * 4 + 2], z2, s);
-      if (q + 3 < npr) s = fma(-lc[(q + 3) * 4 + 3], z3, s);
-      const double z = s * lc[q * 4];
-      b[q * ns + l] = z;
-      z3 = z2; z2 = z1; z1 = z;
+    for (int q0 = npr - 1; q0 >= 0; q0 -= U) {
+      double v[U], L[U][4];
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = max(q0 - u, 0);
+        v[u] = b[q * ns + l];
+#pragma unroll
+        for (int d = 0; d < 4; ++d) L[u][d] = lc[min(q + d, npr - 1) * 4 + d];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) {
+        const int q = q0 - u;
+        if (q >= 0) {
+          double s = v[u];
+          if (q + 1 < npr) s = fma(-L[u][1], z1, s);
+          if (q + 2 < npr) s = fma(-L[u][2], z2, s);
+          if (q + 3 < npr) s = fma(-L[u][3], z3, s);
+          const double z = s * L[u][0];
+          b[q * ns + l] = z;
+          z3 = z2; z2 = z1; z1 = z;
+        }
+      }
     }
   }
 }
@@ -663,11 +689,17 @@ __global__ __launch_bounds__(64) void k_ee_precond_apply(GridDev g, BatchDev b, 
   for (int i = lane; i <= n; i += 64) PO[i] = g.prof_off[i];
   __syncthreads();
   lane_mass_matvec(n, g.ns, mprof, g.first_col, g.prof_off, VV, Y2, lane);
-  // rows [r0, r_end(r0)) fit one stage (every row has at most LBUF entries: checked at launch)
+  // rows [r0, r_end(r0)) fit one stage (every row has at most LBUF entries: checked at launch); 64
+  // candidate ends are tested at once (the offsets increase)
   auto r_end = [&](int r0) {
+    const int limit = PO[r0] + LBUF;
     int r1 = r0 + 1;
-    while (r1 < n && PO[r1 + 1] - PO[r0] <= LBUF) ++r1;
-    return r1;
+    while (true) {
+      const int e = r1 + 1 + lane;
+      const unsigned long long fit = __builtin_amdgcn_ballot_w64(e <= n && PO[min(e, n)] <= limit);
+      r1 += __builtin_popcountll(fit);
+      if (fit != ~0ull) return r1;
+    }
   };
   double reg[PER];
   int r0 = 0, r1 = r_end(0), st = 0;
@@ -714,14 +746,39 @@ __global__ __launch_bounds__(64) void k_ee_precond_apply(GridDev g, BatchDev b, 
       const int fc = act ? (int)FC[i] : 0;
       const int off = act ? PO[i] - base - fc : 0;
       double acc = act ? Y2[i] : 0.0;
-      if (act)
-        for (int j = fc; j < blk0; ++j) acc = fma(-S[off + j], Y2[j], acc);
-      for (int t = 0; t < nb; ++t) {
-        const int j = blk0 + t;
-        const int lo = __builtin_amdgcn_readlane(__double2loint(acc), t);
-        const int hi = __builtin_amdgcn_readlane(__double2hiint(acc), t);
-        const double yj = __hiloint2double(hi, lo);
-        if (act && i > j && j >= fc) acc = fma(-S[off + j], yj, acc);
+      // In both, the LDS operands of eight columns are read together: the columns stay in order,
+      // and only the arithmetic of one step waits for the step before.
+      constexpr int U = 8;
+      if (act) {
+        int j = fc;
+        for (; j + U <= blk0; j += U) {
+          double sj[U], yj[U];
+#pragma unroll
+          for (int u = 0; u < U; ++u) {
+            sj[u] = S[off + j + u];
+            yj[u] = Y2[j + u];
+          }
+#pragma unroll
+          for (int u = 0; u < U; ++u) acc = fma(-sj[u], yj[u], acc);
+        }
+        for (; j < blk0; ++j) acc = fma(-S[off + j], Y2[j], acc);
+      }
+      for (int t0 = 0; t0 < nb; t0 += U) {
+        double sj[U];
+        bool in[U];
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int j = blk0 + t0 + u;
+          in[u] = act && i > j && j >= fc;
+          sj[u] = S[in[u] ? off + j : 0];
+        }
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          const int lo = __builtin_amdgcn_readlane(__double2loint(acc), t0 + u);
+          const int hi = __builtin_amdgcn_readlane(__double2hiint(acc), t0 + u);
+          const double next = fma(-sj[u], __hiloint2double(hi, lo), acc);
+          acc = in[u] ? next : acc;
+        }
       }
       if (act) Y2[i] = acc;
       __syncthreads();

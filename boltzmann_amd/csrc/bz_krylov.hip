@@ -444,14 +444,35 @@ __global__ __launch_bounds__(64) void k_arnoldi_batched(int n, int B, int m, int
   for (int j = lane; j <= i + 1; j += 64) HC[j] = 0.0;
   __syncthreads();
   for (int rep = 0; rep < 2; ++rep) {
-    for (int j = 0; j <= i; ++j) {
-      const double d = wdot(V + ((size_t)j * B + inst) * n, W, n);
-      if (lane == 0) { T[j] = d; HC[j] += d; }
+    // four dot products side by side (each in the order of wdot): their loads and their sums
+    // across the wavefront overlap
+    for (int j0 = 0; j0 <= i; j0 += 4) {
+      double s[4] = {0.0, 0.0, 0.0, 0.0};
+      for (int e = lane; e < n; e += 64) {
+        double vj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vj[u] = V[((size_t)min(j0 + u, i) * B + inst) * n + e];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s[u] = fma(vj[u], W[e], s[u]);
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) s[u] = bz::wave_sum(s[u]);
+#pragma unroll
+      for (int u = 0; u < 4; ++u)
+        if (lane == 0 && j0 + u <= i) { T[j0 + u] = s[u]; HC[j0 + u] += s[u]; }
     }
     __syncthreads();
     for (int e = lane; e < n; e += 64) {
       double s = W[e];
-      for (int j = 0; j <= i; ++j) s = fma(-T[j], V[((size_t)j * B + inst) * n + e], s);
+      int j = 0;
+      for (; j + 4 <= i + 1; j += 4) {
+        double vj[4];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) vj[u] = V[((size_t)(j + u) * B + inst) * n + e];
+#pragma unroll
+        for (int u = 0; u < 4; ++u) s = fma(-T[j + u], vj[u], s);
+      }
+      for (; j <= i; ++j) s = fma(-T[j], V[((size_t)j * B + inst) * n + e], s);
       W[e] = s;
     }
     __syncthreads();
