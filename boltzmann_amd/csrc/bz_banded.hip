@@ -56,6 +56,16 @@ __device__ __forceinline__ void adv_speed(const SweepArgs& a, int s, double& av,
   }
 }
 
+constexpr int kOutside = 0x40000000;               // past the end of every output buffer
+typedef unsigned v2u __attribute__((ext_vector_type(2)));
+
+__device__ __forceinline__ void out_store(const __amdgpu_buffer_rsrc_t& b, int byte, double v) {
+  v2u w;
+  w.x = (unsigned)__double2loint(v);
+  w.y = (unsigned)__double2hiint(v);
+  __builtin_amdgcn_raw_buffer_store_b64(w, b, byte, 0, 0);
+}
+
 // The order of LDS operations within the one wavefront of a workgroup.
 __device__ __forceinline__ void tile_fence() {
   __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
@@ -74,7 +84,7 @@ __device__ __forceinline__ void tile_fence() {
 // storing in turn: 16 x 100 radial lines of 671 points, x and angular lines of the same state,
 // 650 -> 118 us together; 20000 systems of 259, four diagonals, two solves, a product and a
 // bidiagonal solve 909 -> 281 us.
-template <int KIND, int ND>
+template <int KIND, int ND, bool LONG>
 __global__ __launch_bounds__(TS) void k_sweep(SweepArgs a) {
   constexpr bool BIDIAG = (KIND == K_BIDIAG || KIND == K_XSTEP);
   constexpr bool ADV = !BIDIAG && KIND != K_BANDED;
@@ -140,8 +150,17 @@ __global__ __launch_bounds__(TS) void k_sweep(SweepArgs a) {
 #pragma unroll
   for (int d = 0; d < (ND > 1 ? ND - 1 : 1); ++d) y[d] = 0.0;
 
+  // Results past the end of a line or of the batch fall outside the buffer and are dropped: with a
+  // branch for each store the compiler could not count the stores in flight and waited for all of
+  // them before the next chunk.  (LONG: lines whose 64 rows pass the buffer's 2^30 bytes.)
+  const __amdgpu_buffer_rsrc_t out = __builtin_amdgcn_make_buffer_rsrc(
+      a.out + (size_t)sys0 * N, 0, LONG ? 0 : min(TS, a.bsz - sys0) * N * 8, 0x00020000);
+
   const int nchunk = (N + CH - 1) / CH;
   fetch(0);
+  // the first loads complete here, so that the waits inside the loop count only its own
+  __builtin_amdgcn_sched_barrier(0);
+  __builtin_amdgcn_s_waitcnt(0x0F70);
   for (int k = 0; k < nchunk; ++k) {
     const int p = k * CH + lo;
 #pragma unroll
@@ -158,11 +177,20 @@ __global__ __launch_bounds__(TS) void k_sweep(SweepArgs a) {
         if (lane + TS * i < NTD) td[lane + TS * i] = D[i];
     }
     tile_fence();
-    if (k + 1 < nchunk) fetch(k + 1);
+    fetch(k + 1);                       // past the last chunk: the last position again, not used
     const double* mt = td + (fwd ? CH * ND : 0);
+    // The right-hand sides all at once (results go into the same tile) and, for the advection
+    // lines, the coefficients off the recurrence.
+    double rhs[CH], rden[ADV ? CH : 1];
+#pragma unroll
+    for (int q = 0; q < CH; ++q) rhs[q] = tb[lane * ST + q];
+    if constexpr (ADV) {
+#pragma unroll
+      for (int q = 0; q < CH; ++q) rden[q] = 1.0 / fma(t, mt[q * ND], 1.0);
+    }
 #pragma unroll
     for (int q = 0; q < CH; ++q) {
-      const double bi = tb[lane * ST + q];
+      const double bi = rhs[q];
       double val;
       if constexpr (BIDIAG) {
         const double sv = tc[(TS + lane) * ST + q] * y[0];
@@ -176,7 +204,7 @@ __global__ __launch_bounds__(TS) void k_sweep(SweepArgs a) {
         double sv = 0.0;
 #pragma unroll
         for (int d = ND - 1; d >= 1; --d) sv = fma(mt[q * ND + d], y[d - 1], sv);
-        val = fma(-t, sv, bi) * (1.0 / fma(t, mt[q * ND], 1.0));
+        val = fma(-t, sv, bi) * rden[q];
       }
 #pragma unroll
       for (int d = (ND > 1 ? ND - 2 : 0); d >= 1; --d) y[d] = y[d - 1];
@@ -184,11 +212,19 @@ __global__ __launch_bounds__(TS) void k_sweep(SweepArgs a) {
       tb[lane * ST + q] = val;
     }
     tile_fence();
+    double v[CH];
+#pragma unroll
+    for (int u = 0; u < CH; ++u) v[u] = tb[(u * RP + lr) * ST + lo];
 #pragma unroll
     for (int u = 0; u < CH; ++u) {
       const int r = u * RP + lr;
       const bool f = (KIND == K_BANDED || KIND == K_BIDIAG) ? fwd : ((dirs >> r) & 1) != 0;
-      if (p < N && sys0 + r < a.bsz) a.out[(size_t)(sys0 + r) * N + (f ? p : N - 1 - p)] = tb[r * ST + lo];
+      const int c = f ? p : N - 1 - p;
+      if constexpr (!LONG) {
+        out_store(out, p < N ? 8 * (r * N + c) : kOutside, v[u]);
+      } else if (p < N && sys0 + r < a.bsz) {
+        a.out[(size_t)(sys0 + r) * N + c] = v[u];
+      }
     }
     tile_fence();
   }
@@ -253,18 +289,24 @@ __global__ __launch_bounds__(64) void k_xstep_scan(const double* __restrict__ di
   }
 }
 
+template <int KIND, int ND>
+void launch_one(const SweepArgs& a, hipStream_t st) {
+  const dim3 grid((a.bsz + TS - 1) / TS), block(TS);
+  if (a.N < (1 << 20)) hipLaunchKernelGGL((k_sweep<KIND, ND, false>), grid, block, 0, st, a);
+  else hipLaunchKernelGGL((k_sweep<KIND, ND, true>), grid, block, 0, st, a);
+}
+
 template <int KIND>
 int launch_sweep(const SweepArgs& a, int nd, hipStream_t st) {
-  const dim3 grid((a.bsz + TS - 1) / TS), block(TS);
   switch (nd) {
-    case 1: hipLaunchKernelGGL((k_sweep<KIND, 1>), grid, block, 0, st, a); break;
-    case 2: hipLaunchKernelGGL((k_sweep<KIND, 2>), grid, block, 0, st, a); break;
-    case 3: hipLaunchKernelGGL((k_sweep<KIND, 3>), grid, block, 0, st, a); break;
-    case 4: hipLaunchKernelGGL((k_sweep<KIND, 4>), grid, block, 0, st, a); break;
-    case 5: hipLaunchKernelGGL((k_sweep<KIND, 5>), grid, block, 0, st, a); break;
-    case 6: hipLaunchKernelGGL((k_sweep<KIND, 6>), grid, block, 0, st, a); break;
-    case 7: hipLaunchKernelGGL((k_sweep<KIND, 7>), grid, block, 0, st, a); break;
-    case 8: hipLaunchKernelGGL((k_sweep<KIND, 8>), grid, block, 0, st, a); break;
+    case 1: launch_one<KIND, 1>(a, st); break;
+    case 2: launch_one<KIND, 2>(a, st); break;
+    case 3: launch_one<KIND, 3>(a, st); break;
+    case 4: launch_one<KIND, 4>(a, st); break;
+    case 5: launch_one<KIND, 5>(a, st); break;
+    case 6: launch_one<KIND, 6>(a, st); break;
+    case 7: launch_one<KIND, 7>(a, st); break;
+    case 8: launch_one<KIND, 8>(a, st); break;
     default: return BZ_EINVAL;
   }
   BZ_LAUNCH_CHECK();
@@ -273,7 +315,7 @@ int launch_sweep(const SweepArgs& a, int nd, hipStream_t st) {
 
 template <int KIND>
 int launch_bidiag(const SweepArgs& a, hipStream_t st) {
-  hipLaunchKernelGGL((k_sweep<KIND, 2>), dim3((a.bsz + TS - 1) / TS), dim3(TS), 0, st, a);
+  launch_one<KIND, 2>(a, st);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }

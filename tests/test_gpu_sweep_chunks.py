@@ -114,3 +114,14 @@ def test_long_x_lines():
     _lib.call("bz_xstep_bidiag_solve", _dev(diag), _dev(sub), torch.tensor(low, dtype=torch.int32, device="cuda"),
               _dev(b), out, Nr, Nvt, Nx)
     _close(out, ref, 2)
+
+
+def test_very_long_lines():
+    """Lines too long for the 32-bit offsets of a workgroup's results."""
+    from scipy.linalg import solve_banded
+    N = (1 << 20) + 3
+    rng = np.random.default_rng(9)
+    diag, sub, b = rng.uniform(1.0, 2.0, (2, N)), rng.uniform(-0.5, 0.5, (2, N - 1)), rng.normal(size=(2, N))
+    x = rawkernel.bidiagonal_solve_batched(_dev(diag), _dev(sub), _dev(b), True)
+    ref = np.stack([solve_banded((1, 0), np.stack([diag[s], np.append(sub[s], 0.0)]), b[s]) for s in range(2)])
+    _close(x, ref, 2)
