@@ -15,28 +15,30 @@
 
 namespace {
 
-// y = K x over the flat profile: entries are lane-strided (coalesced loads, no
-// dependence between iterations) and accumulated into y[row] with LDS atomics.  Groups of
-// U entries per lane issue all their loads before the first atomic, so a group waits on
-// memory once.  y must be zeroed and synchronised by the caller.
-__device__ void flat_matvec(int P, const double* __restrict__ kp, const unsigned* __restrict__ rc,
-                            const double* __restrict__ x, double* y, int lane) {
+// y += K x, lane t on rows t, t + 64, ...: each row's products are rounded and added to y one by
+// one in the order of its columns, eight entries' loads in flight.  (Adding lane-strided entries
+// into y with LDS atomics kept the loads coalesced, but most of the 64 lanes met in one or two
+// rows.)
+__device__ void row_matvec(int n, const double* __restrict__ kp, const int* __restrict__ first_col,
+                           const int* __restrict__ poff, const double* __restrict__ x, double* y, int lane) {
+#pragma clang fp contract(off)
   constexpr int U = 8;
-  int e0 = lane;
-  for (; e0 + 64 * (U - 1) < P; e0 += 64 * U) {
-    unsigned v[U];
-    double a[U];
+  for (int i = lane; i < n; i += 64) {
+    const int p0 = poff[i], len = poff[i + 1] - p0, fc = first_col[i];
+    double s = y[i];
+    int e = 0;
+    for (; e + U <= len; e += U) {
+      double a[U], v[U];
 #pragma unroll
-    for (int u = 0; u < U; ++u) {
-      v[u] = rc[e0 + 64 * u];
-      a[u] = kp[e0 + 64 * u];
+      for (int u = 0; u < U; ++u) {
+        a[u] = kp[p0 + e + u];
+        v[u] = x[fc + e + u];
+      }
+#pragma unroll
+      for (int u = 0; u < U; ++u) s = s + a[u] * v[u];
     }
-#pragma unroll
-    for (int u = 0; u < U; ++u) atomicAdd(&y[v[u] >> 16], a[u] * x[v[u] & 0xffffu]);
-  }
-  for (int e = e0; e < P; e += 64) {
-    const unsigned v = rc[e];
-    atomicAdd(&y[v >> 16], kp[e] * x[v & 0xffffu]);
+    for (; e < len; ++e) s = s + kp[p0 + e] * x[fc + e];
+    y[i] = s;
   }
 }
 
@@ -45,54 +47,28 @@ __device__ void flat_matvec(int P, const double* __restrict__ kp, const unsigned
 // (d = 0 entry stored inverted, out-of-band entries zero) held in LDS; lanes
 // 0..ns-1 each own one block and carry the last three values in registers.
 __device__ void lane_mass_solve(int ns, int npr, const double* __restrict__ lc, double* __restrict__ b, int lane) {
-  // the LDS operands of U rows are read together, ahead of the recurrence
-  constexpr int U = 4;
   if (lane < ns) {
     const int l = lane;
     double y1 = 0.0, y2 = 0.0, y3 = 0.0;
-    for (int q0 = 0; q0 < npr; q0 += U) {
-      double v[U], L[U][4];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = min(q0 + u, npr - 1);
-        v[u] = b[q * ns + l];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) L[u][d] = lc[q * 4 + d];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u)
-        if (q0 + u < npr) {
-          double s = fma(-L[u][1], y1, v[u]);
-          s = fma(-L[u][2], y2, s);
-          s = fma(-L[u][3], y3, s);
-          const double y = s * L[u][0];
-          b[(q0 + u) * ns + l] = y;
-          y3 = y2; y2 = y1; y1 = y;
-        }
+    for (int q = 0; q < npr; ++q) {
+      const double* L = lc + q * 4;
+      double s = b[q * ns + l];
+      s = fma(-L[1], y1, s);
+      s = fma(-L[2], y2, s);
+      s = fma(-L[3], y3, s);
+      const double y = s * L[0];
+      b[q * ns + l] = y;
+      y3 = y2; y2 = y1; y1 = y;
     }
     double z1 = 0.0, z2 = 0.0, z3 = 0.0;
-    for (int q0 = npr - 1; q0 >= 0; q0 -= U) {
-      double v[U], L[U][4];
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = max(q0 - u, 0);
-        v[u] = b[q * ns + l];
-#pragma unroll
-        for (int d = 0; d < 4; ++d) L[u][d] = lc[min(q + d, npr - 1) * 4 + d];
-      }
-#pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const int q = q0 - u;
-        if (q >= 0) {
-          double s = v[u];
-          if (q + 1 < npr) s = fma(-L[u][1], z1, s);
-          if (q + 2 < npr) s = fma(-L[u][2], z2, s);
-          if (q + 3 < npr) s = fma(-L[u][3], z3, s);
-          const double z = s * L[u][0];
-          b[q * ns + l] = z;
-          z3 = z2; z2 = z1; z1 = z;
-        }
-      }
+    for (int q = npr - 1; q >= 0; --q) {
+      double s = b[q * ns + l];
+      if (q + 1 < npr) s = fma(-lc[(q + 1) * 4 + 1], z1, s);
+      if (q + 2 < npr) s = fma(-lc[(q + 2) * 4 + 2], z2, s);
+      if (q + 3 < npr) s = fma(-lc[(q + 3) * 4 + 3], z3, s);
+      const double z = s * lc[q * 4];
+      b[q * ns + l] = z;
+      z3 = z2; z2 = z1; z1 = z;
     }
   }
 }
@@ -360,18 +336,29 @@ __device__ void back_substitute(int n, const double* __restrict__ urows, int WP,
     }
     if (lane < NRHS) {
       const int j0 = c * CH;
+      // the next row's operands are read before this row's result is stored
+      double u0[W], u1[W], y0 = Y[min(j0 + CH - 1, n - 1)], y1 = 0.0;
+#pragma unroll
+      for (int k = 0; k < W; ++k) u0[k] = stg[(CH - 1) * WP + k];
 #pragma unroll
       for (int tt = CH - 1; tt >= 0; --tt) {
         const int j = j0 + tt;
-        if (j < n) {
-          const lds_double* ur = stg + tt * WP;
-          double sum = Y[j];
+        if (tt > 0) {
+          y1 = Y[min(j - 1, n - 1)];
 #pragma unroll
-          for (int k = W - 1; k >= 1; --k) sum = fma(-ur[k], z[(tt + k) % W], sum);
-          const double zj = sum * ur[0];
+          for (int k = 0; k < W; ++k) u1[k] = stg[(tt - 1) * WP + k];
+        }
+        if (j < n) {
+          double sum = y0;
+#pragma unroll
+          for (int k = W - 1; k >= 1; --k) sum = fma(-u0[k], z[(tt + k) % W], sum);
+          const double zj = sum * u0[0];
           z[tt % W] = zj;
           Y[j] = zj;
         }
+        y0 = y1;
+#pragma unroll
+        for (int k = 0; k < W; ++k) u0[k] = u1[k];
       }
     }
     __syncthreads();

@@ -58,7 +58,7 @@ __global__ __launch_bounds__(64) void k_ee_apply(GridDev g, BatchDev b, int mode
   }
   lane_stage_mass(g, LCH, lane);
   __syncthreads();
-  flat_matvec(g.P, kprof, g.ent_rc, V, AV, lane);                 // (K_x - mu M) v (+ T2 v)
+  row_matvec(n, kprof, g.first_col, g.prof_off, V, AV, lane);     // (K_x - mu M) v (+ T2 v)
   __syncthreads();
   lane_mass_solve(g.ns, g.npr, LCH, AV, lane);                    // M^-1 (...)
   __syncthreads();
@@ -297,12 +297,8 @@ int bz_ee_newton_residual(const bz_grid0d_t* gp, const bz_batch0d_t* bp, const b
   if (ep->ns != g.ns || ep->npr != g.npr || !ep->ccA || !ep->ccB || !ep->h || !ep->g || !ep->negam) return BZ_EINVAL;
   if ((ep->h_lo == nullptr) != (ep->g_lo == nullptr)) return BZ_EINVAL;
   EEDev e{ep->ccA, ep->ccB, ep->h, ep->g, ep->negam, ep->h_lo, ep->g_lo};
-  const long work = (long)b.B * g.P;
-  const int blocks = (int)std::min<long>((work + 255) / 256, 8192);
-  hipLaunchKernelGGL(k_prepare0d, dim3(blocks), dim3(256), 0, stream, g, b);
-  BZ_LAUNCH_CHECK();
-  hipLaunchKernelGGL(k_ee_profile_add, dim3(blocks), dim3(256), 0, stream, g, b, e);
-  BZ_LAUNCH_CHECK();
+  const int rc = launch_prepare(g, b, stream, &e);
+  if (rc != BZ_OK) return rc;
   hipLaunchKernelGGL(k_ee_mu_shift, dim3(b.B), dim3(64), 0, stream, g, b, mu);
   BZ_LAUNCH_CHECK();
   const size_t lds = (size_t)(3 * g.n + 4 * g.npr) * sizeof(double);
