@@ -741,9 +741,9 @@ def main():
         "roofline": {"bound": "valu", "achieved": achieved, "peak": peak, "unit": "TFLOP/s",
                      "frac": achieved / peak, "traffic": traffic,
                      "hbm_frac": (traffic / (kernel_ms.mean() * 1e-3) / 8e12) if traffic else None,
-                     "kernel": "k_prepare0d + k_newton0d<11,2> (one bz_steady_solve_0d call)",
+                     "kernel": "k_prepare0d + k_newton0d<11,5> (one bz_steady_solve_0d call)",
                      "kernel_ms": float(kernel_ms.mean()),
-                     "note": "FP64 VALU kernel limited by the issue rate of the sequential pivot steps (no MFMA); "
+                     "note": "FP64 kernel limited by its traffic and the chain of its four-pivot blocks (FP64 MFMA); "
                              "peak = MI355X FP64 vector peak 78.6 TFLOP/s; achieved = algorithmic flops of the "
                              "profile-LU Newton iterations run / launch time; hbm_frac = traffic / launch time / 8 TB/s"},
         "reference_equivalent_tflops": float(dense_ref * iters.sum() / (kernel_ms.mean() * 1e-3) / 1e12),

@@ -530,9 +530,8 @@ int bz_glow_fluid_step(const BzGlowFluid* g, int flags, double h, double bc_befo
                        hipStream_t stream);
 
 /* Copies of Dp and Dp Dp_mod (given transposed, as in BzGlowFluid) in the order in which
- * bz_glow_fluid_step's register tiles read them for n points (90 < n <= 200), so that the
- * Jacobian is loaded with coalesced reads; each output holds BZ_GLOW_TILE_LEN doubles.  For
- * n <= 90 the step keeps its row layout and nothing is written.  Set-up, once per n. */
+ * bz_glow_fluid_step's register tiles read them for n points (3 <= n <= 200), so that the Jacobian
+ * is loaded with coalesced reads; each output holds BZ_GLOW_TILE_LEN doubles.  Set-up, once per n. */
 int bz_glow_tile_tables(int n, const double* DpT, const double* DppT, double* DpTile, double* DppTile,
                         hipStream_t stream);
 
