@@ -895,7 +895,7 @@ __global__ __launch_bounds__(256) void k_prepare0d(GridDev g, BatchDev b) {
   // an operator entry is read once for them and the instances' coefficients are scalars.  What
   // bounds it: the bytes of the profiles written, next to about nine FP64 instructions per operator
   // and entry.  A flat loop over all entries with a 64-bit division each took 448 us for 4096
-  // instances of n = 387 (598 MB); the whole solve is 137 us shorter.
+  // instances of n = 387 (598 MB), this 314.
   const int nk = g.nop - 1, S = g.S;
   const int e = blockIdx.x * 256 + threadIdx.x;
   if (e >= g.P + g.n) return;
