@@ -251,23 +251,28 @@ __device__ void rotate_column(double* h, long hs, const double* cs, const double
   g[i + 1] = gn;
   if (fabs(gn) <= tol || hn == 0.0) {
     *kdone = i + 1;
-    *done = 1;
+    __hip_atomic_store(done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
   }
 }
 
 // hn = |w| from the partial sums, V_(i+1) = w / hn (not written when hn = 0); the first workgroup
-// rotates column i of H.  A workgroup that starts after the flag is set skips its part of
-// V_(i+1), which nothing reads then.
+// rotates column i of H and may set the stop flag while others of this launch have not read it yet.
+// So one thread reads it for its workgroup (all of whose wavefronts then agree on the barriers and
+// on hn), and a workgroup that finds it set skips its part of V_(i+1) as a whole: no later step and
+// no solution reads that row.
 __global__ __launch_bounds__(OT) void k_orth_finish(const double* __restrict__ norm_partial, int nblk,
                                                     const double* __restrict__ w, double* __restrict__ Vn, long n,
                                                     double* __restrict__ H, int ldh, int i, double* __restrict__ cs,
                                                     double* __restrict__ sn, double* __restrict__ g,
                                                     const double* __restrict__ tol, int* done, int* kdone) {
-  if (*done) return;
   constexpr int CL = 512;                            // columns up to this length are rotated in LDS
   __shared__ double red[OT / 64], hc[CL], sc[CL], ss[CL];
+  __shared__ int stop;
   double t = 0.0;
   for (int k = threadIdx.x; k < nblk; k += OT) t += norm_partial[k];
+  if (threadIdx.x == 0) stop = __hip_atomic_load(done, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  __syncthreads();
+  if (stop) return;
   const double hn = sqrt(block_sum(t, red));
   if (hn != 0.0)
     for (long e = (long)blockIdx.x * OT + threadIdx.x; e < n; e += (long)gridDim.x * OT) Vn[e] = w[e] / hn;
