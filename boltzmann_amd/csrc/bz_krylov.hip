@@ -373,6 +373,18 @@ __global__ __launch_bounds__(OT) void k_gmres_solution(const double* __restrict_
   }
 }
 
+// x += V y over the first *kdone rows: rows past the last step may hold anything
+__global__ __launch_bounds__(OT) void k_gmres_add(const double* __restrict__ V, long ldv, const double* __restrict__ y,
+                                                  const int* __restrict__ kdone, double* __restrict__ x, long n) {
+  const int k = *kdone;
+  for (long e = (long)blockIdx.x * OT + threadIdx.x; e < n; e += (long)gridDim.x * OT) {
+    double s = 0.0;
+#pragma unroll 4
+    for (int j = 0; j < k; ++j) s = fma(y[j], V[(long)j * ldv + e], s);
+    x[e] += s;
+  }
+}
+
 int orth_blocks(long n, long per) { return (int)std::max<long>(1, std::min<long>(256, (n + per - 1) / per)); }
 
 int grid_for(long n) { return (int)std::min<long>((n + NT - 1) / NT, 8192); }
@@ -620,6 +632,13 @@ int bz_gmres_solution(const double* V, long ldv, int m, const double* H, int ldh
   if (n < 1 || ldv < n || m < 1 || m > 8000 || ldh < m || !V || !H || !g || !kdone || !x) return BZ_EINVAL;
   hipLaunchKernelGGL(k_gmres_solution, dim3(orth_blocks(n, OT) * 2), dim3(OT),
                      (size_t)(m <= 64 ? m + m * m : m) * sizeof(double), stream, V, ldv, H, ldh, g, kdone, x, n, m);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
+int bz_gmres_add(const double* V, long ldv, const double* y, const int* kdone, double* x, long n, hipStream_t stream) {
+  if (n < 1 || ldv < n || !V || !y || !kdone || !x) return BZ_EINVAL;
+  hipLaunchKernelGGL(k_gmres_add, dim3(orth_blocks(n, OT) * 2), dim3(OT), 0, stream, V, ldv, y, kdone, x, n);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }

@@ -197,7 +197,7 @@ class ArnoldiCycle:
         if self.m > 8000:                                           # more rows of y than fit the kernel's LDS
             y = torch.zeros(self.m, dtype=torch.float64, device=self.x.device)
             _lib.call("bz_gmres_back_solve", self.H, self.ldh, self.g, _ptr(self.flags, 1), y, self.m)
-            _lib.call("bz_vt_axpy", self.V, self.n, self.m, y, 1, 1.0, self.x, self.x, self.n)
+            _lib.call("bz_gmres_add", self.V, self.n, y, _ptr(self.flags, 1), self.x, self.n)
             return
         _lib.call("bz_gmres_solution", self.V, self.n, self.m, self.H, self.ldh, self.g, _ptr(self.flags, 1), self.x,
                   self.n)

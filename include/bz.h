@@ -361,6 +361,9 @@ int bz_gmres_begin(const double* r, const double* stat, double* V0, long n, int 
 int bz_gmres_solution(const double* V, long ldv, int m, const double* H, int ldh, const double* g, const int* kdone,
                       double* x, long n, hipStream_t stream);
 
+/* x += sum_{j < *kdone} y_j V_j: the update of a cycle of any length from bz_gmres_back_solve's y. */
+int bz_gmres_add(const double* V, long ldv, const double* y, const int* kdone, double* x, long n, hipStream_t stream);
+
 /* GMRES over B independent systems of size n (one per 0D instance), basis
  * V[(j*B + b)*n + e], j = 0..m (m <= 64).  Arnoldi step i: w (B, n) = A M^-1 V_i; classical
  * Gram-Schmidt twice, V_{i+1}, the Givens-rotated column into R[b][i*m + 0..i], cs, sn
