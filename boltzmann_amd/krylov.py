@@ -17,6 +17,7 @@ the reference does.
 """
 import ctypes
 import gc
+import inspect
 
 import torch
 
@@ -245,11 +246,24 @@ class ArnoldiCycle:
         return False, iters
 
 
+def _with_flag(launch):
+    """A launcher (src, dst, done) of one that takes (src, dst) or already the flag.  Without the
+    flag it overwrites dst in steps past convergence too, which nothing reads."""
+    if launch is None:
+        return None
+    try:
+        inspect.signature(launch).bind(None, None, None)
+        return launch
+    except (TypeError, ValueError):
+        return lambda src, dst, done: launch(src, dst)
+
+
 class DeviceGMRES(ArnoldiCycle):
     """Restarted, right-preconditioned GMRES with the whole Arnoldi step on the device, for an
-    operator and a preconditioner given as launchers `matvec(src, dst, done)` and
-    `precond(src, dst, done)` (device addresses of flat float64 vectors of length n; each writes
-    dst only, and nothing when the device flag `done`, if not None, is set).
+    operator and a preconditioner given as launchers `matvec(src, dst)` and `precond(src, dst)`
+    (device addresses of flat float64 vectors of length n; each writes dst only).  A launcher that
+    takes a third argument is given the device flag `done` and may write nothing when it is set
+    (it is None outside a cycle): steps past convergence then cost their launches only.
 
     The method of utils.gmres_pcr (utils.py:1172-1268: right preconditioning, restart,
     tol = max(atol, rtol |b|)) with the host out of the inner loop: the stop test of a step
@@ -262,7 +276,7 @@ class DeviceGMRES(ArnoldiCycle):
 
     def __init__(self, n, restart, dev, matvec, precond, chunk=4, use_graph=True, gs_passes=2):
         super().__init__(n, restart, dev, chunk, gs_passes, use_graph)
-        self.matvec, self.precond = matvec, precond
+        self.matvec, self.precond = _with_flag(matvec), _with_flag(precond)
 
     def product(self, src, out, done):
         self.precond(src, _at(self.t), done)

@@ -1,0 +1,37 @@
+"""DeviceGMRES with launchers (src, dst): the same system as with launchers that also take the stop
+flag, eagerly and from captured graphs, over several cycles with a last chunk of fewer steps."""
+import pytest
+import torch
+
+from boltzmann_amd import _lib
+from boltzmann_amd.krylov import DeviceGMRES
+
+pytestmark = pytest.mark.gpu
+
+
+@pytest.mark.parametrize("flag", [False, True])
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_two_and_three_arguments(flag, use_graph):
+    """Both products by this library's kernels, which may be captured.  The solver's own residual
+    test bounds the solution: the host's residual differs by rounding, n eps |A| |x|."""
+    n, restart = 300, 6
+    print(f"case: flag={flag} graph={use_graph}", flush=True)
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    f64 = dict(dtype=torch.float64, device="cuda")
+    A = torch.eye(n, **f64) + 0.5 / n ** 0.5 * torch.randn((n, n), generator=gen, **f64)
+    P = 0.5 * torch.eye(n, **f64)
+    matvec = lambda src, dst: _lib.call("bz_dgemm_nn", A, n, n, src, 1, dst)
+    precond = lambda src, dst: _lib.call("bz_dgemm_nn", P, n, n, src, 1, dst)
+    if flag:
+        mv, pc = lambda src, dst, done: matvec(src, dst), lambda src, dst, done: precond(src, dst)
+    else:
+        mv, pc = matvec, precond
+    s = DeviceGMRES(n, restart, torch.device("cuda"), mv, pc, use_graph=use_graph)
+    for rep, tol in enumerate((1e-8, 1e-5, 1e-9)):
+        b = torch.randn(n, generator=gen, **f64)
+        x0 = None if rep != 1 else torch.randn(n, generator=gen, **f64)
+        seen = []
+        x, k = s.solve(b, 0.0, tol, 50, x0=x0, callback=seen.append)
+        r = torch.linalg.vector_norm(A.cpu() @ x.cpu() - b.cpu()) / torch.linalg.vector_norm(b.cpu())
+        assert float(r) < 1.01 * tol and seen[-1] < tol
+        assert len(seen) >= 2 and restart < k <= restart * len(seen)
