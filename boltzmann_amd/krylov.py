@@ -239,7 +239,7 @@ class ArnoldiCycle:
             # one read-back per cycle: the true residual, |b|, the tolerance and the step count
             rn, bn, tol, k = self.stat.tolist()
             iters += int(k)
-            if callback is not None:
+            if callback is not None and k > 0:                     # not for a start that is already converged
                 callback(rn / bn if bn > 0 else 0.0)
             if rn < tol:
                 return True, iters

@@ -35,3 +35,23 @@ def test_two_and_three_arguments(flag, use_graph):
         r = torch.linalg.vector_norm(A.cpu() @ x.cpu() - b.cpu()) / torch.linalg.vector_norm(b.cpu())
         assert float(r) < 1.01 * tol and seen[-1] < tol
         assert len(seen) >= 2 and restart < k <= restart * len(seen)
+
+
+@pytest.mark.parametrize("use_graph", [False, True])
+def test_no_callback_for_a_converged_start(use_graph):
+    """One call per cycle that was run: none where |b - A P x0| is below the tolerance."""
+    n = 40
+    f64 = dict(dtype=torch.float64, device="cuda")
+    A = 2.0 * torch.eye(n, **f64)
+    P = torch.eye(n, **f64)
+    s = DeviceGMRES(n, 3, torch.device("cuda"), lambda a, b: _lib.call("bz_dgemm_nn", A, n, n, a, 1, b),
+                    lambda a, b: _lib.call("bz_dgemm_nn", P, n, n, a, 1, b), use_graph=use_graph)
+    b = torch.arange(1.0, n + 1, **f64)
+    seen = []
+    for x0, calls, steps in ((None, 1, 1), (0.5 * b, 0, 0), (b, 1, 1), (0.5 * b, 0, 0)):
+        del seen[:]
+        x, k = s.solve(b, 0.0, 1e-12, 5, x0=x0, callback=seen.append)
+        assert (len(seen), k) == (calls, steps)
+        assert torch.equal(x, 0.5 * b) or float((x - 0.5 * b).abs().max()) < 1e-12 * n
+    x, k = s.solve(0.0 * b, 1e-3, 0.0, 5, callback=seen.append)
+    assert k == 0 and not bool(x.any()) and len(seen) == 0
