@@ -407,14 +407,14 @@ __global__ __launch_bounds__(SWT) void k_fvm_sweep(BzFvm1d3v op, const double* _
 // (upwind, 1 + av dt D_0 >= 1 in the direction of the sweep), so the re-association changes the
 // result at rounding level.  A workgroup holds SB systems (consecutive x) times NSEG segments.
 // What bounds it is the instructions and latency of one thread, with less than a wavefront per
-// SIMD: so pass 2 reuses the coefficients of pass 1 (one division per position) and addresses are
-// 32-bit offsets.  64 segments of half the length were slower (their maps and coefficients do not
-// fit the registers of a 512-thread workgroup).  Measured at 671 x 16 x 100: 18.7 -> 15.8 us.
+// SIMD: so pass 2 reuses the loads and the one division of pass 1 and addresses are 32-bit
+// offsets.  64 segments of half the length were slower (their maps and coefficients do not fit the
+// registers of a 512-thread workgroup).  Measured at 671 x 16 x 100: 18.7 -> 15.8 us.
 constexpr int SCAN_SB = 8, NSEG = 32;
 
 // MAXL > 0: a segment has at most MAXL positions; its loads (right-hand sides and stencil weights,
-// from clamped in-bounds positions) are issued eight positions at a time and the coefficients stay
-// in registers for pass 2; the MAXL = 0 form loads one position at a time, twice.
+// from clamped in-bounds positions) are issued eight positions at a time and stay, with the
+// reciprocals, in registers for pass 2; the MAXL = 0 form loads one position at a time, twice.
 template <int ND, int MAXL, int SB>
 __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                         const double* __restrict__ b, double* __restrict__ out,
@@ -452,13 +452,8 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
       dd[d] = D[d * N + (clamp ? max(0, min(e, N - 1)) : e)];
     }
   };
-  // bi, dd -> alpha, beta (in place; dd[0] is not used again)
-  auto affine = [&](double& bi, double dd[ND]) __attribute__((always_inline)) {
-    const double rden = 1.0 / (1.0 + av * dt * dd[0]);
-    bi *= rden;
-#pragma unroll
-    for (int d = 1; d < ND; ++d) dd[d] *= dtav * rden;
-  };
+  // the division of a position: dd[0] becomes the reciprocal of the denominator
+  auto divide = [&](double dd[ND]) __attribute__((always_inline)) { dd[0] = 1.0 / (1.0 + av * dt * dd[0]); };
   double bv[NL], dv[NL][ND];
   // pass 1: the segment's map, state (y0 .. y_(K-1)), y0 the newest value
   double A[K][K], cv[K];
@@ -468,15 +463,17 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
 #pragma unroll
     for (int q = 0; q < K; ++q) A[r][q] = (r == q) ? 1.0 : 0.0;
   }
-  auto compose = [&](double alpha, const double be[ND]) __attribute__((always_inline)) {
-    double a0[K], c0 = alpha;
+  auto compose = [&](double bi, const double dd[ND]) __attribute__((always_inline)) {
+    const double rdt = dtav * dd[0];
+    double a0[K], c0 = bi * dd[0];
 #pragma unroll
     for (int q = 0; q < K; ++q) a0[q] = 0.0;
 #pragma unroll
     for (int d = ND - 1; d >= 1; --d) {
-      c0 -= be[d] * cv[d - 1];
+      const double beta = rdt * dd[d];
+      c0 -= beta * cv[d - 1];
 #pragma unroll
-      for (int q = 0; q < K; ++q) a0[q] -= be[d] * A[d - 1][q];
+      for (int q = 0; q < K; ++q) a0[q] -= beta * A[d - 1][q];
     }
 #pragma unroll
     for (int r = K - 1; r >= 1; --r) {
@@ -499,7 +496,7 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
 #pragma unroll
       for (int i = i0; i < i0 + BT; ++i)
         if (i < L) {
-          affine(bv[i], dv[i]);
+          divide(dv[i]);
           compose(bv[i], dv[i]);
         }
     }
@@ -507,7 +504,7 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
     for (int p = p_lo; p < p_hi; ++p) {
       double bi, dd[ND];
       coeffs(p, bi, dd, true);
-      affine(bi, dd);
+      divide(dd);
       compose(bi, dd);
     }
   }
@@ -550,11 +547,13 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
   for (int r = 0; r < K; ++r) y[r] = 0.0;
   for (int i = 0; i < grp; ++i) apply(gmap[i * SB + j], y, true);
   for (int i = 0; i < col; ++i) apply(maps[(grp * GS + i) * SB + j], y, true);
-  // pass 2: the recurrence over the segment
-  auto advance = [&](int p, double alpha, const double be[ND]) __attribute__((always_inline)) {
-    double val = alpha;
+  // pass 2: the recurrence over the segment as the sequential sweep evaluates it (with the rounded
+  // beta of pass 1 the result's 2-norm error was a fifth higher where dt av is small)
+  auto advance = [&](int p, double bi, const double dd[ND]) __attribute__((always_inline)) {
+    double sv = 0.0;
 #pragma unroll
-    for (int d = ND - 1; d >= 1; --d) val -= be[d] * y[d - 1];
+    for (int d = ND - 1; d >= 1; --d) sv += dd[d] * y[d - 1];
+    const double val = (bi - sv * dtav) * dd[0];
 #pragma unroll
     for (int d = K - 1; d >= 1; --d) y[d] = y[d - 1];
     y[0] = val;
@@ -569,7 +568,7 @@ __global__ __launch_bounds__(SB * NSEG) void k_fvm_vr_scan(BzFvm1d3v op, const d
     for (int p = p_lo; p < p_hi; ++p) {
       double bi, dd[ND];
       coeffs(p, bi, dd, true);
-      affine(bi, dd);
+      divide(dd);
       advance(p, bi, dd);
     }
   }
