@@ -176,7 +176,7 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
   for (int k = 0; k < GMAX; ++k)
     if (q0 + k < q1) g += op.g_val[q0 + k] * gs[k];
   for (int q = q0 + GMAX; q < q1; ++q) g += op.g_val[q] * s[(size_t)op.g_col[q] * Nx + ix];
-  const double loss = op.loss[r], rvr = 1.0 / op.vr[r], adx = op.dt_x * op.adx[r];
+  const double loss = op.loss[r], vr = op.vr[r], rvr = 1.0 / vr, adx = op.dt_x * op.adx[r];
   const bool inflow = low ? (ix == 0) : (ix == Nx - 1);
   double out[TB];
 #pragma unroll
@@ -198,7 +198,9 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
       au += (t + d < Nvt ? op.dvtR[d * Nvt + t] : 0.0) * xc[HC + i + d];
       ad += (t - d >= 0 ? op.dvtL[d * Nvt + t] : 0.0) * xc[HC + i - d];
     }
-    const double ae = cs * ar - (op.sin_vt[t] * rvr) * (ep ? au : ad);
+    // sin / vr, rounded once: the product with the reciprocal of vr corrected by its remainder
+    const double sn = op.sin_vt[t], s0 = sn * rvr, sv = fma(fma(-vr, s0, sn), rvr, s0);
+    const double ae = cs * ar - sv * (ep ? au : ad);
     out[i] = inflow ? yx : yx - dt * (op.tau_n0np0 * cv + op.tau * (Ex * (op.eq * ae)));
   }
 #pragma unroll

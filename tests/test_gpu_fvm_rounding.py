@@ -79,3 +79,24 @@ def test_radial_scan(Nr, nvr):
     err = lambda x: float(np.linalg.norm(((x - exact) * inner).astype(np.float64)))
     assert err(plain) > 0
     assert err(got) <= 1.08 * err(plain)
+
+
+@pytest.mark.parametrize("nvr,nvt,nx,Nvt", [(4, 4, 2, 16), (3, 3, 3, 12), (4, 4, 2, 6), (2, 2, 2, 8)])
+def test_angular_coefficient(nvr, nvt, nx, Nvt):
+    """The step operator reduced to x + (sin / vr) x at x = 1 (one angular weight of one, E = 1): with
+    the quotient between 2^20 and 2^21 the sum is exact, so the coefficient is the quotient itself.
+    The widths of both fixed stencils, four, two and one ordinates per thread, and the general form."""
+    Nr, Nx = 40, 5
+    rng = np.random.default_rng(nvr * Nvt)
+    sin, vr = rng.uniform(0.75, 1.0, Nvt), 2.0 ** -20 * rng.uniform(0.5, 0.75, Nr)
+    Dt = np.zeros((nvt, Nvt))
+    Dt[0] = 1.0
+    keep = []
+    op = _operator(Nr, Nvt, Nx, nvr, nvt, nx, keep, sin_vt=sin, vr=vr, dvtL=Dt, dvtR=Dt)
+    x = torch.ones((Nr, Nvt, Nx), dtype=torch.float64, device="cuda")
+    y = torch.empty_like(x)
+    _lib.call("bz_fvm_rhs_mvec", op, torch.ones(Nx, dtype=torch.float64, device="cuda"), 1.0, x, y)
+    q = sin[None] / vr[:, None]
+    assert q.min() >= 2.0 ** 20 and q.max() < 2.0 ** 21
+    # the velocity term is zero at the inflow points of either half range
+    np.testing.assert_array_equal(y.cpu().numpy()[:, :, 1:-1] - 1.0, np.repeat(q[:, :, None], Nx - 2, axis=2))
