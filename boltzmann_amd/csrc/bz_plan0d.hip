@@ -114,36 +114,43 @@ int bz_plan_grid0d(int npr, int ns, int nop, const double* const* ops, const dou
   // pattern a slot is held from step first_i - 2W to the pivot step i, which the one-pivot-a-step
   // factorisation needs.  Rows in order of their start take the lowest free slot id.
   const int NG = (W + 2) / 4;
-  std::vector<int> start(n), end(n), order(n);
-  for (int i = 0; i < n; ++i) {
-    start[i] = ee_pattern ? first[i] - 2 * W : first[i] >> 2;
-    end[i] = ee_pattern ? i - 1 : (i >> 2) + NG;
-    order[i] = i;
-  }
-  std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return start[a] < start[b]; });
-  using PI = std::pair<int, int>;
-  std::priority_queue<PI, std::vector<PI>, std::greater<PI>> alive;   // (end, slot)
-  std::priority_queue<int, std::vector<int>, std::greater<int>> free_ids;
   std::vector<std::vector<int>> slot_rows;
-  for (int i : order) {
-    while (!alive.empty() && alive.top().first < start[i]) {
-      free_ids.push(alive.top().second);
-      alive.pop();
+  auto colour = [&](bool one_pivot) {
+    std::vector<int> start(n), end(n), order(n);
+    for (int i = 0; i < n; ++i) {
+      start[i] = one_pivot ? first[i] - 2 * W : first[i] >> 2;
+      end[i] = one_pivot ? i - 1 : (i >> 2) + NG;
+      order[i] = i;
     }
-    int s;
-    if (!free_ids.empty()) {
-      s = free_ids.top();
-      free_ids.pop();
-    } else {
-      s = int(slot_rows.size());
-      slot_rows.emplace_back();
+    std::stable_sort(order.begin(), order.end(), [&](int a, int b) { return start[a] < start[b]; });
+    using PI = std::pair<int, int>;
+    std::priority_queue<PI, std::vector<PI>, std::greater<PI>> alive;   // (end, slot)
+    std::priority_queue<int, std::vector<int>, std::greater<int>> free_ids;
+    slot_rows.clear();
+    for (int i : order) {
+      while (!alive.empty() && alive.top().first < start[i]) {
+        free_ids.push(alive.top().second);
+        alive.pop();
+      }
+      int s;
+      if (!free_ids.empty()) {
+        s = free_ids.top();
+        free_ids.pop();
+      } else {
+        s = int(slot_rows.size());
+        slot_rows.emplace_back();
+      }
+      slot_rows[s].push_back(i);
+      alive.push(PI(end[i], s));
     }
-    slot_rows[s].push_back(i);
-    alive.push(PI(end[i], s));
-  }
-  const int used = int(slot_rows.size());
-  // tables of the one-pivot-a-step form (e-e) have a multiple of 64 slots, the others never
-  const int nslots = ee_pattern ? 64 * std::max(1, (used + 63) / 64) : used + (used % 64 == 0);
+    return int(slot_rows.size());
+  };
+  // tables of the one-pivot-a-step form have a multiple of 64 slots, the others never; so a blocked
+  // schedule that fills the last slot of the largest instance gives way to the other one
+  int used = colour(ee_pattern != 0);
+  const bool one_pivot = ee_pattern || used == (W >= 17 ? 256 : 192);
+  if (one_pivot && !ee_pattern) used = colour(true);
+  const int nslots = one_pivot ? 64 * std::max(1, (used + 63) / 64) : used + (used % 64 == 0);
   std::vector<int> slot_first((nslots + 63) / 64 * 64, -1), sched_next(n, -1);
   for (int s = 0; s < used; ++s) {
     slot_first[s] = slot_rows[s][0];

@@ -22,6 +22,7 @@ import torch
 from . import _lib
 
 PREFETCH_WINDOWS = 2   # rows enter their slot 2W steps before their first column
+MAX_SLOTS = (192, 256)  # row slots of the largest solver instances: windows below 17, from 17
 VEC_ROWS = 12          # n-vectors of per-instance work space (bz_batch0d_t.vec)
 
 
@@ -150,6 +151,18 @@ def tile_schedule(first_col, bw, W):
     return slot_first, sched_next, nslots
 
 
+def solver_schedule(st, one_pivot):
+    """(slot_first, sched_next, nslots) of plan_structure's st for the solver: the blocked form's
+    schedule, or the one-pivot-a-step one (nslots a multiple of 64) where the e-e path asks for it.
+    A blocked schedule that fills the last slot of the largest instance leaves no count that
+    is not a multiple of 64, so such a pattern keeps the other schedule too."""
+    if not one_pivot:
+        sched = tile_schedule(st["first_col"], st["bw"], st["W"])
+        if sched[2] != MAX_SLOTS[st["W"] >= 17] + 1:
+            return sched
+    return st["slot_first"], st["sched_next"], st["nslots"]
+
+
 class SolverTables:
     """Device tables of one grid for bz_steady_solve_0d."""
 
@@ -180,10 +193,7 @@ class SolverTables:
         self.prof_off = i32(st["prof_off"])
         # the e-e path eliminates one pivot at a time and needs the lead of two windows; its tables
         # have nslots a multiple of 64
-        if extra_mask is None:
-            slot_first, sched_next, nslots = tile_schedule(st["first_col"], st["bw"], st["W"])
-        else:
-            slot_first, sched_next, nslots = st["slot_first"], st["sched_next"], st["nslots"]
+        slot_first, sched_next, nslots = solver_schedule(st, extra_mask is not None)
         self.slot_first = i32(slot_first)
         self.sched_next = i32(sched_next)
         self.chunk_levels = i32(st["chunk_levels"])
