@@ -642,12 +642,41 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(W >= 17 ? 1 
   if (lane == 0) s1[inst] = su;
 }
 
+// The same on tables without the e-e pattern (nslots not a multiple of 64), which are planned for the
+// blocked elimination: L at the same profile positions, U rows in that form's layout.  Their
+// pattern holds the whole e-e operator for up to two harmonics.
+template <int W, int T>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(tile_waves<W, T>()))) void k_ee_factor_tiles(
+    GridDev g, BatchDev b, const int* __restrict__ active, double* __restrict__ lprof, double* __restrict__ z1,
+    double* __restrict__ s1) {
+  extern __shared__ __align__(32) double lds[];
+  const int n = g.n, lane = threadIdx.x, inst = blockIdx.x;
+  if (active && !active[inst]) return;
+  constexpr int WP = (W + 1) & ~1;
+  double* PIV = lds;
+  double* Z1 = PIV + piv_len<W>();
+  int2* SC = reinterpret_cast<int2*>(Z1 + n);
+  const double* kprof = b.kprof + (size_t)inst * g.P;
+  double* urows = b.urows + (size_t)inst * n * WP;
+  fill_rowtab(g, SC, lane);
+  for (int i = lane; i < n; i += 64) Z1[i] = g.muhat[i];
+  __syncthreads();
+  factor_tiles<W, T, true, 1>(g, kprof, SC, Z1, Z1, Z1, PIV, urows, lane, lprof + (size_t)inst * g.P);
+  __syncthreads();
+  back_tiles<W, 1>(g, urows, Z1, nullptr, nullptr, lane);
+  __syncthreads();
+  const double su = dot(g.uhat, Z1, n, lane);
+  for (int i = lane; i < n; i += 64) z1[(size_t)inst * n + i] = Z1[i];
+  if (lane == 0) s1[inst] = su;
+}
+
 // Forward solve with the stored unit lower factor, row by row; the profile rows are staged
 // through LDS in chunks of whole rows (at most LBUF entries) with the next chunk's loads in
 // flight (registers) while the current chunk is swept, so the sweep waits on LDS only.
 constexpr int LBUF = 1024;
 
-template <int W>
+// TILES: U rows in the layout of the blocked elimination.
+template <int W, bool TILES>
 __global__ __launch_bounds__(64) void k_ee_precond_apply(GridDev g, BatchDev b, const int* __restrict__ active,
                                                          const double* __restrict__ lprof,
                                                          const double* __restrict__ z1, const double* __restrict__ s1,
@@ -781,7 +810,8 @@ __global__ __launch_bounds__(64) void k_ee_precond_apply(GridDev g, BatchDev b, 
     r0 = r1;
     r1 = r2;
   }
-  back_substitute<W>(n, urows, WP, Y1, Y2, nullptr, STG, lane);
+  if constexpr (TILES) back_tiles<W, 1>(g, urows, Y2, nullptr, nullptr, lane);
+  else back_substitute<W>(n, urows, WP, Y1, Y2, nullptr, STG, lane);
   __syncthreads();
   const double c = -dot(g.uhat, Y2, n, lane) / s1[inst];
   const double* Z1 = z1 + (size_t)inst * n;
@@ -803,6 +833,16 @@ int launch_ee_factor(const GridDev& g, const BatchDev& b, const int* active, dou
   return BZ_OK;
 }
 
+template <int W, int T>
+int launch_ee_factor_tiles(const GridDev& g, const BatchDev& b, const int* active, double* lprof, double* z1, double* s1,
+                           hipStream_t stream) {
+  const size_t lds = (size_t)(g.n + piv_len<W>()) * sizeof(double) + (size_t)g.n * sizeof(int2);
+  if (lds > 64 * 1024 || !fits_offsets(g)) return BZ_EINVAL;
+  hipLaunchKernelGGL((k_ee_factor_tiles<W, T>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1);
+  BZ_LAUNCH_CHECK();
+  return BZ_OK;
+}
+
 template <int W>
 int launch_ee_apply(const GridDev& g, const BatchDev& b, const int* active, const double* lprof, const double* z1,
                     const double* s1, const double* v, double* out, double* outT, hipStream_t stream) {
@@ -810,8 +850,12 @@ int launch_ee_apply(const GridDev& g, const BatchDev& b, const int* active, cons
   const size_t lds = (size_t)(3 * g.n + 2 * W * WP + 2 * LBUF) * sizeof(double) + (size_t)(g.n + 1) * sizeof(int) +
                      (size_t)g.n * sizeof(short);
   if (lds > 64 * 1024 || g.max_row > LBUF) return BZ_EINVAL;
-  hipLaunchKernelGGL((k_ee_precond_apply<W>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1, v, out,
-                     outT);
+  if (g.nslots % 64 == 0)
+    hipLaunchKernelGGL((k_ee_precond_apply<W, false>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1, v,
+                       out, outT);
+  else
+    hipLaunchKernelGGL((k_ee_precond_apply<W, true>), dim3(b.B), dim3(64), lds, stream, g, b, active, lprof, z1, s1, v,
+                       out, outT);
   BZ_LAUNCH_CHECK();
   return BZ_OK;
 }

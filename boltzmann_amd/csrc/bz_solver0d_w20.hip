@@ -20,6 +20,9 @@ int transient_w20(const GridDev& g, const BatchDev& b, double cdt, const double*
 
 int ee_factor_w20(const GridDev& g, const BatchDev& b, const int* active, double* lprof, double* z1, double* s1,
                    hipStream_t s) {
+  if (g.nslots % 64 != 0) {
+    BZ0D_FOR_TILES(20, launch_ee_factor_tiles, g, b, active, lprof, z1, s1, s)
+  }
   BZ0D_FOR_LEVELS(20, launch_ee_factor, g, b, active, lprof, z1, s1, s)
 }
 
