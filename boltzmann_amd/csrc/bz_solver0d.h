@@ -29,6 +29,7 @@
 // structures and the per-window dispatch functions is TU-local (anonymous namespace).
 #pragma once
 #include <algorithm>
+#include <type_traits>
 #include "bz_common.h"
 #include "../../include/bz.h"
 
@@ -478,6 +479,11 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
   constexpr int NG = trail_groups<W>(), WP = (W + 1) & ~1, NX = NG > 4 ? NG - 4 : 0;
   constexpr bool Y16 = NG <= 3;                      // the right-hand sides ride in the 16x16x4 tile
   constexpr int YR = Y16 ? NG : 0;                   // as its element YR
+  // With five groups the compiler, where it keeps part of a tile in accumulation registers, pairs the
+  // publishing stores with wrong offsets (8, 6 and 4 doubles for 64, 48 and 32 in the assembly of
+  // W = 20 with five tiles and more: an offset in units of eight divided by eight once more).
+  // Volatile stores are not paired.
+  using PubPtr = std::conditional_t<(NX > 0), volatile lds_double*, lds_double*>;
   const int n = g.n, bw = g.bw;
   const int q = lane >> 4, a16 = lane & 15, i4 = lane & 3;
   const ProfileBuf kb = profile_buf(kprof, g.P), ub = profile_buf(urows, n * WP);
@@ -560,7 +566,7 @@ __device__ __forceinline__ void factor_tiles(const GridDev& g, const double* __r
         const bool mine = (unsigned)rel < 4u;
         if (wave_any(mine)) {
           if (mine) {
-            lds_double* pk = piv + 4 * q + rel;
+            PubPtr pk = (PubPtr)(piv + 4 * q + rel);
             pk[0] = P[t];
 #pragma unroll
             for (int r = 0; r < NG; ++r) pk[16 * (r > u ? r - u : r - u + NG)] = r < 4 ? R4[t][r < 4 ? r : 0] : RX[NX ? t : 0];
