@@ -781,12 +781,17 @@ __global__ __launch_bounds__(PT) void k_fvm_plane(BzFvm1d3v op, const double* __
 }
 
 // Whether the plane of a radius takes k_fvm_plane: two-point x stencil with at most 8 points per
-// lane, one of the common angular stencils, and a plane that fits 64 KB of LDS with its tables.
+// lane, one of the common angular stencils, a plane that fits 64 KB of LDS with its tables, and
+// either radii for every CU or a small plane.  The kernel takes one workgroup's time over a plane
+// (10 us at 16 x 100, 19 at 24 x 200) with up to 256 radii, where the two sweeps still get faster;
+// against both of them and a moment: 256 radii of 24 x 200 20.7 and 22.8 + 4.9 us, 65 radii 19.4 and
+// 12.3 + 2.9; 65 radii of 16 x 100 11.2 and 8.8 + 2.6, with two launches more.
 size_t plane_doubles(const BzFvm1d3v& op) {
   return (size_t)op.Nvt * op.Nx + 2 * (size_t)op.nvt * op.Nvt + 4 * (size_t)op.Nx;
 }
 bool plane_fits(const BzFvm1d3v& op) {
-  return op.nx == 2 && op.Nx <= 64 * 8 && op.nvt >= 2 && op.nvt <= 5 && plane_doubles(op) <= 8192;
+  return op.nx == 2 && op.Nx <= 64 * 8 && op.nvt >= 2 && op.nvt <= 5 && plane_doubles(op) <= 8192 &&
+         (op.Nr >= 256 || (long)op.Nvt * op.Nx <= 1600);
 }
 
 template <int ND>
