@@ -207,13 +207,18 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
   for (int i = 0; i < TB; ++i) y[((size_t)r * Nvt + t0 + i) * Nx + ix] = out[i];
 }
 
-// Four ordinates per thread where they fit a half range, two for the remaining even half ranges
-// (6, 10, ...), one for odd ones.
+// Ordinates per thread: four where they fit a half range, two for the remaining even half ranges (6,
+// 10, ...), one for odd ones; fewer while that leaves SIMDs without a wavefront (with one ordinate
+// per thread 800 wavefronts of 64 elements, with two 3200), where a thread's own time counts.
+// 65 x 8 x 41: 4.0, 4.1 and 5.6 us with one, two and four; 65 x 16 x 100 5.3, 5.0, 6.1;
+// 256 x 16 x 100 10.6, 9.4, 8.1.
 template <int NX, int NVR, int NVT>
 void launch_matvec_t(const BzFvm1d3v& op, const double* E, double dt, const double* x, const double* s, double* y,
                      const int* done, hipStream_t st) {
   const int mp = op.Nvt / 2;
-  const int tb = mp % 4 == 0 ? 4 : (mp % 2 == 0 ? 2 : 1);
+  const long waves = (long)op.Nr * op.Nvt * op.Nx / 64;
+  const int most = waves < 800 ? 1 : (waves < 3200 ? 2 : 4);
+  const int tb = mp % 4 == 0 && most == 4 ? 4 : (mp % 2 == 0 && most >= 2 ? 2 : 1);
   const int tx = op.Nx <= 64 ? 64 : (op.Nx <= 128 ? 128 : 256);         // x per workgroup
   const long nwg = (long)op.Nr * (op.Nvt / tb) * ((op.Nx + tx - 1) / tx);
   const dim3 grid((unsigned)((nwg + 7) / 8 * 8)), block(tx);

@@ -52,3 +52,35 @@ def test_plane_against_sweeps(Nvt, Nx, nvt):
         _lib.call("bz_fvm_step_product", ops, E, 0.1, 0.3, b[r0:r0 + part].contiguous(), t2, w2, None)
         assert torch.equal(t1, y) and torch.equal(t2, z)
         assert float((w1[r0:r0 + part] - w2).abs().max()) <= 1e-12 * float(w2.abs().max())
+
+
+@pytest.mark.parametrize("nvr,nvt,nx", [(4, 4, 2), (3, 3, 3)])
+@pytest.mark.parametrize("Nvt,Nx", [(16, 100), (8, 130)])
+def test_ordinates_per_thread(nvr, nvt, nx, Nvt, Nx):
+    """The step operator with four, two and one ordinates per thread, by the size of the state: rows of
+    a large state against states of its first radii (the last of which have other radial
+    neighbours).  The same sums in the same order; the compiler may fuse their products otherwise: a
+    few eps of the largest term."""
+    rng = np.random.default_rng(Nx)
+    Nr = 280
+    t = _tables(rng, Nr, Nvt, Nx, nvt, nx)
+    t.update(sin_vt=rng.uniform(0.1, 1.0, Nvt), adx=rng.uniform(0.5, 2.0, Nr), loss=rng.uniform(0.1, 0.5, Nr))
+    for k, shape in (("dvrL", (nvr, Nr)), ("dvrR", (nvr, Nr)), ("dvtL", (nvt, Nvt)), ("dvtR", (nvt, Nvt)),
+                     ("dxL", (nx, Nx)), ("dxR", (nx, Nx))):
+        t[k] = rng.uniform(-1.0, 1.0, shape)
+    E = torch.from_numpy(rng.normal(size=Nx)).cuda()
+    x = torch.from_numpy(rng.normal(size=(Nr, Nvt, Nx))).cuda()
+    keep, outs = [], {}
+    for part in (Nr, 100, 20):
+        waves = part * Nvt * Nx // 64
+        assert (waves >= 3200, 800 <= waves < 3200, waves < 800)[(Nr, 100, 20).index(part)]
+        cut = {k: (v[:part] if k in ("vr", "axvr", "ainv", "adx", "loss") else v[:, :part] if k in ("dvrL", "dvrR") else v)
+               for k, v in t.items()}
+        op = _operator(part, Nvt, Nx, nvr, nvt, nx, keep, **cut)
+        op.dt_x = 0.3
+        y = torch.empty((part, Nvt, Nx), dtype=torch.float64, device="cuda")
+        _lib.call("bz_fvm_rhs_mvec", op, E, 0.2, x[:part].contiguous(), y)
+        outs[part] = y
+    for part in (100, 20):
+        n = part - (nvr - 1)
+        assert float((outs[part][:n] - outs[Nr][:n]).abs().max()) <= 1e-14 * float(outs[Nr].abs().max())
