@@ -104,7 +104,8 @@ __global__ __launch_bounds__(256) void k_fvm_matvec(BzFvm1d3v op, const double* 
 
 // A load at a workgroup-uniform row plus a byte offset of the lane (one instruction, no address
 // arithmetic in the vector unit).
-__device__ __forceinline__ double row_load(const double* row, unsigned off) {
+template <typename Off>
+__device__ __forceinline__ double row_load(const double* row, Off off) {
   return *(const double*)((const char*)row + off);
 }
 
@@ -115,7 +116,8 @@ __device__ __forceinline__ double row_load(const double* row, unsigned off) {
 // scalars, weights outside the domain are zeroed as scalars (their clamped operands are values the
 // stencil uses anyway), the gains and the x weights are shared by the TB ordinates, and the
 // angular sum is taken both ways and chosen once.  Measured at 671 x 16 x 100: 19.3 -> 11.6 us.
-template <int NX, int NVR, int NVT, int GMAX, int TB>
+// Off: byte offsets of 32 bits, or of 64 for states of 2^29 elements and more.
+template <int NX, int NVR, int NVT, int GMAX, int TB, typename Off>
 __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double* __restrict__ E, double dt,
                                                       const double* __restrict__ x, const double* __restrict__ s,
                                                       double* __restrict__ y, const int* __restrict__ done) {
@@ -134,7 +136,7 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
   if (row >= Nr * ntg || ix >= Nx) return;
   const int r = row / ntg, t0 = (row - r * ntg) * TB;
   const bool low = t0 >= Nvt / 2;
-  const unsigned rs8 = (unsigned)Nvt * Nx * 8u, ix8 = ix * 8u;
+  const Off rs8 = (Off)Nvt * Nx * 8, ix8 = (Off)ix * 8;
   const double Ex = E[ix];
   const bool ep = Ex >= 0, up = ep == low;
   const double* xr0 = x + (size_t)r * Nvt * Nx;
@@ -145,7 +147,7 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
   for (int k = 0; k < NC; ++k) xc[k] = row_load(xr0 + (size_t)min(max(t0 - HC + k, 0), Nvt - 1) * Nx, ix8);
 #pragma unroll
   for (int d = 1; d < NVR; ++d) {
-    const unsigned off = ix8 + (up ? min(r + d, Nr - 1) * rs8 : max(r - d, 0) * rs8);
+    const Off off = ix8 + (up ? min(r + d, Nr - 1) * rs8 : max(r - d, 0) * rs8);
 #pragma unroll
     for (int i = 0; i < TB; ++i) xr[i][d] = row_load(x + (size_t)(t0 + i) * Nx, off);
   }
@@ -158,7 +160,7 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
     if (!in) dx[k] = 0.0;
     if (k > 0)
 #pragma unroll
-      for (int i = 0; i < TB; ++i) xn[i][k] = row_load(xr0 + (size_t)(t0 + i) * Nx, in ? 8u * j : ix8);
+      for (int i = 0; i < TB; ++i) xn[i][k] = row_load(xr0 + (size_t)(t0 + i) * Nx, in ? (Off)8 * j : ix8);
   }
   const int q0 = op.g_ptr[r], q1 = op.g_ptr[r + 1];
   const int qmax = max(op.g_ptr[Nr] - 1, 0);
@@ -212,7 +214,7 @@ __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double
 // per thread 800 wavefronts of 64 elements, with two 3200), where a thread's own time counts.
 // 65 x 8 x 41: 4.0, 4.1 and 5.6 us with one, two and four; 65 x 16 x 100 5.3, 5.0, 6.1;
 // 256 x 16 x 100 10.6, 9.4, 8.1.
-template <int NX, int NVR, int NVT>
+template <int NX, int NVR, int NVT, typename Off>
 void launch_matvec_t(const BzFvm1d3v& op, const double* E, double dt, const double* x, const double* s, double* y,
                      const int* done, hipStream_t st) {
   const int mp = op.Nvt / 2;
@@ -222,9 +224,12 @@ void launch_matvec_t(const BzFvm1d3v& op, const double* E, double dt, const doub
   const int tx = op.Nx <= 64 ? 64 : (op.Nx <= 128 ? 128 : 256);         // x per workgroup
   const long nwg = (long)op.Nr * (op.Nvt / tb) * ((op.Nx + tx - 1) / tx);
   const dim3 grid((unsigned)((nwg + 7) / 8 * 8)), block(tx);
-  if (tb == 4) hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 4>), grid, block, 0, st, op, E, dt, x, s, y, done);
-  else if (tb == 2) hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 2>), grid, block, 0, st, op, E, dt, x, s, y, done);
-  else hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 1>), grid, block, 0, st, op, E, dt, x, s, y, done);
+  if (tb == 4)
+    hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 4, Off>), grid, block, 0, st, op, E, dt, x, s, y, done);
+  else if (tb == 2)
+    hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 2, Off>), grid, block, 0, st, op, E, dt, x, s, y, done);
+  else
+    hipLaunchKernelGGL((k_fvm_matvec_t<NX, NVR, NVT, 6, 1, Off>), grid, block, 0, st, op, E, dt, x, s, y, done);
 }
 
 // h = H s on the matrix cores: one workgroup of CC_WAVES wavefronts per 16 x 16 tile of h
@@ -869,10 +874,13 @@ int launch_rhs_mvec(const BzFvm1d3v* op, const double* E, double dt, const doubl
   const long n = (long)nrx * op->Nvt;
   const dim3 grid((unsigned)((n + 255) / 256)), block(256);
   const bool offsets_fit = n < (1L << 29);            // row_load's 32-bit byte offsets
-  if (offsets_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
-    launch_matvec_t<2, 4, 4>(*op, E, dt, x, s, y, done, stream);
-  else if (offsets_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
-    launch_matvec_t<3, 3, 3>(*op, E, dt, x, s, y, done, stream);
+  const bool rows_fit = (long)op->Nr * op->Nvt * ((op->Nx + 63) / 64) < (1L << 30);    // workgroups
+  if (rows_fit && op->nx == 2 && op->nvr == 4 && op->nvt == 4)
+    offsets_fit ? launch_matvec_t<2, 4, 4, unsigned>(*op, E, dt, x, s, y, done, stream)
+                : launch_matvec_t<2, 4, 4, size_t>(*op, E, dt, x, s, y, done, stream);
+  else if (rows_fit && op->nx == 3 && op->nvr == 3 && op->nvt == 3)
+    offsets_fit ? launch_matvec_t<3, 3, 3, unsigned>(*op, E, dt, x, s, y, done, stream)
+                : launch_matvec_t<3, 3, 3, size_t>(*op, E, dt, x, s, y, done, stream);
   else
     hipLaunchKernelGGL(k_fvm_matvec, grid, block, 0, stream, *op, E, dt, x, s, y, done);
   BZ_LAUNCH_CHECK();

@@ -84,3 +84,34 @@ def test_ordinates_per_thread(nvr, nvt, nx, Nvt, Nx):
     for part in (100, 20):
         n = part - (nvr - 1)
         assert float((outs[part][:n] - outs[Nr][:n]).abs().max()) <= 1e-14 * float(outs[Nr].abs().max())
+
+
+@pytest.mark.parametrize("nvr,nvt,nx", [(4, 4, 2), (3, 3, 3)])
+def test_states_past_32_bit_offsets(nvr, nvt, nx):
+    """5.4e8 elements (4.3 GB): the last radii against a state that holds those only; the same kernel
+    but for the width of its offsets, so the same bits."""
+    Nr, Nvt, Nx, part = 1024, 64, 8300, 12
+    assert Nr * Nvt * Nx >= 1 << 29
+    rng = np.random.default_rng(nx)
+    t = _tables(rng, Nr, Nvt, Nx, nvt, nx)
+    t.update(sin_vt=rng.uniform(0.1, 1.0, Nvt), adx=rng.uniform(0.5, 2.0, Nr), loss=rng.uniform(0.1, 0.5, Nr))
+    t.pop("ainv")
+    for k, shape in (("dvrL", (nvr, Nr)), ("dvrR", (nvr, Nr)), ("dvtL", (nvt, Nvt)), ("dvtR", (nvt, Nvt)),
+                     ("dxL", (nx, Nx)), ("dxR", (nx, Nx))):
+        t[k] = rng.uniform(-1.0, 1.0, shape)
+    E = torch.from_numpy(rng.normal(size=Nx)).cuda()
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    x = torch.randn((Nr, Nvt, Nx), dtype=torch.float64, device="cuda", generator=gen)
+    y = torch.empty_like(x)
+    keep = []
+    op = _operator(Nr, Nvt, Nx, nvr, nvt, nx, keep, **t)
+    op.dt_x = 0.3
+    _lib.call("bz_fvm_rhs_mvec", op, E, 0.2, x, y)
+    cut = {k: (v[-part:] if k in ("vr", "axvr", "adx", "loss") else v[:, -part:] if k in ("dvrL", "dvrR") else v)
+           for k, v in t.items()}
+    ops = _operator(part, Nvt, Nx, nvr, nvt, nx, keep, **cut)
+    ops.dt_x = 0.3
+    z = torch.empty((part, Nvt, Nx), dtype=torch.float64, device="cuda")
+    _lib.call("bz_fvm_rhs_mvec", ops, E, 0.2, x[-part:].contiguous(), z)
+    k = part - (nvr - 1)
+    assert torch.equal(y[-k:], z[-k:])
