@@ -55,3 +55,17 @@ def test_no_callback_for_a_converged_start(use_graph):
         assert torch.equal(x, 0.5 * b) or float((x - 0.5 * b).abs().max()) < 1e-12 * n
     x, k = s.solve(0.0 * b, 1e-3, 0.0, 5, callback=seen.append)
     assert k == 0 and not bool(x.any()) and len(seen) == 0
+
+
+@pytest.mark.parametrize("nx,nbins", [(1023, 1), (1024, 1), (1000, 30), (2000, 256), (4096, 256)])
+def test_points_grouped_by_several_workgroups(nx, nbins):
+    """Whole numbers: starts, counts and a stable order, with points in every bin, the last included."""
+    gen = torch.Generator(device="cuda").manual_seed(nx)
+    b = torch.randint(0, nbins, (nx,), generator=gen, dtype=torch.int32, device="cuda")
+    b[-1] = nbins - 1
+    out = [torch.full((k,), -1, dtype=torch.int32, device="cuda") for k in (nbins, nbins, nx)]
+    _lib.call("bz_group_bins", b, nx, nbins, *out)
+    count = torch.bincount(b.cpu().long(), minlength=nbins)
+    assert torch.equal(out[1].cpu().long(), count)
+    assert torch.equal(out[0].cpu().long(), count.cumsum(0) - count)
+    assert torch.equal(out[2].cpu().long(), torch.argsort(b.cpu(), stable=True))
