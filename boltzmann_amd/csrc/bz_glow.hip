@@ -640,7 +640,9 @@ __global__ __launch_bounds__(NT) void k_glow_fluid(BzGlowFluid g, int flags, dou
         }
       }
       const int singular = gf_gauss_jordan<SMAX>(q, S, X, Sc) | 2;     // bit 1: pivoted path
-      gf_newton<SMAX <= 32 ? 8 : 2>(q, S, g, h, singular,
+      // the products' loads in flight beside the matrix; with 100 columns in registers a second one
+      // spilled in every elimination step (829 us against 675 at 129 points, 865 and 735 at 200)
+      gf_newton<SMAX <= 32 ? 8 : 1>(q, S, g, h, singular,
                 [&](const double* rr, double* dx) { gf_apply_inverse<SMAX>(q, S, X, Sc, rr, dx); });
     }
   }
