@@ -174,6 +174,37 @@ __device__ __forceinline__ void gf_apply_inverse(const GfCtx& q, GfShared& S, co
   __syncthreads();
 }
 
+// The largest a of the wavefront and, among equal ones, the lowest ai, in every lane, by swaps and DPP
+// moves (by six shuffles through LDS the pivoted step took 157 us at 75 points and 174 at 88, more
+// than the 147 and 163 of the rows over 1024 threads before; 144 and 160 so).
+__device__ __forceinline__ void gf_argmax(double& a, int& ai) {
+  auto take = [&](double ov, int oi) __attribute__((always_inline)) {
+    const bool better = ov > a || (ov == a && oi < ai);
+    a = better ? ov : a;
+    ai = better ? oi : ai;
+  };
+  {
+    const unsigned lo = (unsigned)__double2loint(a), hi = (unsigned)__double2hiint(a), ix = (unsigned)ai;
+    const auto l = __builtin_amdgcn_permlane32_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane32_swap(hi, hi, false, false);
+    const auto x = __builtin_amdgcn_permlane32_swap(ix, ix, false, false);
+    take(__hiloint2double((int)h[0], (int)l[0]), (int)x[0]);
+    take(__hiloint2double((int)h[1], (int)l[1]), (int)x[1]);
+  }
+  {
+    const unsigned lo = (unsigned)__double2loint(a), hi = (unsigned)__double2hiint(a), ix = (unsigned)ai;
+    const auto l = __builtin_amdgcn_permlane16_swap(lo, lo, false, false);
+    const auto h = __builtin_amdgcn_permlane16_swap(hi, hi, false, false);
+    const auto x = __builtin_amdgcn_permlane16_swap(ix, ix, false, false);
+    take(__hiloint2double((int)h[0], (int)l[0]), (int)x[0]);
+    take(__hiloint2double((int)h[1], (int)l[1]), (int)x[1]);
+  }
+  take(bz::dpp_move<bz::kDppRor8>(a), __builtin_amdgcn_mov_dpp(ai, bz::kDppRor8, 0xf, 0xf, true));
+  take(bz::dpp_move<bz::kDppRor4>(a), __builtin_amdgcn_mov_dpp(ai, bz::kDppRor4, 0xf, 0xf, true));
+  take(bz::dpp_move<bz::kDppXor2>(a), __builtin_amdgcn_mov_dpp(ai, bz::kDppXor2, 0xf, 0xf, true));
+  take(bz::dpp_move<bz::kDppXor1>(a), __builtin_amdgcn_mov_dpp(ai, bz::kDppXor1, 0xf, 0xf, true));
+}
+
 // In-place Gauss-Jordan inverse of the register-resident matrix.  Thread (r, g) keeps the
 // columns g Sc + s of row r; every step all threads rotate their registers by one, so the
 // column eliminated at step m (column m % SMAX of group m / SMAX) always sits in register 0
@@ -209,14 +240,7 @@ __device__ __forceinline__ int gf_gauss_jordan(const GfCtx& q, GfShared& S, doub
           ai = q.r;
         }
       }
-      for (int off = 32; off > 0; off >>= 1) {
-        const double ov = __shfl_xor(a, off, 64);
-        const int oi = __shfl_xor(ai, off, 64);
-        if (ov > a || (ov == a && oi < ai)) {
-          a = ov;
-          ai = oi;
-        }
-      }
+      gf_argmax(a, ai);
       if ((t & 63) == 0) {
         S.candv[w] = a;
         S.candi[w] = ai;
