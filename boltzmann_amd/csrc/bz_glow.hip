@@ -30,7 +30,7 @@ namespace {
 constexpr int GF_THREADS = 512;
 constexpr int GF_WAVES = GF_THREADS / 64;
 constexpr int GF_NMAX = 200;
-constexpr int GF_NPAD = 384;       // >= CG ceil(Np / CG) and CG SMAX for every Np <= 200: padded vectors
+constexpr int GF_NPAD = 384;       // >= CG ceil(Np / CG) for every Np <= 200: padded vectors
 constexpr int BZ_GLOW_TILE_THREADS = 512;   // = GF_THREADS: tables are laid out by thread
 constexpr int GF_TILE_RED = 5000;  // >= max(TR, TC) Npad of the tile layouts below (25 x 200 at 8 x 10)
 
@@ -778,6 +778,9 @@ extern "C" int bz_glow_fluid_step(const BzGlowFluid* g, int flags, double h, dou
   static_assert(25 * 200 <= GF_TILE_RED && 22 * 132 <= GF_TILE_RED, "tile reduction buffer");
   static_assert(25 * 20 <= 512 && 22 * 22 <= 512, "tile threads");
   static_assert((88 + 512 / 88 - 1) / (512 / 88) <= 18, "row layout");
+  // prow is indexed by CG SMAX: most groups at 22 and 23 points, and the other two layouts
+  static_assert(22 * 18 <= GF_THREADS + 64 && (512 / 89) * 32 <= GF_THREADS + 64 && (512 / 129) * 100 <= GF_THREADS + 64,
+                "pivot row buffer");
   const BzGlowFluid gv = *g;
   // the row layout of the eliminating path: up to 18 columns a thread at 88 points, 32 at 128 and
   // 100 at 200 in the 256 registers that 512 threads leave each

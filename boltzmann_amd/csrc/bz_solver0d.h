@@ -112,8 +112,9 @@ using namespace bz0d;
 
 constexpr int kMaxOps = 16;
 // rows of the per-instance work array b.vec (each n doubles): 0 growth vector w, 1 x, 2 M x,
-// 3 third right-hand side, 4..10 the unshifted values of K on the band of M (row i, offset d:
-// row 4 + d, entry i), 11 the Newton step
+// 3 third right-hand side, 4..10 the unshifted values of K on the band of M (row i, offset d: entry
+// 7 i + d of the seven rows in k_newton0d, entry i of row 4 + d in k_newton0d_lane), 11 the Newton
+// step
 constexpr int kVecRows = 12;
 // exact-Newton line search: residual evaluations per step, and the step length below which an
 // accepted step counts as a stall
@@ -989,7 +990,7 @@ __device__ double proj_norm(const double* v, const ProfileBuf& uh, int n, int la
 // exact Newton step p with uhat.p = 0 satisfies K' p = c M uhat + d M x - K' x, d = w.p
 // (the reference's Jacobian, mode 0, takes d = 0).
 //  * Residual evaluation at a point x (row_pass): x is put on u.x = 1, mu = w.x (compensated
-//    dot); one pass over the rows (one lane per row) sets the band of M in the profile to
+//    dot); one pass over the rows (eight lanes to a row) sets the band of M in the profile to
 //    K' = K - mu M from the unshifted values of K (saved at the first pass; the difference is
 //    formed exactly and rounded once) and forms, in compensated arithmetic (TwoProduct by fma,
 //    TwoSum), the right-hand side y3 = c' M uhat - K' x for the coefficient c' of the step
