@@ -100,6 +100,13 @@ class _Grid:
         return b
 
 
+# Small e-e batches at once.  Their host loops take turns at the interpreter lock, and with three or
+# four of them every launch waits for the others' (2000 mixed requests, three mixes: 105, 110 and
+# 99 solves/s with four at once, 148, 156 and 147 with three, 150, 159 and 180 with two, 100, 98
+# and 125 with one; the requests' 99th percentile 17, 16 and 19 s with four, 11, 11 and 10 with two).
+EE_SMALL = 2
+
+
 class ServingEngine:
     def __init__(self, xsec_file, hbm_budget, Te=4.0, ev_max=80.0, q=5, max_batch=4096, rtol=1e-14,
                  max_iter=30, ee_rtol=1e-15, ee_max_iter=60, restart=30, streams=4, ee_min_batch=256,
@@ -118,7 +125,8 @@ class ServingEngine:
         # admitting and retiring the asynchronous batches meanwhile; up to ee_workers of them at
         # once, of different grid signatures (a grid's e-e work space serves one batch at a
         # time), each on an e-e stream of its own (default priority); they wait in their queue
-        # for ee_min_batch requests or ee_max_wait seconds
+        # for ee_min_batch requests or ee_max_wait seconds.  Of batches below ee_min_batch, whose
+        # time is that of the host's launches and not of the kernels, at most EE_SMALL at once.
         self.ee_workers = max(1, int(ee_workers))
         self._ee_pool = concurrent.futures.ThreadPoolExecutor(max_workers=self.ee_workers)
         self.ee_streams = [torch.cuda.Stream(device=self.dev) for _ in range(self.ee_workers)]
@@ -241,6 +249,9 @@ class ServingEngine:
                         busy = [b["key"] for b in inflight if "future" in b]
                         if len(busy) >= self.ee_workers or qk[:3] in busy:
                             continue                           # all e-e workers busy, or this grid's
+                        small = sum(len(b["reqs"]) < self.ee_min_batch for b in inflight if "future" in b)
+                        if len(qq) < self.ee_min_batch and small >= EE_SMALL:
+                            continue                           # and meanwhile the batch grows
                         if (len(qq) < self.ee_min_batch and now - qq[0].arrival < self.ee_max_wait
                                 and i < len(reqs)):
                             continue                           # let the batch grow
