@@ -115,7 +115,8 @@ __device__ __forceinline__ double row_load(const double* row, Off off) {
 // worked out per lane took about 1000 instructions for four elements.  Here rows are addressed by
 // scalars, weights outside the domain are zeroed as scalars (their clamped operands are values the
 // stencil uses anyway), the gains and the x weights are shared by the TB ordinates, and the
-// angular sum is taken both ways and chosen once.  Measured at 671 x 16 x 100: 19.3 -> 11.6 us.
+// angular sum is taken both ways and chosen once.  Measured at 671 x 16 x 100: 19.9 -> 12.9 us (0.9 of
+// it for the quotient sin / vr rounded once).
 // Off: byte offsets of 32 bits, or of 64 for states of 2^29 elements and more.
 template <int NX, int NVR, int NVT, int GMAX, int TB, typename Off>
 __global__ __launch_bounds__(256) void k_fvm_matvec_t(BzFvm1d3v op, const double* __restrict__ E, double dt,
@@ -421,7 +422,7 @@ __global__ __launch_bounds__(SWT) void k_fvm_sweep(BzFvm1d3v op, const double* _
 // What bounds it is the instructions and latency of one thread, with less than a wavefront per
 // SIMD: so pass 2 reuses the loads and the one division of pass 1 and addresses are 32-bit
 // offsets.  64 segments of half the length were slower (their maps and coefficients do not fit the
-// registers of a 512-thread workgroup).  Measured at 671 x 16 x 100: 18.7 -> 15.8 us.
+// registers of a 512-thread workgroup).  Measured at 671 x 16 x 100: 19.3 -> 15.0 us.
 constexpr int SCAN_SB = 8, NSEG = 32;
 
 // MAXL > 0: a segment has at most MAXL positions; its loads (right-hand sides and stencil weights,
